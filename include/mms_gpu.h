@@ -40,8 +40,10 @@ extern "C" {
 /* Part 1: the reference's entry points                                     */
 /* ------------------------------------------------------------------------ */
 
-/* O(N^2) scalar potential phi_i = sum_{j != i} charge_j dx dy dz / |r_i - r_j|
- * over the whole xdim*ydim*zdim grid (cell index z*ydim*xdim + y*xdim + x).
+/* Exact scalar potential phi_i = sum_{j != i} charge_j dx dy dz / |r_i - r_j|
+ * over the whole xdim*ydim*zdim grid (cell index z*ydim*xdim + y*xdim + x):
+ * summed pair by pair on small grids, as an FP64 transform convolution on
+ * larger ones.
  * `potential` is fully overwritten.
  * Replaces: int calc_potential_exact(...)  helper_functions.hpp:31-35,
  *           defined fmm_calc.cu:412-461. */
@@ -107,12 +109,14 @@ int time_marching(unsigned char *material, float *M, float finaltime, float time
 /* Direct-sum potential of device arrays that allocates nothing (no
  * counterpart in the reference: for callers that cannot allocate device
  * memory -- code under stream/graph capture, tight serving loops).  Same
- * kernels and chunking as calc_potential_exact, so the same results bit for
+ * form and kernels as calc_potential_exact, so the same results bit for
  * bit; charge_dev / potential_dev are device arrays of xdim*ydim*zdim
  * floats; enqueued on `stream` (a hipStream_t, NULL = the default stream),
- * returns once enqueued.  The chunk partial sums use a fixed 16 MiB device
- * scratch per GPU: grids needing more (above 2,097,152 cells) are rejected
+ * returns once enqueued.  Tables, work arrays and partial sums use a fixed
+ * 128 MiB device scratch per GPU: grids above 2,097,152 cells are rejected
  * with an error.  Calls that overlap on one GPU share that scratch and race.
+ * A caller that solves one shape again and again keeps its tables in a
+ * context (mms_potential_dev); here they are formed in every call.
  * Variant of calc_potential_exact (fmm_calc.cu:412-461). */
 int mms_potential_exact_noalloc(const float *charge_dev, float *potential_dev, int xdim, int ydim, int zdim,
                                 float dx, float dy, float dz, void *stream);
@@ -125,7 +129,7 @@ int mms_potential_exact_noalloc(const float *charge_dev, float *potential_dev, i
 typedef struct mms_ctx mms_ctx;
 
 enum mms_solver {
-    MMS_SOLVER_DIRECT = 0, /* O(N^2) direct sum                                */
+    MMS_SOLVER_DIRECT = 0, /* exact sum over all pairs (calc_potential_exact)    */
     MMS_SOLVER_FMM = 1,    /* P2M, M2M, M2L, L2L, L2P + near-field P2P          */
     MMS_SOLVER_DIRECT_REFGPU = 2 /* O(N^2) direct sum in the float arithmetic
                               and summation order of the reference's CUDA
@@ -170,7 +174,7 @@ typedef struct {
     int external;               /* enum mms_external                           */
     float hext[3];              /* A/m, for MMS_EXT_CONST                      */
     int m2l_cols;               /* M2L targets per wavefront in 16-column MFMA tiles (4 or 8; 0 = 4) */
-    int direct_split;           /* direct sum: source-chunk multiplier (1, 2 or 4; 0 = 1) */
+    int direct_split;           /* direct sum: source-chunk multiplier of the pair loop (1, 2 or 4; 0 = 1) */
 } mms_params;
 
 /* Create a context owning device state for one film.  material: one byte per

@@ -132,6 +132,11 @@ int mms_ctx::potential(const float *rho_d, float *phi_d) {
     return direct_potential(g, direct, rho_d, phi_d, stream, &prof);
 }
 
+int mms_ctx::charge_potential(const float *m) {
+    if (p.solver == MMS_SOLVER_DIRECT) return direct_potential_of(g, direct, m, rho, phi, stream, &prof);
+    return launch_div(g, m, rho, stream, &prof) || potential(rho, phi);
+}
+
 // one fixed-dt RK4 step on the device: four (div, potential, stage) passes;
 // the stage-0 field is evaluated at M_n.  State returns to m32[cur], which
 // keeps the FP32 copy of M_n through stages 0-2 (the other two slots carry
@@ -143,13 +148,13 @@ int mms_ctx::one_step(float dt) {
     bool accept = (sur_mode == 1);
     for (int s = 0; s < 4; s++) {
         if (p.demag) {
-            if (launch_div(g, in[s], rho, stream, &prof)) return 1;
             // the learned surrogate stands in at RK4 stages 2-3; the solver
             // runs at stages 1 and 4 and, at stage 1, judges the surrogate
             const bool use_sur = sur_mode != 0 && (s == 1 || s == 2) && accept;
             if (use_sur) {
+                if (launch_div(g, in[s], rho, stream, &prof)) return 1;
                 if (surrogate_potential(sur, rho, phi, sur_rscale, sur_oscale, stream, &prof)) return 1;
-            } else if (potential(rho, phi)) {
+            } else if (charge_potential(in[s])) {
                 return 1;
             }
             if (sur_mode != 0 && s == 0) {
@@ -351,8 +356,7 @@ extern "C" int mms_sync(mms_ctx *c) {
 // field at the current state into c->h_aos (and rho/phi)
 static int field_now(mms_ctx *c, const float *m) {
     if (c->p.demag) {
-        if (launch_div(c->g, m, c->rho, c->stream, &c->prof)) return 1;
-        if (c->potential(c->rho, c->phi)) return 1;
+        if (c->charge_potential(m)) return 1;
     }
     return launch_hfield(c->g, c->mat, c->phi, m, c->t_dev, c->h_aos, c->stream, &c->prof);
 }
@@ -744,7 +748,7 @@ extern "C" int rk4_step(float t, float dt, float *t2, const unsigned char *mater
         ex.k_out = (st == 3) ? k_out : nullptr;
         ex.slope_out = (st == 3) ? s_out : nullptr;
         if (st > 0 && demag) {
-            if (launch_div(c->g, in[st], c->rho, s, &c->prof) || c->potential(c->rho, c->phi)) return EXIT_FAILURE;
+            if (c->charge_potential(in[st])) return EXIT_FAILURE;
         }
         if (launch_stage_ex(c->g, c->mat, st, (double)dt, c->phi, in[st], outp[st], c->mn64, c->acc32, c->matl,
                             c->t_dev, ex, s, &c->prof))
@@ -832,7 +836,7 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
     std::vector<float> hostM(3 * n);
     auto field_into = [&](const float *m, float *h_out) -> int {
         if (demag) {
-            if (launch_div(c->g, m, c->rho, s, &c->prof) || c->potential(c->rho, c->phi)) return 1;
+            if (c->charge_potential(m)) return 1;
         }
         return launch_hfield(c->g, c->mat, c->phi, m, c->t_dev, h_out, s, &c->prof);
     };
@@ -858,7 +862,7 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
         for (int st = 0; st < 4 && !status; st++) {
             ex.h_given = (st == 0) ? h_n : nullptr;
             if (st > 0 && demag) {
-                if (launch_div(c->g, in[st], c->rho, s, &c->prof) || c->potential(c->rho, c->phi)) { status = 1; break; }
+                if (c->charge_potential(in[st])) { status = 1; break; }
             }
             if (launch_stage_ex(c->g, c->mat, st, dt, c->phi, in[st], outp[st], c->mn64, c->acc32, c->matl, c->t_dev,
                                 ex, s, &c->prof))

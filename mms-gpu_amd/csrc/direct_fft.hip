@@ -1,0 +1,531 @@
+// direct_fft.hip -- the exact pair potential of large regular grids on gfx950
+// by FP64 transforms.
+//
+//   phi_i = (dV/dx) sum_{j != i} rho_j / |r_i - r_j|_u
+//
+// is a convolution on the grid (fmm_calc.cu:412-461 sums it pair by pair), so
+// the sum over the N^2 pairs is one zero-padded 2D transform per layer, a
+// zd x zd real product per frequency and the transform back.  Everything
+// between the FP32 charges and the FP32 potential is FP64: the error (about
+// 1e-15 of the largest potential) is far below the pair loop's FP32 sums.
+//
+// Three launches (Stockham FFTs in LDS, eight elements a thread, radix 8 with
+// one radix-2 or -4 pass; W[z][kx][y] is stored transposed so that every pass
+// reads and writes runs of consecutive y):
+//   fft_rows     charges (or div M formed in place of the charge kernel) ->
+//                x transforms, two real rows per complex transform;
+//   fft_columns  one kx per workgroup: y transforms of every layer, product
+//                with the kernel's spectrum, inverse y transforms, in place;
+//   fft_back     inverse x transforms, two real rows each, FP32 potential.
+// Measured against the pair loop (FP32 rsqrt pairs, 3.8e12 a second): the
+// 256 x 256 x 3 potential on host arrays 9.46 -> 0.11 ms, an RK4 step of a
+// 161 x 117 x 3 film 3.67 -> 0.13 ms (fft_rows 9.2 us with div M, fft_columns
+// 7.4 us, fft_back 5.8 us an evaluation: launch and load latency at this size);
+// relative error against 64 bits 5.8e-7 -> 2.5e-8.
+// A charge that is not finite would spread through the transforms; fft_rows
+// notes it and fft_back then sums that call pair by pair.
+#include "mms_internal.hpp"
+
+namespace mms {
+namespace {
+
+typedef double2 cd;
+
+constexpr int kTw = 4096;  // entries of the twiddle table, the longest transform
+
+__device__ __forceinline__ cd cmul(cd a, cd b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+__device__ __forceinline__ cd cadd(cd a, cd b) { return make_double2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ cd csub(cd a, cd b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ cd mul_mi(cd a) { return make_double2(a.y, -a.x); }  // -i a
+
+// LDS slot of element i: one free slot in nine keeps the strided stores of
+// the passes on different banks
+__device__ __forceinline__ int slot(int i) { return i + (i >> 3); }
+constexpr int slots(int n) { return n + (n >> 3); }
+
+__device__ __forceinline__ void dft4(cd &a, cd &b, cd &c, cd &d) {
+    const cd s = cadd(a, c), u = csub(a, c), v = cadd(b, d), w = mul_mi(csub(b, d));
+    a = cadd(s, v); b = cadd(u, w); c = csub(s, v); d = csub(u, w);
+}
+
+template <int R>
+__device__ __forceinline__ void dft(cd (&v)[R]) {
+    if constexpr (R == 2) {
+        const cd a = v[0];
+        v[0] = cadd(a, v[1]);
+        v[1] = csub(a, v[1]);
+    } else if constexpr (R == 4) {
+        dft4(v[0], v[1], v[2], v[3]);
+    } else {
+        const double h = 0.70710678118654752440;  // sqrt(1/2)
+        dft4(v[0], v[2], v[4], v[6]);
+        dft4(v[1], v[3], v[5], v[7]);
+        const cd t1 = make_double2(h * (v[3].x + v[3].y), h * (v[3].y - v[3].x));    // w_8 v
+        const cd t2 = mul_mi(v[5]);                                                  // w_8^2 v
+        const cd t3 = make_double2(h * (v[7].y - v[7].x), -h * (v[7].x + v[7].y));  // w_8^3 v
+        const cd e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
+        v[0] = cadd(e0, o0); v[4] = csub(e0, o0);
+        v[1] = cadd(e1, t1); v[5] = csub(e1, t1);
+        v[2] = cadd(e2, t2); v[6] = csub(e2, t2);
+        v[3] = cadd(e3, t3); v[7] = csub(e3, t3);
+    }
+}
+
+// One Stockham pass of radix R after sub-transforms of length NS; thread t of
+// the transform's N / 8.
+template <int N, int R, int NS>
+__device__ __forceinline__ void fft_pass(cd *buf, int t, const cd *__restrict__ tw) {
+    constexpr int Q = 8 / R;
+    cd v[Q][R];
+#pragma unroll
+    for (int b = 0; b < Q; b++) {
+#pragma unroll
+        for (int k = 0; k < R; k++) v[b][k] = buf[slot(t + b * (N / 8) + k * (N / R))];
+        if constexpr (NS > 1) {
+            const cd w1 = tw[((t + b * (N / 8)) & (NS - 1)) * (kTw / (NS * R))];
+            v[b][1] = cmul(v[b][1], w1);
+            if constexpr (R > 2) {
+                const cd w2 = cmul(w1, w1), w3 = cmul(w2, w1);
+                v[b][2] = cmul(v[b][2], w2);
+                v[b][3] = cmul(v[b][3], w3);
+                if constexpr (R > 4) {
+                    const cd w4 = cmul(w2, w2);
+                    v[b][4] = cmul(v[b][4], w4);
+                    v[b][5] = cmul(v[b][5], cmul(w4, w1));
+                    v[b][6] = cmul(v[b][6], cmul(w3, w3));
+                    v[b][7] = cmul(v[b][7], cmul(w4, w3));
+                }
+            }
+        }
+        dft<R>(v[b]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < Q; b++) {
+        const int j = t + b * (N / 8), jm = j & (NS - 1), base = (j - jm) * R + jm;
+#pragma unroll
+        for (int k = 0; k < R; k++) buf[slot(base + k * NS)] = v[b][k];
+    }
+    __syncthreads();
+}
+
+template <int N, int NS>
+__device__ __forceinline__ void fft_rest(cd *buf, int t, const cd *__restrict__ tw) {
+    if constexpr (NS < N) {
+        fft_pass<N, 8, NS>(buf, t, tw);
+        fft_rest<N, NS * 8>(buf, t, tw);
+    }
+}
+
+// Forward transform of buf[slot(0 .. N-1)], N a power of two >= 64; called
+// by every thread of the workgroup (the inverse: re and im swapped before
+// and after).
+template <int N>
+__device__ __forceinline__ void fft(cd *buf, int t, const cd *__restrict__ tw) {
+    constexpr int L = __builtin_ctz(N);
+    if constexpr (L % 3 == 1) {
+        fft_pass<N, 2, 1>(buf, t, tw);
+        fft_rest<N, 2>(buf, t, tw);
+    } else if constexpr (L % 3 == 2) {
+        fft_pass<N, 4, 1>(buf, t, tw);
+        fft_rest<N, 4>(buf, t, tw);
+    } else {
+        fft_rest<N, 1>(buf, t, tw);
+    }
+}
+
+// transforms per workgroup of the row kernels: at least a wave of threads
+// and, up to 2048 points, at least four consecutive rows (64-byte runs of W)
+template <int N>
+constexpr int row_batch() { return N >= 4096 ? 1 : (N >= 256 ? 2 : 512 / N); }
+
+struct FftArgs {
+    const float *rho;  // charges (fft_back's pair sum too)
+    float *rho_out;    // charges formed from m (fft_rows<N, true>)
+    const float *m;    // FP32 SoA magnetisation
+    float *phi;
+    cd *w;             // [zd][nxh][yd]
+    const double *ghat;  // [zd][nxh][ny / 2 + 1]
+    const cd *tw;
+    int *flags;        // [workgroups of fft_rows], then the combined flag
+    int nflags;
+    int xd, yd, zd, nxh, ny;
+    float dx, dy, dz, ay, az;
+    double scale;
+};
+
+template <int N, bool FROM_M>
+__global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
+    constexpr int B = row_batch<N>(), T = N / 8;
+    __shared__ cd lds[B * slots(N)];
+    const int f = threadIdx.x / T, t = threadIdx.x % T;
+    const int z = blockIdx.y, y0 = blockIdx.x * 2 * B, ya = y0 + 2 * f;
+    const long plane = (long)A.xd * A.yd, n = plane * A.zd;
+    const long row = (long)z * plane + (long)ya * A.xd;
+    bool bad = false;
+    float q[8][2];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int x = t + k * T;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            float v = 0.0f;
+            const int y = ya + h;
+            if (x < A.xd && y < A.yd) {
+                const long c = row + (long)h * A.xd + x;
+                if constexpr (FROM_M) {
+                    // div M by the charge kernel's expression (vector_functions.cpp:8-28)
+                    const float *mx = A.m, *my = A.m + n, *mz = A.m + 2 * n;
+                    const float x2 = (x != A.xd - 1) ? mx[c + 1] : 0.0f, x0 = (x != 0) ? mx[c - 1] : 0.0f;
+                    const float y2 = (y != A.yd - 1) ? my[c + A.xd] : 0.0f, yb = (y != 0) ? my[c - A.xd] : 0.0f;
+                    const float z2 = (z != A.zd - 1) ? mz[c + plane] : 0.0f, z0 = (z != 0) ? mz[c - plane] : 0.0f;
+                    v = ((x2 - x0) / A.dx + (y2 - yb) / A.dy + (z2 - z0) / A.dz) * 0.5f;
+                } else {
+                    v = A.rho[c];
+                }
+            }
+            q[k][h] = v;
+        }
+    }
+    cd *buf = lds + f * slots(N);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int x = t + k * T;
+        if constexpr (FROM_M) {
+            if (x < A.xd && ya < A.yd) A.rho_out[row + x] = q[k][0];
+            if (x < A.xd && ya + 1 < A.yd) A.rho_out[row + A.xd + x] = q[k][1];
+        }
+        bad |= !(fabsf(q[k][0]) <= 3.402823466e38f) || !(fabsf(q[k][1]) <= 3.402823466e38f);
+        buf[slot(x)] = make_double2((double)q[k][0], (double)q[k][1]);
+    }
+    const int any = __syncthreads_or(bad ? 1 : 0);
+    if (threadIdx.x == 0) A.flags[blockIdx.y * gridDim.x + blockIdx.x] = any;
+    fft<N>(buf, t, A.tw);
+    // spectra of the two real rows of each transform: with Z = FFT(a + i b),
+    // A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = (Z[k] - conj Z[N-k]) / 2i
+    for (int i = threadIdx.x; i < 2 * B * (N / 2 + 1); i += B * T) {
+        const int r = i % (2 * B), k = i / (2 * B), y = y0 + r;
+        if (y >= A.yd) continue;
+        const cd *zb = lds + (r >> 1) * slots(N);
+        const cd u = zb[slot(k)], v = zb[slot((N - k) & (N - 1))];
+        const cd s = (r & 1) ? make_double2(0.5 * (u.y + v.y), 0.5 * (v.x - u.x))
+                             : make_double2(0.5 * (u.x + v.x), 0.5 * (u.y - v.y));
+        A.w[((long)z * A.nxh + k) * A.yd + y] = s;
+    }
+}
+
+// the layers' product at one (kx, ky): out[z] = sum_z' ghat[|z - z'|] in[z'];
+// re and im are stored swapped (the inverse transform follows)
+template <int ZD, int N>
+__device__ __forceinline__ void layer_product(cd *lds, const double *__restrict__ gh, long gstride, int zd_rt) {
+    constexpr int ZM = ZD ? ZD : 16;
+    const int zd = ZD ? ZD : zd_rt;
+    cd in[ZM];
+#pragma unroll
+    for (int z = 0; z < ZM; z++)
+        if (z < zd) in[z] = lds[z * slots(N)];
+    if constexpr (ZD != 0) {
+        double g[ZM];
+#pragma unroll
+        for (int z = 0; z < ZM; z++) g[z] = gh[z * gstride];
+#pragma unroll
+        for (int z = 0; z < ZM; z++) {
+            double re = 0.0, im = 0.0;
+#pragma unroll
+            for (int s = 0; s < ZM; s++) {
+                re = fma(g[z > s ? z - s : s - z], in[s].x, re);
+                im = fma(g[z > s ? z - s : s - z], in[s].y, im);
+            }
+            lds[z * slots(N)] = make_double2(im, re);
+        }
+    } else {
+        for (int z = 0; z < zd; z++) {
+            double re = 0.0, im = 0.0;
+#pragma unroll
+            for (int s = 0; s < ZM; s++)
+                if (s < zd) {
+                    const double gv = gh[(z > s ? z - s : s - z) * gstride];
+                    re = fma(gv, in[s].x, re);
+                    im = fma(gv, in[s].y, im);
+                }
+            lds[z * slots(N)] = make_double2(im, re);
+        }
+    }
+}
+
+template <int N, int ZD>
+__global__ __launch_bounds__(ZD ? ZD * N / 8 : 1024) void fft_columns(FftArgs A) {
+    extern __shared__ __attribute__((aligned(16))) char fft_lds[];
+    cd *lds = reinterpret_cast<cd *>(fft_lds);
+    constexpr int T = N / 8;
+    const int z = threadIdx.x / T, t = threadIdx.x % T, kx = blockIdx.x;
+    cd *col = A.w + ((long)z * A.nxh + kx) * A.yd;
+    cd *buf = lds + z * slots(N);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int y = t + k * T;
+        buf[slot(y)] = y < A.yd ? col[y] : make_double2(0.0, 0.0);
+    }
+    if (kx == 0) {  // one flag for fft_back
+        int any = 0;
+        for (int i = threadIdx.x; i < A.nflags; i += blockDim.x) any |= A.flags[i];
+        any = __syncthreads_or(any);
+        if (threadIdx.x == 0) A.flags[A.nflags] = any;
+    }
+    __syncthreads();
+    fft<N>(buf, t, A.tw);
+    const long gs = (long)A.nxh * (N / 2 + 1);
+    for (int ky = threadIdx.x; ky < N; ky += blockDim.x) {
+        const double *gh = A.ghat + (long)kx * (N / 2 + 1) + (ky <= N / 2 ? ky : N - ky);
+        layer_product<ZD, N>(lds + slot(ky), gh, gs, A.zd);
+    }
+    __syncthreads();
+    fft<N>(buf, t, A.tw);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int y = t + k * T;
+        if (y < A.yd) {
+            const cd v = buf[slot(y)];
+            col[y] = make_double2(v.y, v.x);
+        }
+    }
+}
+
+// the pair sum of one target (charges that are not finite): as the pair
+// kernels form it, FP32 over 256 sources, FP64 across
+__device__ double pair_sum(const FftArgs &A, int xt, int yt, int zt) {
+    const long n = (long)A.xd * A.yd * A.zd;
+    double acc = 0.0;
+    int xs = 0, ys = 0, zs = 0;
+    for (long base = 0; base < n; base += 256) {
+        const long end = base + 256 < n ? base + 256 : n;
+        float s = 0.0f;
+        for (long j = base; j < end; j++) {
+            const float rx = (float)(xt - xs), ry = (float)(yt - ys) * A.ay, rz = (float)(zt - zs) * A.az;
+            const float r2 = rx * rx + ry * ry + rz * rz;
+            s = fmaf(A.rho[j], r2 > 0.f ? __builtin_amdgcn_rsqf(r2) : 0.f, s);
+            if (++xs == A.xd) { xs = 0; if (++ys == A.yd) { ys = 0; zs++; } }
+        }
+        acc += (double)s;
+    }
+    return acc * A.scale;
+}
+
+template <int N>
+__global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_back(FftArgs A) {
+    constexpr int B = row_batch<N>(), T = N / 8;
+    __shared__ cd lds[B * slots(N)];
+    const int f = threadIdx.x / T, t = threadIdx.x % T;
+    const int z = blockIdx.y, y0 = blockIdx.x * 2 * B, ya = y0 + 2 * f;
+    const long row = ((long)z * A.yd + ya) * A.xd;
+    if (A.flags[A.nflags]) {
+        for (int h = 0; h < 2; h++)
+            for (int x = t; x < A.xd; x += T)
+                if (ya + h < A.yd) A.phi[row + (long)h * A.xd + x] = (float)pair_sum(A, x, ya + h, z);
+        return;
+    }
+    for (int i = threadIdx.x; i < B * (N / 2 + 1); i += B * T) {
+        const int r = i % B, k = i / B, y = y0 + 2 * r;
+        const cd *p = A.w + ((long)z * A.nxh + k) * A.yd + y;
+        const cd u = y < A.yd ? p[0] : make_double2(0.0, 0.0), v = y + 1 < A.yd ? p[1] : make_double2(0.0, 0.0);
+        cd *zb = lds + r * slots(N);
+        // Z[k] = U + i V, Z[N-k] = conj(U) + i conj(V), re and im swapped
+        zb[slot(k)] = make_double2(u.y + v.x, u.x - v.y);
+        if (k > 0 && k < N / 2) zb[slot(N - k)] = make_double2(v.x - u.y, u.x + v.y);
+    }
+    __syncthreads();
+    cd *buf = lds + f * slots(N);
+    fft<N>(buf, t, A.tw);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int x = t + k * T;
+        if (x < A.xd) {
+            const cd v = buf[slot(x)];
+            if (ya < A.yd) A.phi[row + x] = (float)v.y;
+            if (ya + 1 < A.yd) A.phi[row + A.xd + x] = (float)v.x;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void fft_twiddle_kernel(cd *tw) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= kTw) return;
+    double s, c;
+    sincospi(-2.0 * (double)i / (double)kTw, &s, &c);
+    tw[i] = make_double2(c, s);
+}
+
+// Spectrum of 1/r (real and even in both axes): x transforms of the rows
+// |dy| = 0 .. ny/2 into a[dz][kx][y], then y transforms of the mirrored
+// columns, scaled.
+template <int N>
+__global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_rows(double *a, const cd *tw, int nyh, double ay,
+                                                                           double az) {
+    constexpr int T = N / 8;
+    __shared__ cd buf[slots(N)];
+    const int y = blockIdx.x, z = blockIdx.y, t = threadIdx.x % T;
+    for (int x = threadIdx.x; x < N; x += blockDim.x) {
+        const double rx = (double)(x <= N / 2 ? x : N - x), ry = y * ay, rz = z * az;
+        const double r2 = rx * rx + ry * ry + rz * rz;
+        buf[slot(x)] = make_double2(r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0, 0.0);
+    }
+    __syncthreads();
+    fft<N>(buf, t, tw);
+    for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) a[((long)z * (N / 2 + 1) + k) * nyh + y] = buf[slot(k)].x;
+}
+
+template <int N>
+__global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_columns(const double *a, double *ghat, const cd *tw,
+                                                                              int nxh, double scale) {
+    constexpr int T = N / 8;
+    __shared__ cd buf[slots(N)];
+    const int t = threadIdx.x % T;
+    const long o = ((long)blockIdx.y * nxh + blockIdx.x) * (N / 2 + 1);
+    for (int y = threadIdx.x; y < N; y += blockDim.x) buf[slot(y)] = make_double2(a[o + (y <= N / 2 ? y : N - y)], 0.0);
+    __syncthreads();
+    fft<N>(buf, t, tw);
+    for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) ghat[o + k] = buf[slot(k)].x * scale;
+}
+
+int fft_len(int d) {
+    int n = 64;
+    while (n < 2 * d - 1) n <<= 1;
+    return n;
+}
+
+#define MMS_FFT_SIZES(X, n, ...)                                                    \
+    switch (n) {                                                                    \
+    case 64: X(64, __VA_ARGS__); break;                                            \
+    case 128: X(128, __VA_ARGS__); break;                                          \
+    case 256: X(256, __VA_ARGS__); break;                                          \
+    case 512: X(512, __VA_ARGS__); break;                                          \
+    case 1024: X(1024, __VA_ARGS__); break;                                        \
+    case 2048: X(2048, __VA_ARGS__); break;                                        \
+    case 4096: X(4096, __VA_ARGS__); break;                                        \
+    default: set_error("direct sum: transform length"); return 1;                  \
+    }
+
+template <int N>
+int launch_rows(const FftArgs &A, bool from_m, hipStream_t s) {
+    constexpr int B = row_batch<N>();
+    dim3 grid((A.yd + 2 * B - 1) / (2 * B), A.zd);
+    if (from_m)
+        hipLaunchKernelGGL((fft_rows<N, true>), grid, dim3(B * N / 8), 0, s, A);
+    else
+        hipLaunchKernelGGL((fft_rows<N, false>), grid, dim3(B * N / 8), 0, s, A);
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int N, int ZD>
+int launch_columns_z(const FftArgs &A, hipStream_t s) {
+    if constexpr (ZD * N <= 8192) {
+        // set on every call (a host-side table write) rather than remembered per device
+        const size_t lds = sizeof(cd) * (size_t)A.zd * slots(N);
+        MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_columns<N, ZD>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        hipLaunchKernelGGL((fft_columns<N, ZD>), dim3(A.nxh), dim3(A.zd * (N / 8)), lds, s, A);
+        MMS_HIP(hipGetLastError());
+        return 0;
+    } else {
+        set_error("direct sum: transforms exceed LDS");
+        return 1;
+    }
+}
+
+template <int N>
+int launch_columns(const FftArgs &A, hipStream_t s) {
+    switch (A.zd) {
+    case 1: return launch_columns_z<N, 1>(A, s);
+    case 2: return launch_columns_z<N, 2>(A, s);
+    case 3: return launch_columns_z<N, 3>(A, s);
+    case 4: return launch_columns_z<N, 4>(A, s);
+    default: return launch_columns_z<N, 0>(A, s);
+    }
+}
+
+template <int N>
+int launch_back(const FftArgs &A, hipStream_t s) {
+    constexpr int B = row_batch<N>();
+    dim3 grid((A.yd + 2 * B - 1) / (2 * B), A.zd);
+    hipLaunchKernelGGL((fft_back<N>), grid, dim3(B * N / 8), 0, s, A);
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
+int row_blocks(int nx, const Grid &g) {
+    const int b = nx >= 4096 ? 1 : (nx >= 256 ? 2 : 512 / nx);
+    return ((g.yd + 2 * b - 1) / (2 * b)) * g.zd;
+}
+
+}  // namespace
+
+bool direct_fft_fits(const Grid &g) {
+    // transforms of at most 4096 points, layers of one kx together in LDS
+    // (16 bytes x zd x 9/8 ny <= 147 KB)
+    return g.xd <= 2048 && g.yd <= 2048 && g.zd <= 16 && (long)g.zd * fft_len(g.yd) <= 8192;
+}
+
+// bytes of the tables (kept by a plan) and of the work arrays; both 256-byte multiples
+size_t direct_fft_table_bytes(const Grid &g) {
+    const size_t nxh = fft_len(g.xd) / 2 + 1, nyh = fft_len(g.yd) / 2 + 1;
+    return (sizeof(cd) * kTw + sizeof(double) * g.zd * nxh * nyh + 255) & ~(size_t)255;
+}
+size_t direct_fft_work_bytes(const Grid &g) {
+    const size_t nxh = fft_len(g.xd) / 2 + 1, nyh = fft_len(g.yd) / 2 + 1;
+    const size_t w = sizeof(cd) * g.zd * nxh * g.yd, a = sizeof(double) * g.zd * nxh * nyh;
+    return ((w > a ? w : a) + sizeof(int) * (row_blocks(fft_len(g.xd), g) + 1) + 511) & ~(size_t)255;
+}
+
+int direct_fft_tables(const Grid &g, void *table, void *work, hipStream_t s) {
+    const int nx = fft_len(g.xd), ny = fft_len(g.yd), nxh = nx / 2 + 1, nyh = ny / 2 + 1;
+    cd *tw = static_cast<cd *>(table);
+    double *ghat = reinterpret_cast<double *>(tw + kTw), *a = static_cast<double *>(work);
+    const double ay = (double)g.dy / (double)g.dx, az = (double)g.dz / (double)g.dx;
+    const double scale = (double)g.dy * (double)g.dz / ((double)nx * (double)ny);
+    hipLaunchKernelGGL(fft_twiddle_kernel, dim3(kTw / 256), dim3(256), 0, s, tw);
+    MMS_HIP(hipGetLastError());
+#define X(N, ...)                                                                                                      \
+    hipLaunchKernelGGL((fft_kernel_rows<N>), dim3(nyh, g.zd), dim3(N / 8 < 64 ? 64 : N / 8), 0, s, a, tw, nyh, ay, az)
+    MMS_FFT_SIZES(X, nx, 0)
+#undef X
+    MMS_HIP(hipGetLastError());
+#define X(N, ...)                                                                                                 \
+    hipLaunchKernelGGL((fft_kernel_columns<N>), dim3(nxh, g.zd), dim3(N / 8 < 64 ? 64 : N / 8), 0, s, a, ghat, tw, \
+                       nxh, scale)
+    MMS_FFT_SIZES(X, ny, 0)
+#undef X
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
+int direct_fft_potential(const Grid &g, const void *table, void *work, const float *m, float *rho, float *phi,
+                         hipStream_t s) {
+    const int nx = fft_len(g.xd), ny = fft_len(g.yd), nxh = nx / 2 + 1, nyh = ny / 2 + 1;
+    FftArgs A{};
+    A.rho = rho; A.rho_out = rho; A.m = m; A.phi = phi;
+    A.tw = static_cast<const cd *>(table);
+    A.ghat = reinterpret_cast<const double *>(A.tw + kTw);
+    A.w = static_cast<cd *>(work);
+    const size_t w = sizeof(cd) * (size_t)g.zd * nxh * g.yd, a = sizeof(double) * (size_t)g.zd * nxh * nyh;
+    A.flags = reinterpret_cast<int *>(static_cast<char *>(work) + (((w > a ? w : a) + 15) & ~(size_t)15));
+    A.nflags = row_blocks(nx, g);
+    A.xd = g.xd; A.yd = g.yd; A.zd = g.zd; A.nxh = nxh; A.ny = ny;
+    A.dx = g.dx; A.dy = g.dy; A.dz = g.dz; A.ay = g.ay; A.az = g.az;
+    A.scale = (double)g.dy * (double)g.dz;
+#define X(N, ...) \
+    if (launch_rows<N>(A, m != nullptr, s)) return 1
+    MMS_FFT_SIZES(X, nx, 0)
+#undef X
+#define X(N, ...) \
+    if (launch_columns<N>(A, s)) return 1
+    MMS_FFT_SIZES(X, ny, 0)
+#undef X
+#define X(N, ...) \
+    if (launch_back<N>(A, s)) return 1
+    MMS_FFT_SIZES(X, nx, 0)
+#undef X
+    return 0;
+}
+
+}  // namespace mms

@@ -1,11 +1,15 @@
-// direct_sum.hip -- O(N^2) scalar potential on gfx950.
+// direct_sum.hip -- the exact pair sum of the scalar potential on gfx950.
 //
 // phi_i = (dV/dx) * sum_{j != i} rho_j / |r_i - r_j|_u   with distances in units
 // of dx (r_u = (dxi, dyi*ay, dzi*az)), the computation of the reference's
 // calc_potential_exact (fmm_calc.cu:412-461) and calc_potential_exact_kernel
 // (potential_calc.cu:18-116).
 //
-// Work split: a 2D grid of (target block of 256) x (source chunk).  A block
+// Three forms (direct_form): direct_small_kernel on a 1/r table in LDS for
+// small grids, FP64 transforms (direct_fft.hip) for larger ones, and the pair
+// loop over source chunks for grids that fit neither (very long or many layers).
+//
+// The pair loop: a 2D grid of (target block of 256) x (source chunk).  A block
 // stages its chunk through LDS in tiles of 256 sources as float4 (x, y, z,
 // rho) built from the linear index once per tile; every lane then walks the
 // tile with LDS broadcast reads (one ds_read_b128 per source per wave).  Each
@@ -26,10 +30,14 @@ namespace {
 constexpr int TB = 256;    // targets per block (one per lane)
 constexpr int TILE = 256;  // sources per LDS tile
 
-// Chunk partial sums of the entry point that allocates nothing
-// (mms_potential_exact_noalloc): 16 MiB per GPU, held until the process ends.
-constexpr long kScratchDoubles = 2L * 1024 * 1024;
-static __device__ __align__(256) double scratch[kScratchDoubles];
+// Scratch of the entry point that allocates nothing
+// (mms_potential_exact_noalloc), per GPU, held until the process ends: chunk
+// partial sums (16 MiB for its largest grids) or the transforms' tables and
+// work arrays (at most 32 bytes a cell each while no side is padded more
+// than four times; 121 MiB is the most any grid of 2,097,152 cells takes).
+constexpr long kScratchCells = 2L * 1024 * 1024;
+constexpr size_t kScratchBytes = 128u << 20;
+static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
 
 __global__ __launch_bounds__(TB) void direct_partial_kernel(const float *__restrict__ rho, double *__restrict__ part,
                                                             int xd, int yd, int zd, float ay, float az,
@@ -81,6 +89,153 @@ __global__ __launch_bounds__(256) void direct_reduce_kernel(const double *__rest
     double s = 0.0;
     for (int c = 0; c < nchunk; c++) s += part[(long)c * n + t];
     phi[t] = (float)(s * scale);
+}
+
+// Small grids: the 1/r table G[|dz|][|dy|][|dx|] (FP64 rounded once, G[0] = 0
+// excludes the cell itself) and every charge in LDS.  A thread sums four
+// consecutive x targets: their seven table entries of four sources slide
+// along the row, so four LDS words and one 16-byte charge read serve 16
+// products (the batch's table kernel reads a word per product).  A workgroup
+// takes kSmallGroups such groups and splits the source rows (in pieces of
+// kSmallRun) over 32 slices, so that a 32 x 32 x 3 film has 48 workgroups of
+// eight waves; FP32 over a piece, FP64 across pieces and slices.  With FROM_M
+// every workgroup forms all charges itself (div M, vector_functions.cpp:8-28)
+// and a separate charge launch falls away; what bounds the kernel is the
+// latency of those loads, so a thread has kSmallBatch cells' loads in flight.
+// A step of the 32 x 32 x 3 film: 128 us with charge, pair loop and reduction
+// as three launches an evaluation, 93 us so; error against 64 bits 6e-7 -> 2.8e-7.
+constexpr int kSmallGroups = 16, kSmallSlices = 32, kSmallRun = 128, kSmallBatch = 8;
+constexpr int kSmallThreads = kSmallGroups * kSmallSlices;
+// e / d for 0 <= e < 2^21 with inv = 1 / d: (e + 1/2) / d is at least 1 / 2d
+// away from an integer, the rounding at most e 2^-22 / d
+__device__ __forceinline__ int small_div(int e, float inv) { return (int)(((float)e + 0.5f) * inv); }
+struct SmallShape {
+    int xq, ts;      // row lengths in LDS: charges (4 mod 8: rows on different banks), table (odd)
+    int rows, nseg;
+};
+__host__ __device__ inline SmallShape small_shape(int xd, int yd, int zd) {
+    SmallShape h;
+    const int r4 = (xd + 3) & ~3;
+    h.xq = (r4 & 7) ? r4 : r4 + 4;
+    h.ts = xd | 1;
+    h.rows = yd * zd;
+    h.nseg = (r4 + kSmallRun - 1) / kSmallRun;
+    return h;
+}
+// the table's LDS floats: reads pass a row's end by at most 3 entries
+__host__ __device__ inline int small_table_floats(const SmallShape &h) { return (h.rows * h.ts + 7) & ~3; }
+size_t small_lds(const Grid &g) {
+    const SmallShape h = small_shape(g.xd, g.yd, g.zd);
+    const size_t q = (size_t)h.rows * h.xq, red = 2 * 4 * kSmallGroups * kSmallSlices;
+    return sizeof(float) * ((size_t)small_table_floats(h) + (q > red ? q : red));
+}
+
+__global__ __launch_bounds__(256) void small_table_kernel(float *__restrict__ tab, int xd, int yd, int zd, double ay,
+                                                          double az) {
+    const SmallShape h = small_shape(xd, yd, zd);
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= small_table_floats(h)) return;
+    const int r = e / h.ts, x = e - r * h.ts, z = r / yd, y = r - z * yd;
+    const double ry = y * ay, rz = z * az, r2 = (double)x * x + ry * ry + rz * rz;
+    tab[e] = (r < h.rows && r2 > 0.0) ? (float)(1.0 / sqrt(r2)) : 0.0f;
+}
+
+template <bool FROM_M>
+__global__ __launch_bounds__(kSmallThreads) void direct_small_kernel(const float *__restrict__ src,
+                                                                     float *__restrict__ rho_out,
+                                                                     float *__restrict__ phi,
+                                                                     const float *__restrict__ gtab, int xd, int yd,
+                                                                     int zd, float dx, float dy, float dz,
+                                                                     double scale) {
+    extern __shared__ __attribute__((aligned(16))) float slds[];
+    const SmallShape h = small_shape(xd, yd, zd);
+    const int tf = small_table_floats(h), n = xd * h.rows, nq = h.rows * h.xq, plane = xd * yd;
+    float *tab = slds, *q = slds + tf;
+    const float ixq = 1.0f / (float)h.xq, iyd = 1.0f / (float)yd;
+    for (int e0 = threadIdx.x, k0 = 0; e0 < nq; e0 += kSmallThreads * kSmallBatch, k0 += kSmallBatch) {
+        constexpr int NV = FROM_M ? 6 : 1;
+        float v[kSmallBatch][NV];
+#pragma unroll
+        for (int k = 0; k < kSmallBatch; k++) {
+            const int e = e0 + k * kSmallThreads, r = small_div(e, ixq), x = e - r * h.xq, c = r * xd + x;
+            const bool ok = e < nq && x < xd;
+            if constexpr (FROM_M) {
+                const int z = small_div(r, iyd), y = r - z * yd;
+                const float *mx = src, *my = src + n, *mz = src + 2 * n;
+                v[k][0] = (ok && x != xd - 1) ? mx[c + 1] : 0.0f;
+                v[k][1] = (ok && x != 0) ? mx[c - 1] : 0.0f;
+                v[k][2] = (ok && y != yd - 1) ? my[c + xd] : 0.0f;
+                v[k][3] = (ok && y != 0) ? my[c - xd] : 0.0f;
+                v[k][4] = (ok && z != zd - 1) ? mz[c + plane] : 0.0f;
+                v[k][5] = (ok && z != 0) ? mz[c - plane] : 0.0f;
+            } else {
+                v[k][0] = ok ? src[c] : 0.0f;
+            }
+        }
+        if (k0 == 0)  // the table, while the first charges' loads are in flight
+            for (int e = threadIdx.x; e < tf / 4; e += kSmallThreads)
+                reinterpret_cast<float4 *>(tab)[e] = reinterpret_cast<const float4 *>(gtab)[e];
+#pragma unroll
+        for (int k = 0; k < kSmallBatch; k++) {
+            const int e = e0 + k * kSmallThreads;
+            float c = v[k][0];
+            if constexpr (FROM_M) c = ((v[k][0] - v[k][1]) / dx + (v[k][2] - v[k][3]) / dy + (v[k][4] - v[k][5]) / dz) * 0.5f;
+            if (e < nq) {
+                q[e] = c;
+                if constexpr (FROM_M) {  // one workgroup writes each charge
+                    const int r = small_div(e, ixq), x = e - r * h.xq;
+                    if (x < xd && (k0 + k) % gridDim.x == blockIdx.x) rho_out[r * xd + x] = c;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    const int ngx = (xd + 3) >> 2, ngroup = ngx * h.rows;
+    const float ingx = 1.0f / (float)ngx, inseg = 1.0f / (float)h.nseg;
+    const int gi = threadIdx.x % kSmallGroups, sl = threadIdx.x / kSmallGroups;
+    const int grp = blockIdx.x * kSmallGroups + gi;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (grp < ngroup) {
+        const int rt = small_div(grp, ingx), xt = 4 * (grp - rt * ngx), zt = small_div(rt, iyd), yt = rt - zt * yd;
+        for (int it = sl; it < h.rows * h.nseg; it += kSmallSlices) {
+            const int rs = small_div(it, inseg), xs0 = (it - rs * h.nseg) * kSmallRun, zs = small_div(rs, iyd);
+            const int ys = rs - zs * yd, xs1 = xs0 + kSmallRun < xd ? xs0 + kSmallRun : xd;
+            const float *g = tab + (abs(zt - zs) * yd + abs(yt - ys)) * h.ts;
+            const float4 *qr = reinterpret_cast<const float4 *>(q + rs * h.xq);
+            // w0 .. w6 = G[|xt - xs - 3|] .. G[|xt - xs + 3|]: entries of the sources xs .. xs + 3
+            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+            int d = xt - xs0;
+            float w4 = g[abs(d + 1)], w5 = g[abs(d + 2)], w6 = g[abs(d + 3)];
+#pragma unroll 4
+            for (int xs = xs0; xs < xs1; xs += 4, d -= 4) {
+                const float4 c = qr[xs >> 2];
+                const float w0 = g[abs(d - 3)], w1 = g[abs(d - 2)], w2 = g[abs(d - 1)], w3 = g[abs(d)];
+                s0 = fmaf(c.x, w3, s0); s1 = fmaf(c.x, w4, s1); s2 = fmaf(c.x, w5, s2); s3 = fmaf(c.x, w6, s3);
+                s0 = fmaf(c.y, w2, s0); s1 = fmaf(c.y, w3, s1); s2 = fmaf(c.y, w4, s2); s3 = fmaf(c.y, w5, s3);
+                s0 = fmaf(c.z, w1, s0); s1 = fmaf(c.z, w2, s1); s2 = fmaf(c.z, w3, s2); s3 = fmaf(c.z, w4, s3);
+                s0 = fmaf(c.w, w0, s0); s1 = fmaf(c.w, w1, s1); s2 = fmaf(c.w, w2, s2); s3 = fmaf(c.w, w3, s3);
+                w4 = w0; w5 = w1; w6 = w2;
+            }
+            acc[0] += (double)s0; acc[1] += (double)s1; acc[2] += (double)s2; acc[3] += (double)s3;
+        }
+    }
+    __syncthreads();  // the charges' LDS becomes the slices' sums [slice][target]
+    double *red = reinterpret_cast<double *>(q);
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[sl * 4 * kSmallGroups + 4 * gi + i] = acc[i];
+    __syncthreads();
+    // 8 threads per target, four slices each
+    const int o = threadIdx.x >> 3, p = threadIdx.x & 7;
+    double v = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) v += red[(4 * p + k) * 4 * kSmallGroups + o];
+#pragma unroll
+    for (int m = 1; m < 8; m <<= 1) v += __shfl_xor(v, m);
+    const int go = blockIdx.x * kSmallGroups + (o >> 2);
+    if (p == 0 && go < ngroup) {
+        const int r = small_div(go, ingx), x = 4 * (go - r * ngx) + (o & 3);
+        if (x < xd) phi[r * xd + x] = (float)(v * scale);
+    }
 }
 
 // FP64 probe oracle on the device: a 2D grid of (block of 256 probes) x
@@ -371,18 +526,76 @@ static void direct_chunks(long n, int split, long *chunk, int *nchunk) {
     *nchunk = (int)((n + c - 1) / c);
 }
 
+// Which form serves a grid.  One RK4 step of a film (four evaluations and
+// stage kernels, step graph), table / transforms: 32x32x3 93 / 115 us, 40x40x3
+// 103 / 110, 48x48x3 114 / 111, 55x55x3 126 / 105, 100x30x3 138 / 117 us, so the
+// line lies at 6,000 cells.  The pair loop (37 ms a step on 161x117x3, where
+// the transforms take 1.3) keeps the grids that fit neither.
+constexpr long kTableCells = 6000;
+constexpr size_t kSmallLds = 80 * 1024;
+DirectForm direct_form(const Grid &g) {
+    const long n = g.n();
+    const bool table = n <= 16384 && small_lds(g) <= kSmallLds, fft = direct_fft_fits(g);
+    if (table && (n <= kTableCells || !fft)) return kDirectTable;
+    return fft ? kDirectFft : kDirectChunks;
+}
+
+static int small_table(const Grid &g, float *tab, hipStream_t s) {
+    const int tf = small_table_floats(small_shape(g.xd, g.yd, g.zd));
+    hipLaunchKernelGGL(small_table_kernel, dim3((tf + 255) / 256), dim3(256), 0, s, tab, g.xd, g.yd, g.zd,
+                       (double)g.dy / (double)g.dx, (double)g.dz / (double)g.dx);
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
+// m not null: the charges are formed from m and left in rho
+static int small_potential(const Grid &g, const float *tab, const float *m, float *rho, const float *rho_in, float *phi,
+                           hipStream_t s) {
+    const int groups = ((g.xd + 3) / 4) * g.yd * g.zd;
+    const dim3 grid((groups + kSmallGroups - 1) / kSmallGroups);
+    const size_t lds = small_lds(g);
+    const double scale = (double)g.dy * (double)g.dz;
+    // the attribute is set on every call (a host-side table write) rather than remembered per device
+    if (m) {
+        MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&direct_small_kernel<true>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+        hipLaunchKernelGGL(direct_small_kernel<true>, grid, dim3(kSmallThreads), lds, s, m, rho, phi, tab, g.xd, g.yd, g.zd, g.dx,
+                           g.dy, g.dz, scale);
+    } else {
+        MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&direct_small_kernel<false>),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+        hipLaunchKernelGGL(direct_small_kernel<false>, grid, dim3(kSmallThreads), lds, s, rho_in, nullptr, phi, tab, g.xd, g.yd,
+                           g.zd, g.dx, g.dy, g.dz, scale);
+    }
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
 int DirectPlan::init(const Grid &g, int split_) {
     release();
     split = (split_ == 2 || split_ == 4) ? split_ : 1;
     const long n = g.n();
-    direct_chunks(n, split, &chunk, &nchunk);
-    MMS_HIP(hipMalloc(&part, sizeof(double) * (size_t)n * nchunk));
+    form = direct_form(g);
+    if (form == kDirectTable) {
+        MMS_HIP(hipMalloc(&table, sizeof(float) * small_table_floats(small_shape(g.xd, g.yd, g.zd))));
+        if (small_table(g, static_cast<float *>(table), nullptr)) return 1;
+        MMS_HIP(hipStreamSynchronize(nullptr));
+    } else if (form == kDirectFft) {
+        MMS_HIP(hipMalloc(&table, direct_fft_table_bytes(g)));
+        MMS_HIP(hipMalloc(&work, direct_fft_work_bytes(g)));
+        if (direct_fft_tables(g, table, work, nullptr)) return 1;
+        MMS_HIP(hipStreamSynchronize(nullptr));
+    } else {
+        direct_chunks(n, split, &chunk, &nchunk);
+        MMS_HIP(hipMalloc(&work, sizeof(double) * (size_t)n * nchunk));
+    }
     return 0;
 }
 
 void DirectPlan::release() {
-    if (part) (void)hipFree(part);
-    part = nullptr;
+    if (table) (void)hipFree(table);
+    if (work) (void)hipFree(work);
+    table = work = nullptr;
     nchunk = 0;
 }
 
@@ -409,8 +622,26 @@ static int direct_launch(const Grid &g, long chunk, int nchunk, double *part, co
 
 int direct_potential(const Grid &g, DirectPlan &plan, const float *rho, float *phi, hipStream_t s,
                      Profiler *prof) {
-    MMS_CHECK(plan.part != nullptr, "direct solver plan not initialised");
-    return direct_launch(g, plan.chunk, plan.nchunk, plan.part, rho, phi, s, prof);
+    MMS_CHECK(plan.table != nullptr || plan.work != nullptr, "direct solver plan not initialised");
+    if (plan.form == kDirectChunks)
+        return direct_launch(g, plan.chunk, plan.nchunk, static_cast<double *>(plan.work), rho, phi, s, prof);
+    KTimer kt(prof, K_DIRECT);
+    if (plan.form == kDirectTable)
+        return small_potential(g, static_cast<const float *>(plan.table), nullptr, nullptr, rho, phi, s);
+    return direct_fft_potential(g, plan.table, plan.work, nullptr, const_cast<float *>(rho), phi, s);
+}
+
+int direct_potential_of(const Grid &g, DirectPlan &plan, const float *m, float *rho, float *phi, hipStream_t s,
+                        Profiler *prof) {
+    MMS_CHECK(plan.table != nullptr || plan.work != nullptr, "direct solver plan not initialised");
+    if (plan.form == kDirectChunks) {
+        if (launch_div(g, m, rho, s, prof)) return 1;
+        return direct_launch(g, plan.chunk, plan.nchunk, static_cast<double *>(plan.work), rho, phi, s, prof);
+    }
+    KTimer kt(prof, K_DIRECT);
+    if (plan.form == kDirectTable)
+        return small_potential(g, static_cast<const float *>(plan.table), m, rho, nullptr, phi, s);
+    return direct_fft_potential(g, plan.table, plan.work, m, rho, phi, s);
 }
 
 // Device address of this GPU's `scratch`, looked up once per device with
@@ -466,12 +697,12 @@ int direct_probes_f64(const Grid &g, const float *rho, const int64_t *probes, in
 
 }  // namespace mms
 
-// Direct-sum potential from device arrays without any allocation: the chunk
-// partial sums live in the file-scope `scratch` array of each GPU; the
-// kernels and the chunking are those of calc_potential_exact, so the results
-// are the same bit for bit.  Calls that overlap on one GPU share `scratch`
-// and race.  Every partial is written before it is read, so nothing has to
-// be cleared between calls.
+// Direct-sum potential from device arrays without any allocation: tables,
+// work arrays or chunk partial sums live in the file-scope `scratch` array of
+// each GPU; the form, kernels and chunking are those of calc_potential_exact,
+// so the results are the same bit for bit.  Calls that overlap on one GPU
+// share `scratch` and race.  Every value is written before it is read, so
+// nothing has to be cleared between calls.
 extern "C" int mms_potential_exact_noalloc(const float *charge_dev, float *potential_dev, int xdim, int ydim,
                                            int zdim, float dx, float dy, float dz, void *stream) {
     using namespace mms;
@@ -483,17 +714,30 @@ extern "C" int mms_potential_exact_noalloc(const float *charge_dev, float *poten
     g.dx = dx; g.dy = dy; g.dz = dz;
     g.ay = dy / dx; g.az = dz / dx;
     const long n = g.n();
+    if (n > kScratchCells) {
+        set_error("mms_potential_exact_noalloc: grid of " + std::to_string(n) + " cells exceeds the scratch (at most " +
+                  std::to_string(kScratchCells) + " cells)");
+        return 1;
+    }
+    double *mem = nullptr;
+    if (scratch_ptr(&mem)) return 1;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const DirectForm form = direct_form(g);
+    if (form == kDirectTable) {
+        float *tab = reinterpret_cast<float *>(mem);
+        if (small_table(g, tab, s)) return 1;
+        return small_potential(g, tab, nullptr, nullptr, charge_dev, potential_dev, s);
+    }
+    if (form == kDirectFft) {
+        const size_t tb = direct_fft_table_bytes(g);
+        MMS_CHECK(tb + direct_fft_work_bytes(g) <= kScratchBytes, "mms_potential_exact_noalloc: scratch too small");
+        void *work = reinterpret_cast<char *>(mem) + tb;
+        if (direct_fft_tables(g, mem, work, s)) return 1;
+        return direct_fft_potential(g, mem, work, nullptr, const_cast<float *>(charge_dev), potential_dev, s);
+    }
     long chunk = 0;
     int nchunk = 0;
     direct_chunks(n, 1, &chunk, &nchunk);
-    if (n * nchunk > kScratchDoubles) {
-        set_error("mms_potential_exact_noalloc: grid of " + std::to_string(n) + " cells needs " +
-                  std::to_string(n * nchunk) + " partial sums; the scratch holds " + std::to_string(kScratchDoubles) +
-                  " (at most 2,097,152 cells)");
-        return 1;
-    }
-    double *part = nullptr;
-    if (scratch_ptr(&part)) return 1;
-    return direct_launch(g, chunk, nchunk, part, charge_dev, potential_dev, static_cast<hipStream_t>(stream),
-                         nullptr);
+    MMS_CHECK(sizeof(double) * (size_t)(n * nchunk) <= kScratchBytes, "mms_potential_exact_noalloc: scratch too small");
+    return direct_launch(g, chunk, nchunk, mem, charge_dev, potential_dev, s, nullptr);
 }

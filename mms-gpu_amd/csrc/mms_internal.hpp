@@ -70,16 +70,35 @@ struct KTimer {
 };
 
 // --------------------------------------------------------- direct solver --
+// Forms of the exact pair sum (direct_form): small grids by the 1/r table in
+// LDS, larger ones by FP64 transforms, grids beyond both by the pair loop
+// over source chunks.
+enum DirectForm { kDirectTable = 0, kDirectFft = 1, kDirectChunks = 2 };
+DirectForm direct_form(const Grid &g);
 struct DirectPlan {
+    DirectForm form = kDirectChunks;
     int nchunk = 0;      // source chunks
     long chunk = 0;      // sources per chunk
-    double *part = nullptr;  // [nchunk][n] partial sums
-    int split = 1;           // multiplier on the number of source chunks
+    void *table = nullptr;  // 1/r table, or the transforms' tables
+    void *work = nullptr;   // the transforms' work arrays, or [nchunk][n] partial sums
+    int split = 1;          // multiplier on the number of source chunks
     int init(const Grid &g, int split = 1);
     void release();
 };
 int direct_potential(const Grid &g, DirectPlan &plan, const float *rho, float *phi,
                      hipStream_t s, Profiler *prof);
+// charge rho = div m (by the charge kernel's expression) and its potential
+int direct_potential_of(const Grid &g, DirectPlan &plan, const float *m, float *rho, float *phi, hipStream_t s,
+                        Profiler *prof);
+// FP64 transforms (direct_fft.hip): whether a grid fits them, the bytes and
+// contents of the tables and work arrays, and the potential of rho (m not
+// null: rho = div m is formed first)
+bool direct_fft_fits(const Grid &g);
+size_t direct_fft_table_bytes(const Grid &g);
+size_t direct_fft_work_bytes(const Grid &g);
+int direct_fft_tables(const Grid &g, void *table, void *work, hipStream_t s);
+int direct_fft_potential(const Grid &g, const void *table, void *work, const float *m, float *rho, float *phi,
+                         hipStream_t s);
 // the float arithmetic and summation order of the reference's CUDA direct-sum kernel
 int direct_refgpu_potential(const Grid &g, const float *rho, float *phi, hipStream_t s, Profiler *prof);
 int direct_probes_f64(const Grid &g, const float *rho, const int64_t *probes, int np,
@@ -295,5 +314,6 @@ struct mms_ctx {
     hipGraphExec_t graph = nullptr;
     float graph_dt = 0.0f;
     int potential(const float *rho_d, float *phi_d);
+    int charge_potential(const float *m);  // rho = div m and its potential phi
     int one_step(float dt);
 };
