@@ -9,7 +9,8 @@
 //
 // Layout: M stage values are FP32 SoA planes [3][n] (x plane, y plane, z plane),
 // the RK4 base M_n and the slope accumulator are FP64 SoA [3][n].  Each thread
-// owns one (x,y) column and walks z, keeping the z-1/z/z+1 values in registers;
+// owns one (x,y) column and walks z, keeping the z-1/z/z+1 values in registers
+// (on films of less than about a million cells: one cell, split_layers);
 // in-plane neighbours come from the caches (blocks are 64 x 4 columns, or
 // 256 x 8 for the four-cells-per-thread stage kernel, so the y-neighbour rows
 // of a block are resident in L1/L2).
@@ -53,7 +54,17 @@ __device__ __forceinline__ void batch_column(const int4 &t, const BatchFilm &f, 
     x = ok ? col - y * f.xd : f.xd;
 }
 
-template <int ZD>
+// The z walk of a thread: its whole column, or with SPLIT the one layer
+// blockIdx.y, whose z neighbours are then loaded like the others (the same
+// values, so the same results).
+struct Layers { int first, end; };
+template <bool SPLIT>
+__device__ __forceinline__ Layers layers(int zd) {
+    if constexpr (SPLIT) return Layers{(int)blockIdx.y, (int)blockIdx.y + 1};
+    return Layers{0, zd};
+}
+
+template <int ZD, bool SPLIT = false>
 __device__ __forceinline__ void div_column(const float *__restrict__ m, float *__restrict__ rho, int x, int y, int xd,
                                            int yd, int zd_rt, long n, float dx, float dy, float dz) {
     const int zd = ZD ? ZD : zd_rt;
@@ -61,9 +72,10 @@ __device__ __forceinline__ void div_column(const float *__restrict__ m, float *_
     const long plane = (long)xd * yd;
     const float *mx = m, *my = m + n, *mz = m + 2 * n;
     const long c0 = (long)y * xd + x;
-    float zprev = 0.0f, zcur = mz[c0];
+    const Layers zl = layers<SPLIT>(zd);
+    float zprev = (SPLIT && zl.first > 0) ? mz[c0 + (zl.first - 1) * plane] : 0.0f, zcur = mz[c0 + zl.first * plane];
 #pragma unroll
-    for (int z = 0; z < zd; z++) {
+    for (int z = zl.first; z < zl.end; z++) {
         const long c = (long)z * plane + c0;
         const float znext = (z != zd - 1) ? mz[c + plane] : 0.0f;
         const float x2 = (x != xd - 1) ? mx[c + 1] : 0.0f;
@@ -76,13 +88,13 @@ __device__ __forceinline__ void div_column(const float *__restrict__ m, float *_
     }
 }
 
-template <int ZD>
+template <int ZD, bool SPLIT>
 __global__ __launch_bounds__(BX * BY) void div_kernel(const float *__restrict__ m, float *__restrict__ rho, int xd,
                                                       int yd, int zd, float dx, float dy, float dz) {
     const int ntx = (xd + BX - 1) / BX, nty = (yd + BY - 1) / BY;
     int tx, ty;
     if (!xcd_tile(ntx, ntx * nty, tx, ty)) return;
-    div_column<ZD>(m, rho, tx * BX + threadIdx.x, ty * BY + threadIdx.y, xd, yd, zd, (long)xd * yd * zd, dx, dy, dz);
+    div_column<ZD, SPLIT>(m, rho, tx * BX + threadIdx.x, ty * BY + threadIdx.y, xd, yd, zd, (long)xd * yd * zd, dx, dy, dz);
 }
 
 // Four consecutive x cells per thread (xd a multiple of 4): 16-byte loads and
@@ -190,7 +202,7 @@ __device__ inline void llg_rhs(float Mx, float My, float Mz, float Hx, float Hy,
 // step at stage ST (field computed here, no extra outputs, M_{n+1} written
 // over the base), compiled without the per-stage branches; ST = -1: every
 // option at run time.
-template <int ZD, int ST>
+template <int ZD, int ST, bool SPLIT>
 __device__ __forceinline__ void stage_column_r(const StageArgs &A, const float *__restrict__ m_in_,
                                                float *__restrict__ m_out_, double *__restrict__ mn_,
                                                float *__restrict__ acc_, double *__restrict__ mn_out_,
@@ -222,13 +234,19 @@ __device__ __forceinline__ void stage_column_r(const StageArgs &A, const float *
     const long iyu = yu ? xd : 0, iyl = yl ? xd : 0;
 
     // z-rotation registers
+    const Layers zl = layers<SPLIT>(zd);
+    const long cf = zl.first * plane + c0;
     float pprev = 0.0f, pcur = 0.0f;
     float mxp = 0.0f, myp = 0.0f, mzp = 0.0f;
-    float mxc = mx[c0], myc = my[c0], mzc = mz[c0];
-    if (need_field && A.demag) pcur = phi_[c0];
+    float mxc = mx[cf], myc = my[cf], mzc = mz[cf];
+    if (need_field && A.demag) pcur = phi_[cf];
+    if (SPLIT && zl.first > 0) {
+        mxp = mx[cf - plane]; myp = my[cf - plane]; mzp = mz[cf - plane];
+        if (need_field && A.demag) pprev = phi_[cf - plane];
+    }
 
 #pragma unroll
-    for (int z = 0; z < zd; z++) {
+    for (int z = zl.first; z < zl.end; z++) {
         const long c = (long)z * plane + c0;
         const bool ztop = (z != zd - 1);
         float mxn = 0.0f, myn = 0.0f, mzn = 0.0f, pnext = 0.0f;
@@ -341,23 +359,23 @@ __device__ __forceinline__ void stage_column_r(const StageArgs &A, const float *
     }
 }
 
-template <int ZD, int ST>
+template <int ZD, int ST, bool SPLIT = false>
 __device__ __forceinline__ void stage_column(const StageArgs &A, int x, int y, int xd, int yd, int zd_rt, long off,
                                              long n, float hx, float hy, float hz) {
     if (x >= xd || y >= yd) return;
-    stage_column_r<ZD, ST>(A, A.m_in + off, A.m_out + off, A.mn + off, A.acc + off, A.mn_out ? A.mn_out + off : nullptr,
+    stage_column_r<ZD, ST, SPLIT>(A, A.m_in + off, A.m_out + off, A.mn + off, A.acc + off, A.mn_out ? A.mn_out + off : nullptr,
                        A.phi ? A.phi + off : nullptr, A.matl ? A.matl + off : nullptr,
                        A.m_base ? A.m_base + off : nullptr, A.m_keep ? A.m_keep + off : nullptr, A.h_given, A.h_out,
                        A.k_out, A.slope_out, x, y, xd, yd,
                        zd_rt, n, hx, hy, hz);
 }
 
-template <int ZD, int ST>
+template <int ZD, int ST, bool SPLIT>
 __global__ __launch_bounds__(BX * BY) void stage_kernel(StageArgs A) {
     const int ntx = (A.xd + BX - 1) / BX, nty = (A.yd + BY - 1) / BY;
     int tx, ty;
     if (!xcd_tile(ntx, ntx * nty, tx, ty)) return;
-    stage_column<ZD, ST>(A, tx * BX + threadIdx.x, ty * BY + threadIdx.y, A.xd, A.yd, A.zd, 0, (long)A.xd * A.yd * A.zd,
+    stage_column<ZD, ST, SPLIT>(A, tx * BX + threadIdx.x, ty * BY + threadIdx.y, A.xd, A.yd, A.zd, 0, (long)A.xd * A.yd * A.zd,
                      A.hx, A.hy, A.hz);
 }
 
@@ -596,7 +614,9 @@ __global__ __launch_bounds__(BX * BY) void hfield_kernel(StageArgs A) {
     float hex = A.hx, hey = A.hy, hez = A.hz;
     if (A.external == 1) { hex = ramp_hx(t, A.inv_mu0); hey = 0.0f; hez = 0.0f; }
     const float dx2 = A.dx * A.dx, dy2 = A.dy * A.dy, dz2 = A.dz * A.dz;
-    for (int z = 0; z < zd; z++) {
+    // one layer per grid z, or the whole column
+    const int zf = gridDim.z > 1 ? (int)blockIdx.z : 0, ze = gridDim.z > 1 ? zf + 1 : zd;
+    for (int z = zf; z < ze; z++) {
         const long c = (long)z * plane + c0;
         float Hx = 0.0f, Hy = 0.0f, Hz = 0.0f;
         if (A.demag) {
@@ -721,17 +741,17 @@ StageArgs make_args(const Grid &g, const Material &mat) {
 
 // The plain resident step runs the stage kernel compiled for its stage; a
 // stage with extra inputs or outputs runs the run-time form.
-template <int ZD>
+template <int ZD, bool SPLIT>
 void launch_stage_zd(dim3 grid, dim3 block, hipStream_t s, const StageArgs &A, bool plain) {
     if (!plain) {
-        hipLaunchKernelGGL((stage_kernel<ZD, -1>), grid, block, 0, s, A);
+        hipLaunchKernelGGL((stage_kernel<ZD, -1, SPLIT>), grid, block, 0, s, A);
         return;
     }
     switch (A.stage) {
-    case 0: hipLaunchKernelGGL((stage_kernel<ZD, 0>), grid, block, 0, s, A); break;
-    case 1: hipLaunchKernelGGL((stage_kernel<ZD, 1>), grid, block, 0, s, A); break;
-    case 2: hipLaunchKernelGGL((stage_kernel<ZD, 2>), grid, block, 0, s, A); break;
-    default: hipLaunchKernelGGL((stage_kernel<ZD, 3>), grid, block, 0, s, A);
+    case 0: hipLaunchKernelGGL((stage_kernel<ZD, 0, SPLIT>), grid, block, 0, s, A); break;
+    case 1: hipLaunchKernelGGL((stage_kernel<ZD, 1, SPLIT>), grid, block, 0, s, A); break;
+    case 2: hipLaunchKernelGGL((stage_kernel<ZD, 2, SPLIT>), grid, block, 0, s, A); break;
+    default: hipLaunchKernelGGL((stage_kernel<ZD, 3, SPLIT>), grid, block, 0, s, A);
     }
 }
 
@@ -762,11 +782,27 @@ unsigned xcd_grid(const Grid &g) {
     return (unsigned)(8 * ((ntiles + 7) / 8));
 }
 
+// Films below kSplitCells run one cell per thread, a workgroup per layer
+// (SPLIT): a thread per column leaves most CUs idle there, and a kernel lasts
+// as long as one thread's chain of dependent loads.  Four stage kernels of a
+// step, thread per column / per cell (us): 32x32x3 45.3 / 18.0, 128x128x4
+// 45.1 / 18.5, 256x256x3 46.8 / 22.1, 400x400x3 56.6 / 34.6, 512x512x3
+// 62.9 / 46.9, 705x498x4 (1.4 M cells) 92.9 / 92.3; above, the walk's fewer
+// loads count.
+constexpr long kSplitCells = 1L << 20;
+bool split_layers(const Grid &g) { return g.n() < kSplitCells; }
+
 }  // namespace
 
 int launch_div(const Grid &g, const float *m, float *rho, hipStream_t s, Profiler *prof) {
     KTimer kt(prof, K_DIV);
     dim3 block(BX, BY);
+    if (split_layers(g)) {
+        hipLaunchKernelGGL((div_kernel<0, true>), dim3(xcd_grid(g), g.zd), block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx,
+                           g.dy, g.dz);
+        MMS_HIP(hipGetLastError());
+        return 0;
+    }
     if (g.xd % 4 == 0 && ((reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(rho)) & 15) == 0) {
         const long ntiles = (long)((g.xd + 4 * BX - 1) / (4 * BX)) * ((g.yd + BY - 1) / BY);
         dim3 grid((unsigned)(8 * ((ntiles + 7) / 8)));
@@ -780,9 +816,9 @@ int launch_div(const Grid &g, const float *m, float *rho, hipStream_t s, Profile
     }
     dim3 grid(xcd_grid(g));
     switch (g.zd) {
-    case 3: hipLaunchKernelGGL(div_kernel<3>, grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz); break;
-    case 4: hipLaunchKernelGGL(div_kernel<4>, grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz); break;
-    default: hipLaunchKernelGGL(div_kernel<0>, grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz);
+    case 3: hipLaunchKernelGGL((div_kernel<3, false>), grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz); break;
+    case 4: hipLaunchKernelGGL((div_kernel<4, false>), grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz); break;
+    default: hipLaunchKernelGGL((div_kernel<0, false>), grid, block, 0, s, m, rho, g.xd, g.yd, g.zd, g.dx, g.dy, g.dz);
     }
     MMS_HIP(hipGetLastError());
     return 0;
@@ -804,10 +840,16 @@ int launch_stage_ex(const Grid &g, const Material &mat, int stage, double dt, co
     const uintptr_t al = reinterpret_cast<uintptr_t>(m_in) | reinterpret_cast<uintptr_t>(m_out) |
                          reinterpret_cast<uintptr_t>(mn) | reinterpret_cast<uintptr_t>(acc) |
                          reinterpret_cast<uintptr_t>(phi) | reinterpret_cast<uintptr_t>(ex.m_base);
-    // MMS_GPU_STAGE_ONE_CELL=1 keeps the one-cell form (the four-cell form's
-    // results are bitwise the same; the switch lets tests show it)
+    // MMS_GPU_STAGE_ONE_CELL=1 keeps the one-cell column walk (the four-cell
+    // and per-layer forms' results are bitwise the same; the switch lets tests show it)
     const char *one = std::getenv("MMS_GPU_STAGE_ONE_CELL");
-    if (plain && !(one && one[0] == '1') && g.xd % 4 == 0 && (al & 15) == 0 &&
+    const bool walk = one && one[0] == '1';
+    if (split_layers(g) && !walk) {
+        launch_stage_zd<0, true>(dim3(xcd_grid(g), g.zd), block, s, A, plain);
+        MMS_HIP(hipGetLastError());
+        return 0;
+    }
+    if (plain && !walk && g.xd % 4 == 0 && (al & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(matl) & 3) == 0) {
         const long ntiles = (long)((g.xd + 4 * BX - 1) / (4 * BX)) * ((g.yd + BY4 - 1) / BY4);
         dim3 grid4((unsigned)(8 * ((ntiles + 7) / 8))), block4(BX, BY4);
@@ -820,9 +862,9 @@ int launch_stage_ex(const Grid &g, const Material &mat, int stage, double dt, co
         return 0;
     }
     switch (g.zd) {
-    case 3: launch_stage_zd<3>(grid, block, s, A, plain); break;
-    case 4: launch_stage_zd<4>(grid, block, s, A, plain); break;
-    default: launch_stage_zd<0>(grid, block, s, A, plain);
+    case 3: launch_stage_zd<3, false>(grid, block, s, A, plain); break;
+    case 4: launch_stage_zd<4, false>(grid, block, s, A, plain); break;
+    default: launch_stage_zd<0, false>(grid, block, s, A, plain);
     }
     MMS_HIP(hipGetLastError());
     return 0;
@@ -840,7 +882,7 @@ int launch_hfield(const Grid &g, const Material &mat, const float *phi, const fl
     KTimer kt(prof, K_HFIELD);
     StageArgs A = make_args(g, mat);
     A.phi = phi; A.m_in = m; A.t_dev = t_dev; A.h_out = H_aos;
-    dim3 grid((g.xd + BX - 1) / BX, (g.yd + BY - 1) / BY), block(BX, BY);
+    dim3 grid((g.xd + BX - 1) / BX, (g.yd + BY - 1) / BY, split_layers(g) ? g.zd : 1), block(BX, BY);
     hipLaunchKernelGGL(hfield_kernel, grid, block, 0, s, A);
     MMS_HIP(hipGetLastError());
     return 0;
