@@ -369,14 +369,8 @@ extern "C" int mms_hfield(mms_ctx *c, float *H) {
     return 0;
 }
 
-// energy (eV) and torque from the AoS field h at state m (reference units)
-static int energy_torque_of(mms_ctx *c, const float *m, const float *h, double *E, double *T) {
-    const long n = c->g.n();
-    if (launch_energy_h(m, h, c->matl, n, c->red, c->red_blocks, c->stream, &c->prof)) return 1;
-    std::vector<double> part(2 * c->red_blocks);
-    MMS_HIP(hipMemcpyAsync(part.data(), c->red, sizeof(double) * 2 * c->red_blocks, hipMemcpyDeviceToHost,
-                           c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
+// energy (eV) and torque (reference units) from the energy kernel's block partials
+static void energy_torque_sum(const mms_ctx *c, const double *part, double *E, double *T) {
     double e = 0, t = 0;
     for (int i = 0; i < c->red_blocks; i++) {
         e += part[2 * i];
@@ -385,6 +379,17 @@ static int energy_torque_of(mms_ctx *c, const float *m, const float *h, double *
     const double dV = (double)(c->g.dx * c->g.dy * c->g.dz);
     *E = e * (-0.5 * (double)c->p.mu_0 * dV / 1.6e-19);
     *T = t / c->p.Ms / c->p.Ms;
+}
+
+// energy (eV) and torque from the AoS field h at state m (reference units)
+static int energy_torque_of(mms_ctx *c, const float *m, const float *h, double *E, double *T) {
+    const long n = c->g.n();
+    if (launch_energy_h(m, h, c->matl, n, c->red, c->red_blocks, c->stream, &c->prof)) return 1;
+    std::vector<double> part(2 * c->red_blocks);
+    MMS_HIP(hipMemcpyAsync(part.data(), c->red, sizeof(double) * 2 * c->red_blocks, hipMemcpyDeviceToHost,
+                           c->stream));
+    MMS_HIP(hipStreamSynchronize(c->stream));
+    energy_torque_sum(c, part.data(), E, T);
     return 0;
 }
 
@@ -773,26 +778,65 @@ extern "C" int rk4_step(float t, float dt, float *t2, const unsigned char *mater
 }
 
 // ---------------------------------------------------------- time loop --
-static int mavg_of(mms_ctx *c, const float *m, double out[5]) {
-    if (launch_mavg(m, c->matl, c->g.n(), c->red, c->red_blocks, c->stream)) return 1;
-    std::vector<double> part(5 * c->red_blocks);
-    MMS_HIP(hipMemcpyAsync(part.data(), c->red, sizeof(double) * 5 * c->red_blocks, hipMemcpyDeviceToHost, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    for (int q = 0; q < 5; q++) out[q] = 0;
-    for (int i = 0; i < c->red_blocks; i++)
-        for (int q = 0; q < 5; q++) out[q] += part[5 * i + q];
-    return 0;
-}
-
-static int write_vector3d(FILE *fh, const float *M, int zd, int yd, int xd) {
-    for (int z = 0; z < zd; z++)
-        for (int x = 0; x < xd; x++)
-            for (int y = 0; y < yd; y++) {
-                const float *v = M + 3 * ((long)z * yd * xd + (long)y * xd + x);
-                fprintf(fh, "%g %g %g \n", v[0], v[1], v[2]);
-            }
-    return 0;
-}
+// What the time loop holds on the device and the host beside the context:
+// block partials of the energy and averages, the next time value and the
+// text of the dump, in pinned memory so that their copies are enqueued and a
+// step waits for the device once.
+namespace {
+struct LoopState {
+    double *red = nullptr;  // device [2 + 5][red_blocks]
+    double *pin = nullptr;  // the same on the host, then t
+    hipEvent_t ready = nullptr;
+    TextDump text;
+    bool ramp = false;
+    int init(mms_ctx *c) {
+        MMS_HIP(hipMalloc(&red, sizeof(double) * 7 * c->red_blocks));
+        MMS_HIP(hipHostMalloc(&pin, sizeof(double) * (7 * c->red_blocks + 1), hipHostMallocDefault));
+        MMS_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
+        ramp = c->p.external == MMS_EXT_RAMP;
+        return text.init(c->g);
+    }
+    ~LoopState() {
+        if (red) (void)hipFree(red);
+        if (pin) (void)hipHostFree(pin);
+        if (ready) (void)hipEventDestroy(ready);
+        text.release();
+    }
+    // t for the ramp field (the previous copy has been waited for)
+    int set_time(mms_ctx *c, double t) {
+        c->t_host = t;
+        if (!ramp) return 0;
+        double *v = pin + 7 * c->red_blocks;
+        *v = t;
+        MMS_HIP(hipMemcpyAsync(c->t_dev, v, sizeof(double), hipMemcpyHostToDevice, c->stream));
+        return 0;
+    }
+    // energy, torque and averages of the state m with field h, enqueued
+    int reduce(mms_ctx *c, const float *m, const float *h) {
+        if (launch_energy_h(m, h, c->matl, c->g.n(), red, c->red_blocks, c->stream, &c->prof)) return 1;
+        if (launch_mavg(m, c->matl, c->g.n(), red + 2 * c->red_blocks, c->red_blocks, c->stream)) return 1;
+        MMS_HIP(hipMemcpyAsync(pin, red, sizeof(double) * 7 * c->red_blocks, hipMemcpyDeviceToHost, c->stream));
+        MMS_HIP(hipEventRecord(ready, c->stream));
+        return 0;
+    }
+    int wait() {
+        MMS_HIP(hipEventSynchronize(ready));
+        return 0;
+    }
+    void averages(const mms_ctx *c, double out[5]) const {
+        for (int q = 0; q < 5; q++) out[q] = 0;
+        for (int i = 0; i < c->red_blocks; i++)
+            for (int q = 0; q < 5; q++) out[q] += pin[2 * c->red_blocks + 5 * i + q];
+    }
+    // the dump's pieces from `first` on, one after the other
+    int dump_rest(mms_ctx *c, const float *m, FILE *fh, long first) {
+        for (; first < text.blocks; first += text.cap) {
+            if (text.enqueue(m, first, c->stream) || text.write(fh, first)) return 1;
+        }
+        return 0;
+    }
+};
+}  // namespace
 
 extern "C" int time_marching(unsigned char *material, float *M, float finaltime, float timestep, int xdim, int ydim,
                              int zdim, float dx, float dy, float dz, int P, float mu_0, float Ms, float Aexch,
@@ -833,7 +877,8 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
     double dt = timestep, t = 0.0;
     int tindex = 0, consecutive_error_count = 0;
     bool accepted = false;
-    std::vector<float> hostM(3 * n);
+    LoopState loop;
+    if (!status && loop.init(c)) status = 1;
     auto field_into = [&](const float *m, float *h_out) -> int {
         if (demag) {
             if (c->charge_potential(m)) return 1;
@@ -848,10 +893,13 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
     // non-material cells (ode_functions.cpp:165,102), so every stage and
     // accepted state holds 0 there; the initial field above used M as given
     if (!status && !c->all_magnetic && launch_zero_nonmagnetic(c->m32[c->cur], c->matl, n, s)) status = 1;
+    if (!status && energy_torque_of(c, c->m32[c->cur], h_n, &Ed, &torque0)) status = 1;
+    E = (float)Ed;
+    // a dump that fits the buffer is written while the next step runs
+    const bool defer = loop.text.blocks <= loop.text.cap;
+    bool pending = false;
     while (!status && t <= finaltime) {
-        if (mms_set_time_nolock(c, t)) { status = 1; break; }
-        if (energy_torque_of(c, c->m32[c->cur], h_n, &Ed, &torque0)) { status = 1; break; }
-        E = (float)Ed;
+        if (loop.set_time(c, t)) { status = 1; break; }
         // RK4 step: stages read/write m32 slots other than cur; stage 3
         // proposes mnew64; k1 takes the field H as given (H3 = H,
         // ode_functions.cpp:246-247), not recomputed at the current time
@@ -872,7 +920,14 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
         // post-step field H2 at the proposal (m32[d]), at the unadvanced t
         // as in the reference (ode_functions.cpp:267)
         double E2d = 0, torqued = 0;
-        if (field_into(c->m32[d], h_2) || energy_torque_of(c, c->m32[d], h_2, &E2d, &torqued)) { status = 1; break; }
+        if (field_into(c->m32[d], h_2) || loop.reduce(c, c->m32[d], h_2)) { status = 1; break; }
+        // the last accepted step's text, while this step runs; then the
+        // proposal's, taken up if the step is accepted
+        if (pending && loop.text.write(fhM, 0)) { status = 1; break; }
+        pending = false;
+        if (defer && loop.text.enqueue(c->m32[d], 0, s)) { status = 1; break; }
+        if (loop.wait()) { status = 1; break; }
+        energy_torque_sum(c, loop.pin, &E2d, &torqued);
         const float E2 = (float)E2d, torque = (float)torqued;
         if (E2 - E > .1) {
             // rejected: M and H stay as they were
@@ -896,11 +951,14 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
             c->cur = d;
             std::swap(c->mn64, c->mnew64);
             std::swap(h_n, h_2);
+            // M and H are now the proposal's, and so is the energy that the
+            // next step is held against
+            E = E2;
             // log line
             double avg[5];
-            if (mavg_of(c, c->m32[c->cur], avg)) { status = 1; break; }
-            if (mms_get_m(c, hostM.data())) { status = 1; break; }
-            write_vector3d(fhM, hostM.data(), zdim, ydim, xdim);
+            loop.averages(c, avg);
+            if (!defer && loop.dump_rest(c, c->m32[c->cur], fhM, 0)) { status = 1; break; }
+            pending = defer;
             const double cnt = avg[4] > 0 ? avg[4] : 1;
             fprintf(fh, "%d, %g, %g, %g, %g, %g, %g, %g, %g \n", tindex, t, dt, E2, avg[0] / cnt / Ms,
                     avg[1] / cnt / Ms, avg[2] / cnt / Ms, avg[3] / cnt / Ms, torque);
@@ -914,6 +972,8 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
         }
         fflush(NULL);
     }
+    if (hipStreamSynchronize(s) != hipSuccess) status = 1;
+    else if (pending && loop.text.write(fhM, 0)) status = 1;
     // M is overwritten with the last accepted state (unchanged if none was)
     if (!status && accepted && mms_get_m(c, M)) status = 1;
     fclose(fh);

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <stdio.h>
 #include <string>
 #include <vector>
 #include <map>
@@ -273,6 +274,20 @@ int launch_add_time(double *t_dev, double dt, hipStream_t s);
 // zero the FP32 SoA planes [3][n] of m on non-material cells
 int launch_zero_nonmagnetic(float *m, const uint8_t *matl, long n, hipStream_t s);
 int launch_fill_f32(float *p, float v, long n, hipStream_t s);
+
+// ------------------------------------------------------------ text dump --
+// "%g %g %g \n" lines of an FP32 SoA state in z, x, y order, formatted on the
+// device in blocks of 256 lines; at most `cap` blocks are held at a time.
+struct TextDump {
+    Grid g{};
+    long blocks = 0, cap = 0;
+    char *dev = nullptr, *pin = nullptr;
+    hipEvent_t copied = nullptr;
+    int init(const Grid &g);
+    void release();
+    int enqueue(const float *m, long first, hipStream_t s);
+    int write(FILE *fh, long first) const;
+};
 
 }  // namespace mms
 
