@@ -116,6 +116,7 @@ struct FilmDesc { int xd, yd; long off; };
 struct FilmSet { const FilmDesc *desc; long stride; int zd; };  // desc null: single film
 struct FmmPlan {
     int P = 0, K = 0, KP = 0, w = 4, Lmax = 0, Lleaf = 0, zd = 0;
+    int xd = 0, yd = 0;            // cells (a batch: the side of its size class)
     int precision = MMS_M2L_FP32;  // requested form (mms_m2l_precision)
     int m2l_mode = MMS_M2L_FP32;   // M2L operands: FP32, BF16, BF16X3 or FP16
     bool near_f16 = false;         // leaf-8 near field in scaled FP16 (else BF16 split / FP32)

@@ -56,7 +56,9 @@ __device__ __forceinline__ void batch_column(const int4 &t, const BatchFilm &f, 
 
 // The z walk of a thread: its whole column, or with SPLIT the one layer
 // blockIdx.y, whose z neighbours are then loaded like the others (the same
-// values, so the same results).
+// expressions on the same values; the compiler may fuse a multiply-add
+// differently, which after hundreds of steps shows in the last bit of a cell
+// or two in a million).
 struct Layers { int first, end; };
 template <bool SPLIT>
 __device__ __forceinline__ Layers layers(int zd) {
