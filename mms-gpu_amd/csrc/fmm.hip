@@ -605,7 +605,7 @@ __global__ __launch_bounds__(256) void down_coarse_kernel(const float *__restric
 }
 
 // -------------------------------------------------------- M2L + L2L --
-// A workgroup owns a dense TX x 16 block of target boxes (TX = 16 or 32) of one
+// A workgroup owns a dense TX x 16 block of target boxes (TX = 8, 16 or 32) of one
 // target layer; wave w handles child parity (w & 1, w >> 1): an SX x 8
 // sub-lattice (SX = TX / 2) of targets in NC = SX / 2 MFMA column tiles of 16.
 // The source window holds the tile plus a 3-box halo: (TX + 6) x 22 boxes.
@@ -1410,12 +1410,9 @@ __global__ __launch_bounds__(256) void p2p_16bit_kernel(const float *__restrict_
 }
 
 // -------------------------------------------------------------- dispatch --
-template <int KP, int MODE, int NC>
+template <int KP, int MODE, int NC, int ZP>
 int launch_m2l(const FmmPlan &pl, hipStream_t s) {
     typedef M2LCfg<KP, MODE, NC> C;
-    // target layers per staged source window (two for 16- and 32-slot blocks;
-    // 64-slot blocks need the registers of a 256-thread workgroup)
-    constexpr int ZP = (KP <= 32) ? 2 : 1;
     static int attr_done = 0;
     if (!attr_done) {
         MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&m2l_mfma_kernel<KP, MODE, NC, ZP>),
@@ -1449,14 +1446,49 @@ int launch_m2l(const FmmPlan &pl, hipStream_t s) {
     return 0;
 }
 
+// Workgroups of an M2L launch with NC column tiles and ZP target layers each.
+template <int NC>
+long m2l_groups(const FmmPlan &pl, int ZP) {
+    long tiles = 0;
+    for (int L = 2; L <= pl.Lleaf; L++) {
+        const int span = pl.w << (pl.Lleaf - L), bx = (pl.xd + span - 1) / span, by = (pl.yd + span - 1) / span;
+        tiles += (long)((bx + 4 * NC - 1) / (4 * NC)) * ((by + 15) / 16);
+    }
+    return tiles * pl.nfilm * ((pl.zd + ZP - 1) / ZP) * pl.zd;
+}
+
+// Shape of the M2L workgroups.  A workgroup's products last as long however
+// few of them there are (FP32: 11 us for 16-slot, 46 us for 32-slot blocks with
+// two layers and four column tiles, two waves on a SIMD), so launches that
+// leave CUs idle take half the columns (NC = 2), and FP32, whose products take
+// all of its time, one target layer (ZP = 1) as well.  RK4 steps in us with
+// four columns and two layers / this rule: FP32 leaf 4, 64x64x3 P 3 173 / 142,
+// 256x256x3 P 4 213 / 187, 200x200x2 P 6 390 / 231, 250x190x4 P 6 412 / 363,
+// 400x300x3 P 6 558 / 446; BF16 split leaf 8, 700x700x2 372 / 301, 512x512x2
+// 267 / 247.  kM2lFill = 600 workgroups of the narrow shape: with more, four columns are
+// as good or better (FP32 1024x1024x4 leaf 8 1856 against 1917, BF16 split
+// 1024x1024x2 441 against 472).  The scaled FP16 forms gain nothing from
+// narrower windows beyond 128 x 128 cells and keep the wide shape.
+constexpr long kM2lFill = 600;
+
 template <int KP, int MODE>
 int launch_m2l_nc(const FmmPlan &pl, hipStream_t s) {
+    // target layers per staged source window: two for 16- and 32-slot blocks
+    // (64-slot blocks need the registers of a 256-thread workgroup)
+    constexpr int ZP = (KP <= 32) ? 2 : 1;
     // wide tiles (8 column tiles per wave) when the source window fits in LDS
     if constexpr (M2LCfg<KP, MODE, 8>::lds_bytes <= 160 * 1024) {
-        if (pl.m2l_cols == 8) return launch_m2l<KP, MODE, 8>(pl, s);
+        if (pl.m2l_cols == 8) return launch_m2l<KP, MODE, 8, ZP>(pl, s);
     }
     static_assert(M2LCfg<KP, MODE, 4>::lds_bytes <= 160 * 1024, "M2L source window exceeds LDS");
-    return launch_m2l<KP, MODE, 4>(pl, s);
+    if constexpr (KP <= 32 && MODE == MMS_M2L_FP32) {
+        if (m2l_groups<2>(pl, 1) <= kM2lFill) return launch_m2l<KP, MODE, 2, 1>(pl, s);
+        return launch_m2l<KP, MODE, 4, 1>(pl, s);
+    }
+    if constexpr (KP <= 32 && MODE == MMS_M2L_BF16X3) {
+        if (m2l_groups<2>(pl, 1) <= kM2lFill) return launch_m2l<KP, MODE, 2, 2>(pl, s);
+    }
+    return launch_m2l<KP, MODE, 4, ZP>(pl, s);
 }
 
 template <int KP>

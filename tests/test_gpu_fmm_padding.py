@@ -22,3 +22,18 @@ def test_fmm_on_the_boxes_that_hold_cells(mg, dims, leaf, form, tol):
         pot = f.potential(q.ravel())
     ref = fo.FmmOracle(xd, yd, zd, 4, w=leaf).potential_units(q.astype(float)).ravel() * float(D5[0]) ** 2
     assert np.linalg.norm(pot - ref) / np.linalg.norm(ref) < tol
+
+
+# both sides of the line between the narrow and the wide M2L workgroups, one and two target layers in the last group
+@pytest.mark.parametrize("dims,P", [((96, 96, 3), 4), ((96, 96, 1), 6), ((250, 190, 4), 6), ((300, 280, 3), 6),
+                                    ((300, 280, 3), 3)])
+@pytest.mark.parametrize("form,tol", [("fp32", 2e-6), ("bf16x3", 2e-5)])
+def test_m2l_workgroup_shapes(mg, dims, P, form, tol):
+    from oracle import fmm_oracle as fo
+    xd, yd, zd = dims
+    q = (np.random.default_rng(yd).normal(size=(zd, yd, xd)) * 1e14).astype(F)
+    prec = {"fp32": mg.M2L_FP32, "bf16x3": mg.M2L_BF16X3}[form]
+    with mg.Film(*dims, *D5, solver=mg.SOLVER_FMM, P=P, m2l_precision=prec, leaf_width=4) as f:
+        pot = f.potential(q.ravel())
+    ref = fo.FmmOracle(xd, yd, zd, P, w=4).potential_units(q.astype(float)).ravel() * float(D5[0]) ** 2
+    assert np.linalg.norm(pot - ref) / np.linalg.norm(ref) < tol
