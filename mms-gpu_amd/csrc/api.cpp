@@ -118,6 +118,7 @@ static void ctx_free(mms_ctx *c) {
     for (void *b : bufs)
         if (b) (void)hipFree(b);
     c->direct.release();
+    c->refgpu.release();
     c->fmm.release();
     c->sur.release();
     if (c->phi_s) (void)hipFree(c->phi_s);
@@ -128,7 +129,7 @@ static void ctx_free(mms_ctx *c) {
 
 int mms_ctx::potential(const float *rho_d, float *phi_d) {
     if (p.solver == MMS_SOLVER_FMM) return fmm_potential(g, fmm, rho_d, phi_d, stream, &prof);
-    if (p.solver == MMS_SOLVER_DIRECT_REFGPU) return direct_refgpu_potential(g, rho_d, phi_d, stream, &prof);
+    if (p.solver == MMS_SOLVER_DIRECT_REFGPU) return direct_refgpu_potential(g, refgpu, rho_d, phi_d, stream, &prof);
     return direct_potential(g, direct, rho_d, phi_d, stream, &prof);
 }
 
@@ -214,6 +215,8 @@ extern "C" int mms_create(mms_ctx **out, const mms_params *p, const unsigned cha
         st = c->fmm.init(c->g, c->p.P, c->p.leaf_width, c->p.m2l_precision, c->p.m2l_cols);
     else if (c->p.solver == MMS_SOLVER_DIRECT)
         st = c->direct.init(c->g, c->p.direct_split);
+    else
+        st = c->refgpu.init(c->g);
     if (st) { ctx_free(c.get()); return 1; }
     *out = c.release();
     return 0;

@@ -101,7 +101,18 @@ int direct_fft_tables(const Grid &g, void *table, void *work, hipStream_t s);
 int direct_fft_potential(const Grid &g, const void *table, void *work, const float *m, float *rho, float *phi,
                          hipStream_t s);
 // the float arithmetic and summation order of the reference's CUDA direct-sum kernel
-int direct_refgpu_potential(const Grid &g, const float *rho, float *phi, hipStream_t s, Profiler *prof);
+struct RefgpuPlan {
+    double *tab = nullptr;  // 1 / r of the absolute offsets (null: the dividing kernel alone)
+    double *qd = nullptr;   // rho dV of a call, then part and need
+    float *part = nullptr;  // [split][n] sums of the partials of equal t mod split
+    int split = 4;          // 4 or 16
+    int *need = nullptr;    // 1: this call's charges need the dividing kernel
+    float qmin = 0.0f;
+    int init(const Grid &g);
+    void release();
+};
+int direct_refgpu_potential(const Grid &g, const RefgpuPlan &plan, const float *rho, float *phi, hipStream_t s,
+                            Profiler *prof);
 int direct_probes_f64(const Grid &g, const float *rho, const int64_t *probes, int np,
                       double *out, hipStream_t s, Profiler *prof);
 
@@ -316,6 +327,7 @@ struct mms_ctx {
     std::vector<unsigned char> host_matl;
     bool all_magnetic = true;       // every cell magnetic: stage kernels skip the material bytes
     mms::DirectPlan direct;
+    mms::RefgpuPlan refgpu;
     mms::FmmPlan fmm;
     mms::Profiler prof;
     // learned surrogate: 0 off, 1 at RK4 stages 2-3 always, 2 at stages 2-3

@@ -85,3 +85,46 @@ def test_transforms_leave_nonfinite_charges_to_the_pair_sum(mg, bad):
     assert np.isnan(pot[4321]) and (np.all(np.isnan(other)) if np.isnan(bad) else np.all(other == bad))
     assert mg.calc_potential_exact(q, *dims, *d, again, 1, 0) == 0
     assert np.array_equal(again, good) and np.all(np.isfinite(good))
+
+
+# the reference's order from the 1/r table: first size that takes it and the last that does not, rows shorter and
+# longer than a chunk, sources in one row or one column, a last chunk that is cut and chunks without sources
+@pytest.mark.parametrize("dims", [(64, 64, 1), (65, 63, 1), (4100, 1, 1), (1, 4100, 1), (1, 1, 4099), (37, 12, 11),
+                                  (5, 900, 1), (1025, 4, 1)])
+def test_reference_order_table_against_the_restated_kernel(mg, orc, dims):
+    n = int(np.prod(dims))
+    q = _charge(n, n)
+    q[::7] = 0.0
+    d = (F(5e-9), F(4e-9), F(3e-9))
+    pot = np.full(n, np.nan, F)
+    assert mg.calc_potential_exact_gpu(q, *dims, *d, pot) == 0, mg.last_error()
+    assert np.array_equal(pot, orc.calc_potential_exact_refgpu(q, dims, d))
+
+
+@pytest.mark.parametrize("dims", [(70, 61, 1), (512, 513, 1)])
+def test_reference_order_table_and_division_agree(mg, dims):
+    """A charge so small that its quotients are denormal sends the call to the
+    dividing kernel; it changes no sum, so both give the same bits."""
+    n = int(np.prod(dims))
+    q = _charge(n, 5)
+    q[n // 3] = 0.0
+    d = (F(5e-9),) * 3
+    a, b = np.zeros(n, F), np.zeros(n, F)
+    assert mg.calc_potential_exact_gpu(q, *dims, *d, a) == 0
+    q[n // 3] = F(1e-21)  # q dV about 1e-46, 0 in float or denormal
+    q[n // 3 + 1] = F(1e-19)
+    assert mg.calc_potential_exact_gpu(q, *dims, *d, b) == 0
+    q[n // 3 + 1] = 0.0
+    q[n // 3] = 0.0
+    assert mg.calc_potential_exact_gpu(q, *dims, *d, a) == 0
+    assert np.array_equal(a, b)
+
+
+def test_reference_order_leaves_nonfinite_charges_to_the_division(mg, orc):
+    dims, d = (80, 60, 1), (F(5e-9),) * 3
+    q = _charge(4800, 6)
+    for bad in (np.inf, np.nan):
+        q[1234] = bad
+        pot = np.zeros(4800, F)
+        assert mg.calc_potential_exact_gpu(q, *dims, *d, pot) == 0
+        assert np.array_equal(pot, orc.calc_potential_exact_refgpu(q, dims, d), equal_nan=True)
