@@ -219,6 +219,7 @@ extern "C" int mms_create(mms_ctx **out, const mms_params *p, const unsigned cha
         st = c->refgpu.init(c->g);
     if (st) { ctx_free(c.get()); return 1; }
     *out = c.release();
+    transfer_user(1);
     return 0;
 }
 
@@ -226,13 +227,14 @@ extern "C" int mms_destroy(mms_ctx *c) {
     if (!c) return 0;
     ctx_free(c);
     delete c;
+    transfer_user(-1);
     return 0;
 }
 
 static int upload_m(mms_ctx *c, const float *M) {
     const long n = c->g.n();
     float *staging = c->aux_aos;  // device AoS staging
-    MMS_HIP(hipMemcpyAsync(staging, M, sizeof(float) * 3 * n, hipMemcpyHostToDevice, c->stream));
+    if (copy_to_device(M, staging, sizeof(float) * 3 * n, c->stream)) return 1;
     if (launch_soa_from_aos(staging, c->m32[c->cur], c->mn64, n, c->stream)) return 1;
     return 0;
 }
@@ -250,17 +252,13 @@ extern "C" int mms_get_m(mms_ctx *c, float *M) {
     MMS_CHECK(c && M, "null argument");
     const long n = c->g.n();
     if (launch_aos_from_soa(c->m32[c->cur], c->aux_aos, n, c->stream)) return 1;
-    MMS_HIP(hipMemcpyAsync(M, c->aux_aos, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    return 0;
+    return copy_to_host(M, c->aux_aos, sizeof(float) * 3 * n, c->stream);
 }
 
 extern "C" int mms_set_time(mms_ctx *c, double t) {
     MMS_CHECK(c, "null context");
     c->t_host = t;
-    MMS_HIP(hipMemcpyAsync(c->t_dev, &c->t_host, sizeof(double), hipMemcpyHostToDevice, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    return 0;
+    return launch_set_time(c->t_dev, t, c->stream);
 }
 
 extern "C" int mms_steps(mms_ctx *c, int nsteps, float dt, int use_graph) {
@@ -314,11 +312,9 @@ extern "C" int mms_surrogate_potential_dev(mms_ctx *c, const float *rho_dev, flo
 extern "C" int mms_surrogate_potential(mms_ctx *c, const float *charge, float *potential) {
     MMS_CHECK(c && charge && potential, "null argument");
     const long n = c->g.n();
-    MMS_HIP(hipMemcpyAsync(c->rho, charge, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
+    if (copy_to_device(charge, c->rho, sizeof(float) * n, c->stream)) return 1;
     if (mms_surrogate_potential_dev(c, c->rho, c->phi)) return 1;
-    MMS_HIP(hipMemcpyAsync(potential, c->phi, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    return 0;
+    return copy_to_host(potential, c->phi, sizeof(float) * n, c->stream);
 }
 
 extern "C" int mms_surrogate_mode(mms_ctx *c, int mode, float tol) {
@@ -367,9 +363,7 @@ static int field_now(mms_ctx *c, const float *m) {
 extern "C" int mms_hfield(mms_ctx *c, float *H) {
     MMS_CHECK(c && H, "null argument");
     if (field_now(c, c->m32[c->cur])) return 1;
-    MMS_HIP(hipMemcpyAsync(H, c->h_aos, sizeof(float) * 3 * c->g.n(), hipMemcpyDeviceToHost, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    return 0;
+    return copy_to_host(H, c->h_aos, sizeof(float) * 3 * c->g.n(), c->stream);
 }
 
 // energy (eV) and torque (reference units) from the energy kernel's block partials
@@ -410,11 +404,9 @@ extern "C" int mms_potential_dev(mms_ctx *c, const float *rho_dev, float *phi_de
 extern "C" int mms_potential(mms_ctx *c, const float *charge, float *potential) {
     MMS_CHECK(c && charge && potential, "null argument");
     const long n = c->g.n();
-    MMS_HIP(hipMemcpyAsync(c->rho, charge, sizeof(float) * n, hipMemcpyHostToDevice, c->stream));
+    if (copy_to_device(charge, c->rho, sizeof(float) * n, c->stream)) return 1;
     if (c->potential(c->rho, c->phi)) return 1;
-    MMS_HIP(hipMemcpyAsync(potential, c->phi, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream));
-    MMS_HIP(hipStreamSynchronize(c->stream));
-    return 0;
+    return copy_to_host(potential, c->phi, sizeof(float) * n, c->stream);
 }
 
 extern "C" int mms_potential_probes_f64(mms_ctx *c, const float *charge, const int64_t *probes, int np,
@@ -703,16 +695,10 @@ extern "C" int Hfield(const float *M, float *H, float *charge, float *potential,
     const long n = c->g.n();
     if (upload_m(c, M) || mms_set_time_nolock(c, (double)t)) return EXIT_FAILURE;
     if (field_now(c, c->m32[c->cur])) return EXIT_FAILURE;
-    if (hipMemcpyAsync(H, c->h_aos, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-        return EXIT_FAILURE;
-    if (demag) {
-        if (charge && hipMemcpyAsync(charge, c->rho, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-            return EXIT_FAILURE;
-        if (potential &&
-            hipMemcpyAsync(potential, c->phi, sizeof(float) * n, hipMemcpyDeviceToHost, c->stream) != hipSuccess)
-            return EXIT_FAILURE;
-    }
-    if (hipStreamSynchronize(c->stream) != hipSuccess) { set_error("Hfield: stream failure"); return EXIT_FAILURE; }
+    const Xfer out[3] = {{H, c->h_aos, sizeof(float) * 3 * n},
+                         {demag ? charge : nullptr, c->rho, sizeof(float) * n},
+                         {demag ? potential : nullptr, c->phi, sizeof(float) * n}};
+    if (copy_to_host(out, 3, c->stream)) return EXIT_FAILURE;
     return EXIT_SUCCESS;
 }
 
@@ -732,21 +718,16 @@ extern "C" int rk4_step(float t, float dt, float *t2, const unsigned char *mater
     const long n = c->g.n();
     hipStream_t s = c->stream;
     // device staging: aux_aos = [H in | k out | slope out]; the caller's M2
-    // (FP32 SoA) goes to the unused FP64 proposal buffer: non-material cells
-    // keep it, and this_slope's, as the reference leaves them untouched there
+    // (through the slope's place) goes to the unused FP64 proposal buffer as FP32 SoA:
+    // non-material cells keep it, and this_slope's, as the reference leaves
+    // them untouched there
     float *h_in = c->aux_aos, *k_out = c->aux_aos + 3 * n, *s_out = c->aux_aos + 6 * n;
     float *m2_keep = reinterpret_cast<float *>(c->mnew64);
-    if (mms_set_time_nolock(c, (double)t)) return EXIT_FAILURE;
-    if (hipMemcpyAsync(c->h_aos, M, sizeof(float) * 3 * n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        launch_soa_from_aos(c->h_aos, c->m32[0], c->mn64, n, s) ||
-        hipMemcpyAsync(c->h_aos, M2, sizeof(float) * 3 * n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        launch_soa_from_aos(c->h_aos, m2_keep, nullptr, n, s) ||
-        hipMemcpyAsync(h_in, H, sizeof(float) * 3 * n, hipMemcpyHostToDevice, s) != hipSuccess ||
-        (this_slope &&
-         hipMemcpyAsync(k_out, this_slope, sizeof(float) * 3 * n, hipMemcpyHostToDevice, s) != hipSuccess)) {
-        set_error("rk4_step: upload failed");
+    const size_t vec = sizeof(float) * 3 * n;
+    const Xfer in_x[4] = {up(M, c->h_aos, vec), up(M2, s_out, vec), up(H, h_in, vec), up(this_slope, k_out, vec)};
+    if (mms_set_time_nolock(c, (double)t) || copy_to_device(in_x, 4, s) ||
+        launch_soa_from_aos(c->h_aos, c->m32[0], c->mn64, n, s) || launch_soa_from_aos(s_out, m2_keep, nullptr, n, s))
         return EXIT_FAILURE;
-    }
     StageExtra ex{nullptr, nullptr, nullptr, nullptr, normalize, nullptr, c->m32[0], m2_keep};
     const float *in[4] = {c->m32[0], c->m32[1], c->m32[2], c->m32[1]};
     float *outp[4] = {c->m32[1], c->m32[2], c->m32[1], c->m32[2]};
@@ -765,36 +746,32 @@ extern "C" int rk4_step(float t, float dt, float *t2, const unsigned char *mater
     // outputs
     float *m_aos = c->aux_aos;  // h_in no longer needed
     if (launch_aos_from_soa(c->m32[2], m_aos, n, s)) return EXIT_FAILURE;
-    bool ok = hipMemcpyAsync(M2, m_aos, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s) == hipSuccess &&
-              hipMemcpyAsync(H, c->h_aos, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s) == hipSuccess;
-    if (ok && slope) ok = hipMemcpyAsync(slope, s_out, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s) == hipSuccess;
-    if (ok && this_slope)
-        ok = hipMemcpyAsync(this_slope, k_out, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, s) == hipSuccess;
-    if (ok && demag && charge)
-        ok = hipMemcpyAsync(charge, c->rho, sizeof(float) * n, hipMemcpyDeviceToHost, s) == hipSuccess;
-    if (ok && demag && potential)
-        ok = hipMemcpyAsync(potential, c->phi, sizeof(float) * n, hipMemcpyDeviceToHost, s) == hipSuccess;
-    if (ok) ok = hipStreamSynchronize(s) == hipSuccess;
-    if (!ok) { set_error("rk4_step: download failed"); return EXIT_FAILURE; }
+    const Xfer out_x[6] = {{M2, m_aos, vec},
+                           {H, c->h_aos, vec},
+                           {slope, s_out, vec},
+                           {this_slope, k_out, vec},
+                           {demag ? charge : nullptr, c->rho, sizeof(float) * n},
+                           {demag ? potential : nullptr, c->phi, sizeof(float) * n}};
+    if (copy_to_host(out_x, 6, s)) return EXIT_FAILURE;
     if (t2) *t2 = t + dt;
     return EXIT_SUCCESS;
 }
 
 // ---------------------------------------------------------- time loop --
 // What the time loop holds on the device and the host beside the context:
-// block partials of the energy and averages, the next time value and the
-// text of the dump, in pinned memory so that their copies are enqueued and a
-// step waits for the device once.
+// block partials of the energy and averages and the text of the dump, in
+// pinned memory so that their copies are enqueued and a step waits for the
+// device once.
 namespace {
 struct LoopState {
     double *red = nullptr;  // device [2 + 5][red_blocks]
-    double *pin = nullptr;  // the same on the host, then t
+    double *pin = nullptr;  // the same on the host
     hipEvent_t ready = nullptr;
     TextDump text;
     bool ramp = false;
     int init(mms_ctx *c) {
         MMS_HIP(hipMalloc(&red, sizeof(double) * 7 * c->red_blocks));
-        MMS_HIP(hipHostMalloc(&pin, sizeof(double) * (7 * c->red_blocks + 1), hipHostMallocDefault));
+        MMS_HIP(hipHostMalloc(&pin, sizeof(double) * 7 * c->red_blocks, hipHostMallocDefault));
         MMS_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
         ramp = c->p.external == MMS_EXT_RAMP;
         return text.init(c->g);
@@ -805,14 +782,10 @@ struct LoopState {
         if (ready) (void)hipEventDestroy(ready);
         text.release();
     }
-    // t for the ramp field (the previous copy has been waited for)
+    // t for the ramp field
     int set_time(mms_ctx *c, double t) {
         c->t_host = t;
-        if (!ramp) return 0;
-        double *v = pin + 7 * c->red_blocks;
-        *v = t;
-        MMS_HIP(hipMemcpyAsync(c->t_dev, v, sizeof(double), hipMemcpyHostToDevice, c->stream));
-        return 0;
+        return ramp ? launch_set_time(c->t_dev, t, c->stream) : 0;
     }
     // energy, torque and averages of the state m with field h, enqueued
     int reduce(mms_ctx *c, const float *m, const float *h) {

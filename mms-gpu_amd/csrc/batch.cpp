@@ -275,6 +275,7 @@ extern "C" int mms_batch_create(mms_batch **out, const mms_params *common, int n
     b->mat.hext[0] = b->mat.hext[1] = b->mat.hext[2] = 0.0f;
     if (batch_build(b.get(), films, material)) { batch_free(b.get()); return 1; }
     *out = b.release();
+    transfer_user(1);
     return 0;
 }
 
@@ -282,12 +283,13 @@ extern "C" int mms_batch_destroy(mms_batch *b) {
     if (!b) return 0;
     batch_free(b);
     delete b;
+    transfer_user(-1);
     return 0;
 }
 
 extern "C" int mms_batch_set_m(mms_batch *b, const float *M) {
     MMS_CHECK(b && M, "null argument");
-    MMS_HIP(hipMemcpyAsync(b->aos, M, sizeof(float) * 3 * b->ntot, hipMemcpyHostToDevice, b->stream));
+    if (copy_to_device(M, b->aos, sizeof(float) * 3 * b->ntot, b->stream)) return 1;
     if (launch_soa_from_aos(b->aos, b->m32[b->cur], b->mn64, b->ntot, b->stream)) return 1;
     MMS_HIP(hipStreamSynchronize(b->stream));
     return 0;
@@ -296,9 +298,7 @@ extern "C" int mms_batch_set_m(mms_batch *b, const float *M) {
 extern "C" int mms_batch_get_m(mms_batch *b, float *M) {
     MMS_CHECK(b && M, "null argument");
     if (launch_aos_from_soa(b->m32[b->cur], b->aos, b->ntot, b->stream)) return 1;
-    MMS_HIP(hipMemcpyAsync(M, b->aos, sizeof(float) * 3 * b->ntot, hipMemcpyDeviceToHost, b->stream));
-    MMS_HIP(hipStreamSynchronize(b->stream));
-    return 0;
+    return copy_to_host(M, b->aos, sizeof(float) * 3 * b->ntot, b->stream);
 }
 
 extern "C" int mms_batch_steps(mms_batch *b, int nsteps, float dt, int use_graph) {
@@ -327,7 +327,7 @@ extern "C" int mms_batch_steps(mms_batch *b, int nsteps, float dt, int use_graph
 
 extern "C" int mms_batch_potential(mms_batch *b, const float *charge, float *potential) {
     MMS_CHECK(b && charge && potential, "null argument");
-    MMS_HIP(hipMemcpyAsync(b->rho, charge, sizeof(float) * b->ntot, hipMemcpyHostToDevice, b->stream));
+    if (copy_to_device(charge, b->rho, sizeof(float) * b->ntot, b->stream)) return 1;
     if (b->ndirect_items) {
         const double scale = (double)(b->gcommon.dx * b->gcommon.dy * b->gcommon.dz) / (double)b->gcommon.dx;
         if (direct_batch_potential(b->rho, b->phi, b->d_direct, b->ndirect_items, b->d_films, b->gcommon.ay,
@@ -336,9 +336,7 @@ extern "C" int mms_batch_potential(mms_batch *b, const float *charge, float *pot
     }
     for (size_t k = 0; k < b->fmm.size(); k++)
         if (fmm_potential(b->fmm_grid[k], *b->fmm[k], b->rho, b->phi, b->stream, &b->prof)) return 1;
-    MMS_HIP(hipMemcpyAsync(potential, b->phi, sizeof(float) * b->ntot, hipMemcpyDeviceToHost, b->stream));
-    MMS_HIP(hipStreamSynchronize(b->stream));
-    return 0;
+    return copy_to_host(potential, b->phi, sizeof(float) * b->ntot, b->stream);
 }
 
 extern "C" int mms_batch_sync(mms_batch *b) {

@@ -209,7 +209,8 @@ struct SurrogatePlan {
 long surrogate_weight_count();
 long surrogate_param_count();
 void surrogate_api_to_param(const float *api, float *param);
-void surrogate_param_to_api(const float *param, float *api);
+// device arrays: parameters in device layout -> weights in API order
+int surrogate_param_to_api(const float *param, float *api, hipStream_t s);
 // forward pass (with sp.train the pre-activations are kept for surrogate_backward)
 int surrogate_potential(SurrogatePlan &sp, const float *rho, float *phi, float rscale, float oscale, hipStream_t s,
                         Profiler *prof);
@@ -283,9 +284,31 @@ constexpr size_t kDirectTableLds = 96 * 1024;  // films whose table and charges 
 size_t direct_table_lds(int xd, int yd, int zd);
 int launch_aos_from_soa(const float *soa32, float *aos, long n, hipStream_t s);
 int launch_add_time(double *t_dev, double dt, hipStream_t s);
+int launch_set_time(double *t_dev, double t, hipStream_t s);
 // zero the FP32 SoA planes [3][n] of m on non-material cells
 int launch_zero_nonmagnetic(float *m, const uint8_t *matl, long n, hipStream_t s);
 int launch_fill_f32(float *p, float v, long n, hipStream_t s);
+
+// ------------------------------------------------------------ host copies --
+// The caller's arrays to or from the device through pinned chunks, all of a
+// call back to back, ordered on the stream; a null host array is skipped.  To
+// the device: the host arrays may be read until the stream is waited for (as
+// every entry point does before it returns).  To the host: the arrays are
+// complete.  transfer_user: +1 / -1 per live context, trainer
+// and batch (the pinned memory goes with the last).
+struct Xfer { void *host; void *dev; size_t bytes; };
+int copy_to_device(const Xfer *x, int count, hipStream_t s);
+int copy_to_host(const Xfer *x, int count, hipStream_t s);
+void transfer_user(int delta);
+inline Xfer up(const void *host, void *dev, size_t bytes) { return Xfer{const_cast<void *>(host), dev, bytes}; }
+inline int copy_to_device(const void *host, void *dev, size_t bytes, hipStream_t s) {
+    const Xfer x = up(host, dev, bytes);
+    return copy_to_device(&x, 1, s);
+}
+inline int copy_to_host(void *host, const void *dev, size_t bytes, hipStream_t s) {
+    const Xfer x{host, const_cast<void *>(dev), bytes};
+    return copy_to_host(&x, 1, s);
+}
 
 // ------------------------------------------------------------ text dump --
 // "%g %g %g \n" lines of an FP32 SoA state in z, x, y order, formatted on the

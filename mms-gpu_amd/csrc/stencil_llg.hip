@@ -717,6 +717,7 @@ __global__ void zero_nonmagnetic_kernel(float *__restrict__ m, const uint8_t *__
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256L)
         if (!matl[i]) { m[i] = 0.0f; m[n + i] = 0.0f; m[2 * n + i] = 0.0f; }
 }
+__global__ void set_time_kernel(double *t, double v) { *t = v; }
 __global__ void add_time_kernel(double *t, double dt) { *t += dt; }
 __global__ void fill_f32_kernel(float *p, float v, long n) {
     for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += (long)gridDim.x * 256L) p[i] = v;
@@ -947,6 +948,11 @@ int launch_aos_from_soa(const float *soa32, float *aos, long n, hipStream_t s) {
 }
 int launch_zero_nonmagnetic(float *m, const uint8_t *matl, long n, hipStream_t s) {
     hipLaunchKernelGGL(zero_nonmagnetic_kernel, dim3(grid1d(n)), dim3(256), 0, s, m, matl, n);
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+int launch_set_time(double *t_dev, double t, hipStream_t s) {
+    hipLaunchKernelGGL(set_time_kernel, dim3(1), dim3(1), 0, s, t_dev, t);
     MMS_HIP(hipGetLastError());
     return 0;
 }

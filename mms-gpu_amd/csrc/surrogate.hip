@@ -1163,28 +1163,31 @@ void surrogate_api_to_param(const float *api, float *prm) {
     std::copy(api + o, api + o + C + 1, prm + OFF_WP);
 }
 
-void surrogate_param_to_api(const float *prm, float *api) {
-    long o = 0;
-    for (int co = 0; co < C; co++)
-        for (int pl = 0; pl < 3; pl++)
-            for (int tap = 0; tap < 9; tap++) api[o + (co * 3 + pl) * 9 + tap] = prm[OFF_L + co * 32 + tap * 3 + pl];
-    o += C * 27;
-    for (int co = 0; co < C; co++) api[o + co] = prm[OFF_BL + co];
-    o += C;
-    auto conv = [&](long off) {
-        for (int co = 0; co < C; co++)
-            for (int ci = 0; ci < C; ci++)
-                for (int tap = 0; tap < 9; tap++) api[o + (co * C + ci) * 9 + tap] = prm[off + ((long)tap * C + co) * C + ci];
-        o += CONVN;
-        for (int co = 0; co < C; co++) api[o + co] = prm[off + CONVN + co];
-        o += C;
+// One thread per weight: device layout -> API order (the inverse of surrogate_api_to_param).
+__global__ __launch_bounds__(256) void sur_to_api_kernel(const float *__restrict__ prm, float *__restrict__ api, long n) {
+    const long e = blockIdx.x * 256L + threadIdx.x;
+    if (e >= n) return;
+    constexpr long NL = C * 27, NB = CONVN + C, OA1 = NL + C, OA2 = OA1 + NB, OAM = OA2 + NB, OA3 = OAM + 1024L * C * C,
+                   OAP = OA3 + NB;
+    auto conv = [&](long off, long o) {  // [co][ci][tap] <- [tap][co][ci], then the biases
+        return o < CONVN ? off + ((o % 9) * C + o / 9 / C) * C + (o / 9) % C : off + o;
     };
-    conv(OFF_W1);
-    conv(OFF_W2);
-    std::copy(prm + OFF_WM, prm + OFF_WM + 1024L * C * C, api + o);
-    o += 1024L * C * C;
-    conv(OFF_W3);
-    std::copy(prm + OFF_WP, prm + OFF_WP + C + 1, api + o);
+    long src;
+    if (e < NL) src = OFF_L + e / 27 * 32 + (e % 9) * 3 + (e % 27) / 9;
+    else if (e < OA1) src = OFF_BL + (e - NL);
+    else if (e < OA2) src = conv(OFF_W1, e - OA1);
+    else if (e < OAM) src = conv(OFF_W2, e - OA2);
+    else if (e < OA3) src = OFF_WM + (e - OAM);
+    else if (e < OAP) src = conv(OFF_W3, e - OA3);
+    else src = OFF_WP + (e - OAP);
+    api[e] = prm[src];
+}
+
+int surrogate_param_to_api(const float *prm, float *api, hipStream_t s) {
+    const long n = surrogate_weight_count();
+    hipLaunchKernelGGL(sur_to_api_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, prm, api, n);
+    MMS_HIP(hipGetLastError());
+    return 0;
 }
 
 int SurrogatePlan::init(const Grid &g_, int zf_, const float *weights, bool train_, hipStream_t s) {

@@ -102,7 +102,7 @@ struct mms_sur_trainer {
     long npf = 0;
     hipStream_t stream = nullptr;
     SurrogatePlan sp;
-    float *d_m = nullptr, *d_v = nullptr, *d_grad = nullptr;
+    float *d_m = nullptr, *d_v = nullptr, *d_grad = nullptr, *d_api = nullptr;  // d_api: a download in API order
     long step = 0;
     // training set [cap][npf] and 1 / sum phi^2 per pair
     long npairs = 0, cap = 0;
@@ -116,11 +116,13 @@ struct mms_sur_trainer {
     ~mms_sur_trainer() {
         if (solver) mms_destroy(solver);
         sp.release();
-        void *bufs[] = {d_m, d_v, d_grad, d_rho, d_phi, d_brho, d_bphi, d_bphs, d_binv};
+        void *bufs[] = {d_m, d_v, d_grad, d_api, d_rho, d_phi, d_brho, d_bphi, d_bphs, d_binv};
         for (void *b : bufs)
             if (b) (void)hipFree(b);
         if (stream) (void)hipStreamDestroy(stream);
+        transfer_user(-1);
     }
+    mms_sur_trainer() { transfer_user(1); }
 };
 
 namespace {
@@ -180,6 +182,12 @@ int gradient(mms_sur_trainer *t, const long *idx, double *loss) {
     return 0;
 }
 
+// parameters or gradient to the host in API order
+int download(mms_sur_trainer *t, const float *param, float *api) {
+    if (surrogate_param_to_api(param, t->d_api, t->stream)) return 1;
+    return copy_to_host(api, t->d_api, sizeof(float) * surrogate_weight_count(), t->stream);
+}
+
 }  // namespace
 
 extern "C" int mms_surrogate_trainer_create(mms_sur_trainer **out, int xdim, int ydim, int zdim, float dx, float Ms,
@@ -203,6 +211,7 @@ extern "C" int mms_surrogate_trainer_create(mms_sur_trainer **out, int xdim, int
     MMS_HIP(hipMalloc(&t->d_m, sizeof(float) * np));
     MMS_HIP(hipMalloc(&t->d_v, sizeof(float) * np));
     MMS_HIP(hipMalloc(&t->d_grad, sizeof(float) * np));
+    MMS_HIP(hipMalloc(&t->d_api, sizeof(float) * surrogate_weight_count()));
     MMS_HIP(hipMemsetAsync(t->d_m, 0, sizeof(float) * np, t->stream));
     MMS_HIP(hipMemsetAsync(t->d_v, 0, sizeof(float) * np, t->stream));
     MMS_HIP(hipMemsetAsync(t->d_grad, 0, sizeof(float) * np, t->stream));
@@ -263,11 +272,9 @@ extern "C" int mms_surrogate_trainer_add(mms_sur_trainer *t, int npairs, const f
     MMS_CHECK(t && npairs >= 0 && charge && potential, "bad argument");
     if (reserve(t, t->npairs + npairs)) return 1;
     const long n = t->npf;
-    MMS_HIP(hipMemcpyAsync(t->d_rho + t->npairs * n, charge, sizeof(float) * npairs * n, hipMemcpyHostToDevice,
-                           t->stream));
-    MMS_HIP(hipMemcpyAsync(t->d_phi + t->npairs * n, potential, sizeof(float) * npairs * n, hipMemcpyHostToDevice,
-                           t->stream));
-    MMS_HIP(hipStreamSynchronize(t->stream));
+    const Xfer x[2] = {up(charge, t->d_rho + t->npairs * n, sizeof(float) * npairs * n),
+                       up(potential, t->d_phi + t->npairs * n, sizeof(float) * npairs * n)};
+    if (copy_to_device(x, 2, t->stream)) return 1;
     for (int k = 0; k < npairs; k++) {
         t->npairs++;
         if (append_norm(t, t->npairs - 1)) return 1;
@@ -291,12 +298,7 @@ extern "C" int mms_surrogate_trainer_get_pair(mms_sur_trainer *t, long i, float 
 extern "C" int mms_surrogate_trainer_gradient(mms_sur_trainer *t, const long *idx, float *grad, double *loss) {
     MMS_CHECK(t, "null trainer");
     if (gradient(t, idx, loss)) return 1;
-    if (grad) {
-        std::vector<float> g((size_t)surrogate_param_count());
-        MMS_HIP(hipMemcpy(g.data(), t->d_grad, sizeof(float) * g.size(), hipMemcpyDeviceToHost));
-        surrogate_param_to_api(g.data(), grad);
-    }
-    return 0;
+    return grad ? download(t, t->d_grad, grad) : 0;
 }
 
 extern "C" int mms_surrogate_trainer_step(mms_sur_trainer *t, const long *idx, float lr, double *loss) {
@@ -325,17 +327,11 @@ extern "C" int mms_surrogate_trainer_eval(mms_sur_trainer *t, const long *idx, d
 
 extern "C" int mms_surrogate_trainer_weights(mms_sur_trainer *t, float *weights) {
     MMS_CHECK(t && weights, "bad argument");
-    std::vector<float> p((size_t)surrogate_param_count());
-    MMS_HIP(hipStreamSynchronize(t->stream));
-    MMS_HIP(hipMemcpy(p.data(), t->sp.d_param, sizeof(float) * p.size(), hipMemcpyDeviceToHost));
-    surrogate_param_to_api(p.data(), weights);
-    return 0;
+    return download(t, t->sp.d_param, weights);
 }
 
 extern "C" int mms_surrogate_trainer_predict(mms_sur_trainer *t, const long *idx, float *potential) {
     MMS_CHECK(t && potential, "bad argument");
     if (forward_batch(t, idx)) return 1;
-    MMS_HIP(hipMemcpyAsync(potential, t->d_bphs, sizeof(float) * t->npf * t->batch, hipMemcpyDeviceToHost, t->stream));
-    MMS_HIP(hipStreamSynchronize(t->stream));
-    return 0;
+    return copy_to_host(potential, t->d_bphs, sizeof(float) * t->npf * t->batch, t->stream);
 }
