@@ -1196,6 +1196,17 @@ __global__ __launch_bounds__(256) void p2p_mfma_kernel(const float *__restrict__
 // the FP16 conversion and the sums by 1 / s afterwards (exact), the 1/r
 // operator (values in (0, 1]) is stored as plain FP16.
 // The downward pass adds the far field afterwards.
+// Bound by the matrix pipe once its operands are there (1024 x 1024 x 4, FP16
+// hi/lo operator: 15.4 us of products, about 8 us of window staging, a launch)
+// if each step's operands (operators from the L2, window from LDS) are
+// requested before the products of the step before.  The compiler's scheduler
+// moves loads down to their first use, where each step waits for them;
+// sched_barrier around the products keeps them apart: 42.9 -> 39.0 us there,
+// 33.6 -> 27.7 us on 705 x 498 x 4 in the BF16 form.  Operators two to four
+// steps ahead take no less and cost registers that the M2L workgroups beside
+// this kernel need (1024 x 1024 x 4 step 699 -> 717 us).
+// The window is read in groups of four x neighbours with the addresses
+// formed once for all layers (one cell at a time: 47.3 and 37.2 us).
 // NF: 0 = BF16 hi/lo split of operator and charges (3 products), 1 = scaled
 // FP16 operator and charges (1 product), 2 = FP16 hi/lo split of the operator
 // against the scaled FP16 charges (2 products).
@@ -1221,39 +1232,69 @@ __global__ __launch_bounds__(256) void p2p_16bit_kernel(const float *__restrict_
     const int x0 = blockIdx.x * TWX, y0 = blockIdx.y * TWY;
     const long plane = (long)xd * yd;
     float inv_s = 1.0f;
+    // The window of a layer in groups of four x neighbours: NK groups a
+    // thread, at the same rows and columns in every layer.
+    constexpr int QX = SWX / 4, NQ = SWY * QX, NK = (NQ + 255) / 256;
+    int goff[NK], loff[NK];  // global offset of the group (-1: outside the film), LDS offset (-1: no group)
+    int gxk[NK];
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+        const int e = threadIdx.x + 256 * k, row = e / QX, q = e - row * QX;
+        const int gx = x0 - W + 4 * q, gy = y0 - W + row;
+        loff[k] = e < NQ ? row * SP + 4 * q : -1;
+        goff[k] = (e < NQ && gx >= 0 && gx < xd && gy >= 0 && gy < yd) ? gy * xd + gx : -1;
+        gxk[k] = gx;
+    }
+    // whole 16-byte groups when rows and layers start on 16 bytes
+    const bool vec = (xd & 3) == 0 && (reinterpret_cast<size_t>(rho) & 15) == 0;  // uniform
+    auto ld = [&](int k, int zs) {
+        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (goff[k] < 0 || zs >= zd) return v;
+        const float *p = rho + (long)zs * plane + goff[k];
+        if (vec) return *reinterpret_cast<const f32x4 *>(p);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            if (gxk[k] + t < xd) v[t] = p[t];
+        return v;
+    };
+    auto pack = [](unsigned short h0, unsigned short h1, unsigned short h2, unsigned short h3) {
+        return make_uint2(h0 | ((unsigned)h1 << 16), h2 | ((unsigned)h3 << 16));
+    };
     if constexpr (F16) {
-        // The window's largest |charge| fixes the scale: up to 4 layers
-        // (64 charges per thread) the window is loaded once into registers,
-        // deeper films read it twice (maximum, then the scaled values).
-        constexpr int BATCH = 16, HOLD = 64;
-        const int ne = zd * SWY * SWX;
-        auto ld = [&](int e) {  // e >= ne reads nothing and returns 0
-            const int zs = e / (SWY * SWX), r = e % (SWY * SWX), sy = r / SWX, sx = r % SWX;
-            const int gx = x0 - W + sx, gy = y0 - W + sy;
-            return (e < ne && gx >= 0 && gx < xd && gy >= 0 && gy < yd) ? rho[(long)zs * plane + (long)gy * xd + gx]
-                                                                      : 0.0f;
+        // The window's largest |charge| fixes the scale: up to 4 layers the
+        // window is loaded once into registers, deeper films read it twice
+        // (maximum, then the scaled values).
+        auto st = [&](int k, int zs, f32x4 v, float sc) {
+            if (loff[k] < 0 || zs >= zd) return;
+            unsigned short h[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) h[t] = __builtin_bit_cast(unsigned short, (_Float16)(v[t] * sc));
+            *reinterpret_cast<uint2 *>(qh + zs * SWY * SP + loff[k]) = pack(h[0], h[1], h[2], h[3]);
         };
-        auto st = [&](int e, float v, float sc) {
-            if (e >= ne) return;
-            const int zs = e / (SWY * SWX), r = e % (SWY * SWX), sy = r / SWX, sx = r % SWX;
-            qh[(zs * SWY + sy) * SP + sx] = __builtin_bit_cast(unsigned short, (_Float16)(v * sc));
+        auto amax = [](float m, f32x4 v) {
+            return fmaxf(fmaxf(m, fmaxf(fabsf(v[0]), fabsf(v[1]))), fmaxf(fabsf(v[2]), fabsf(v[3])));
         };
-        const bool hold = ne <= 256 * HOLD;  // uniform
-        float vh[HOLD];
+        constexpr int HOLD = 4;  // layers
+        const bool hold = zd <= HOLD;  // uniform
+        f32x4 vh[HOLD][NK];
         float mx = 0.0f;
         if (hold) {
 #pragma unroll
-            for (int k = 0; k < HOLD; k++) vh[k] = ld(threadIdx.x + 256 * k);
+            for (int z = 0; z < HOLD; z++)
 #pragma unroll
-            for (int k = 0; k < HOLD; k++) mx = fmaxf(mx, fabsf(vh[k]));
+                for (int k = 0; k < NK; k++) vh[z][k] = ld(k, z);
+#pragma unroll
+            for (int z = 0; z < HOLD; z++)
+#pragma unroll
+                for (int k = 0; k < NK; k++) mx = amax(mx, vh[z][k]);
         } else {
-#pragma unroll 1
-            for (int e0 = 0; e0 < ne; e0 += 256 * BATCH) {
-                float vb[BATCH];
+#pragma unroll 2
+            for (int z = 0; z < zd; z++) {
+                f32x4 vb[NK];
 #pragma unroll
-                for (int k = 0; k < BATCH; k++) vb[k] = ld(e0 + threadIdx.x + 256 * k);
+                for (int k = 0; k < NK; k++) vb[k] = ld(k, z);
 #pragma unroll
-                for (int k = 0; k < BATCH; k++) mx = fmaxf(mx, fabsf(vb[k]));
+                for (int k = 0; k < NK; k++) mx = amax(mx, vb[k]);
             }
         }
 #pragma unroll
@@ -1269,40 +1310,42 @@ __global__ __launch_bounds__(256) void p2p_16bit_kernel(const float *__restrict_
         inv_s = __uint_as_float((unsigned)(127 - es) << 23);
         if (hold) {
 #pragma unroll
-            for (int k = 0; k < HOLD; k++) st(threadIdx.x + 256 * k, vh[k], sc);
+            for (int z = 0; z < HOLD; z++)
+#pragma unroll
+                for (int k = 0; k < NK; k++) st(k, z, vh[z][k], sc);
         } else {
-#pragma unroll 1
-            for (int e0 = 0; e0 < ne; e0 += 256 * BATCH) {
-                float vb[BATCH];
+#pragma unroll 2
+            for (int z = 0; z < zd; z++) {
+                f32x4 vb[NK];
 #pragma unroll
-                for (int k = 0; k < BATCH; k++) vb[k] = ld(e0 + threadIdx.x + 256 * k);
+                for (int k = 0; k < NK; k++) vb[k] = ld(k, z);
 #pragma unroll
-                for (int k = 0; k < BATCH; k++) st(e0 + threadIdx.x + 256 * k, vb[k], sc);
+                for (int k = 0; k < NK; k++) st(k, z, vb[k], sc);
             }
         }
-    } else {   // charges of the window, 16 loads per thread in flight per batch
-        constexpr int BATCH = 16;
-        const int ne = zd * SWY * SWX;
+    } else {   // charges of the window, four layers' loads in flight
 #pragma unroll 1
-        for (int e0 = 0; e0 < ne; e0 += 256 * BATCH) {
-            float vb[BATCH];
+        for (int z0 = 0; z0 < zd; z0 += 4) {
+            f32x4 vb[4][NK];
 #pragma unroll
-            for (int k = 0; k < BATCH; k++) {
-                const int e = e0 + threadIdx.x + 256 * k;
-                const int zs = e / (SWY * SWX), r = e % (SWY * SWX), sy = r / SWX, sx = r % SWX;
-                const int gx = x0 - W + sx, gy = y0 - W + sy;
-                vb[k] = (e < ne && gx >= 0 && gx < xd && gy >= 0 && gy < yd) ? rho[(long)zs * plane + (long)gy * xd + gx]
-                                                                             : 0.0f;
-            }
+            for (int z = 0; z < 4; z++)
 #pragma unroll
-            for (int k = 0; k < BATCH; k++) {
-                const int e = e0 + threadIdx.x + 256 * k;
-                if (e >= ne) break;
-                const int zs = e / (SWY * SWX), r = e % (SWY * SWX), sy = r / SWX, sx = r % SWX;
-                const unsigned short h = f2bf(vb[k]);
-                qh[(zs * SWY + sy) * SP + sx] = h;
-                ql[(zs * SWY + sy) * SP + sx] = f2bf(vb[k] - bf2f(h));
-            }
+                for (int k = 0; k < NK; k++) vb[z][k] = ld(k, z0 + z);
+#pragma unroll
+            for (int z = 0; z < 4; z++)
+#pragma unroll
+                for (int k = 0; k < NK; k++) {
+                    if (loff[k] < 0 || z0 + z >= zd) continue;
+                    unsigned short h[4], l[4];
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        h[t] = f2bf(vb[z][k][t]);
+                        l[t] = f2bf(vb[z][k][t] - bf2f(h[t]));
+                    }
+                    const int o = (z0 + z) * SWY * SP + loff[k];
+                    *reinterpret_cast<uint2 *>(qh + o) = pack(h[0], h[1], h[2], h[3]);
+                    *reinterpret_cast<uint2 *>(ql + o) = pack(l[0], l[1], l[2], l[3]);
+                }
         }
     }
     __syncthreads();
@@ -1313,6 +1356,37 @@ __global__ __launch_bounds__(256) void p2p_16bit_kernel(const float *__restrict_
         for (int r = 0; r < RT; r++)
 #pragma unroll
             for (int c = 0; c < NCB; c++) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // Operators (hi, lo) by ph and index - 14 ph, window fragments by the
+        // step's parity.  All indices are constants once the steps are
+        // unrolled, and only the current and the next step's are live: registers.
+        BV Oh[3][14], Ol[3][14], bh[2][NCB], bl[2][NCB];
+        auto op_layer = [&](int zt, int zs) {
+            const int dzi = (zs > zt ? zs - zt : zt - zs) + zd - 1;  // 1/r is even in dz
+            return reinterpret_cast<const BV *>(afrag) + (long)dzi * 42 * 2 * 64 + lane;
+        };
+        auto loadA = [&](BV (&h)[14], BV (&l)[14], const BV *A, int st) {
+            const int ph = st / 6, aa = st % 6;
+#pragma unroll
+            for (int i = aa ? 2 * aa + 2 : 0; i < 2 * aa + 4; i++) {
+                h[i] = A[(14 * ph + i) * 2 * 64];
+                if constexpr (OP_LO) l[i] = A[((14 * ph + i) * 2 + 1) * 64];
+            }
+        };
+        auto loadB = [&](BV (&h)[NCB], BV (&l)[NCB], int base, int st) {
+            // lane group g reads 8 sources of window row 4 aa + srow at column scol
+            const int ph = st / 6, aa = st % 6, fl = 32 * ph + 8 * g, srow = fl / 24, scol = fl % 24;
+            const int ro = base + (4 * aa + srow) * SP + scol;
+#pragma unroll
+            for (int c = 0; c < NCB; c++) {
+                const int jx = 4 * c + (j16 & 3);
+                h[c] = *reinterpret_cast<const BV *>(qh + ro + W * jx);
+                if constexpr (!F16) l[c] = *reinterpret_cast<const BV *>(ql + ro + W * jx);
+            }
+        };
+        const BV *Ac = op_layer(zt, 0);
+        int bcur = W * jy * SP;
+        loadA(Oh[0], Ol[0], Ac, 0);
+        loadB(bh[0], bl[0], bcur, 0);
 #pragma unroll 1
         for (int zs = 0; zs < zd; zs++) {
             // products of this source layer go to fresh accumulators that are
@@ -1323,59 +1397,32 @@ __global__ __launch_bounds__(256) void p2p_16bit_kernel(const float *__restrict_
             for (int r = 0; r < RT; r++)
 #pragma unroll
                 for (int c = 0; c < NCB; c++) accz[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const int dzi = (zs > zt ? zs - zt : zt - zs) + zd - 1;  // 1/r is even in dz
-            const unsigned short *Ab = afrag + (long)dzi * 42 * 2 * 64 * 8 + lane * 8;
-            auto loadA = [&](BV &h, BV &l, int op) {
-                h = *reinterpret_cast<const BV *>(Ab + (long)(op * 2) * 64 * 8);
-                if constexpr (OP_LO) l = *reinterpret_cast<const BV *>(Ab + (long)(op * 2 + 1) * 64 * 8);
-            };
-            const int bbase = (zs * SWY + W * jy) * SP;  // row 0 of this lane's box window in layer zs
+            const int zn = zs + 1 < zd ? zs + 1 : zs;  // next source layer
+            const BV *An = op_layer(zt, zn);
+            const int bnext = (zn * SWY + W * jy) * SP;
+            // 18 k steps (ph, aa): flat window sources 96 aa + 32 ph .. + 31 of
+            // rows of 24 packed back to back.  Pair p takes operator (ph, d =
+            // 4 aa - 2 p), index 14 ph + 2 aa - p + 3: two new operators a step, four at aa = 0.
 #pragma unroll
-            for (int ph = 0; ph < 3; ph++) {
-                // k step (a, ph) = flat window sources 96 a + 32 ph .. + 31 (rows of 24 packed
-                // back to back): lane group g reads 8 sources of row 4 a + srow at column scol
-                const int fl = 32 * ph + 8 * g, srow = fl / 24, scol = fl % 24;
-                // window: A[p] = operator (ph, d = 4 a - 2 p), index 14 ph + 2 a - p + 3;
-                // An0 / An1 = pairs 0 / 1 of step a + 1
-                BV Ah[4], Al[4], An0h, An0l, An1h, An1l;
+            for (int st = 0; st < 18; st++) {
+                const int sn = (st + 1) % 18;  // the next step, of the next layer after the last
+                loadA(Oh[sn / 6], Ol[sn / 6], sn ? Ac : An, sn);
+                loadB(bh[sn & 1], bl[sn & 1], sn ? bcur : bnext, sn);
+                __builtin_amdgcn_sched_barrier(0);
+                const int ph = st / 6, aa = st % 6;
 #pragma unroll
-                for (int p = 0; p < 4; p++) loadA(Ah[p], Al[p], 14 * ph + 3 - p);
-                loadA(An0h, An0l, 14 * ph + 5);
-                loadA(An1h, An1l, 14 * ph + 4);
-#pragma unroll
-                for (int aa = 0; aa < 6; aa++) {
-                    const int ro = bbase + (4 * aa + srow) * SP + scol;
-                    BV bh[NCB], bl[NCB];
+                for (int p = 0; p < 4; p++)
 #pragma unroll
                     for (int c = 0; c < NCB; c++) {
-                        const int jx = 4 * c + (j16 & 3);
-                        bh[c] = *reinterpret_cast<const BV *>(qh + ro + W * jx);
-                        if constexpr (!F16) bl[c] = *reinterpret_cast<const BV *>(ql + ro + W * jx);
+                        const BV ah = Oh[ph][2 * aa - p + 3], al = Ol[ph][2 * aa - p + 3];
+                        accz[p][c] = mfma32(ah, bh[st & 1][c], accz[p][c]);
+                        if constexpr (!F16) accz[p][c] = mfma32(ah, bl[st & 1][c], accz[p][c]);
+                        if constexpr (OP_LO) accz[p][c] = mfma32(al, bh[st & 1][c], accz[p][c]);
                     }
-#pragma unroll
-                    for (int p = 0; p < 4; p++)
-#pragma unroll
-                        for (int c = 0; c < NCB; c++) {
-                            accz[p][c] = mfma32(Ah[p], bh[c], accz[p][c]);
-                            if constexpr (!F16) {
-                                accz[p][c] = mfma32(Ah[p], bl[c], accz[p][c]);
-                                accz[p][c] = mfma32(Al[p], bh[c], accz[p][c]);
-                            } else if constexpr (NF == 2) {
-                                accz[p][c] = mfma32(Al[p], bh[c], accz[p][c]);
-                            }
-                        }
-                    if (aa < 5) {  // slide: pairs 2, 3 of step a + 1 use pairs 0, 1 of step a
-                        Ah[3] = Ah[1]; Al[3] = Al[1];
-                        Ah[2] = Ah[0]; Al[2] = Al[0];
-                        Ah[0] = An0h; Al[0] = An0l;
-                        Ah[1] = An1h; Al[1] = An1l;
-                        if (aa < 4) {
-                            loadA(An0h, An0l, 14 * ph + 2 * aa + 7);
-                            loadA(An1h, An1l, 14 * ph + 2 * aa + 6);
-                        }
-                    }
-                }
+                __builtin_amdgcn_sched_barrier(0);
             }
+            Ac = An;
+            bcur = bnext;
 #pragma unroll
             for (int r = 0; r < RT; r++)
 #pragma unroll
