@@ -609,19 +609,29 @@ __global__ __launch_bounds__(256) void down_coarse_kernel(const float *__restric
 // target layer; wave w handles child parity (w & 1, w >> 1): an SX x 8
 // sub-lattice (SX = TX / 2) of targets in NC = SX / 2 MFMA column tiles of 16.
 // The source window holds the tile plus a 3-box halo: (TX + 6) x 22 boxes.
-// Interaction-list offsets (ox + 3) | (oy + 3) << 4 of child parity p =
-// px + 2 py: the 6 x 6 block [-2-px, 3-px] x [-2-py, 3-py] of source boxes
-// minus the 3 x 3 neighbourhood (children of the parent's neighbours minus
-// own neighbours, Box.cu:121-145).
-// The 28th entry repeats the 27th: the second offset of the last pair in the
-// 16-slot form, whose operator block is zero.
-#define MMS_M2L_OFFSETS                                                                                           \
-    {{17, 18, 19, 20, 21, 22, 33, 37, 38, 49, 53, 54, 65, 69, 70, 81, 82, 83, 84, 85, 86, 97, 98, 99, 100, 101, 102, 102}, \
-     {16, 17, 18, 19, 20, 21, 32, 33, 37, 48, 49, 53, 64, 65, 69, 80, 81, 82, 83, 84, 85, 96, 97, 98, 99, 100, 101, 101}, \
-     {1, 2, 3, 4, 5, 6, 17, 18, 19, 20, 21, 22, 33, 37, 38, 49, 53, 54, 65, 69, 70, 81, 82, 83, 84, 85, 86, 86},           \
-     {0, 1, 2, 3, 4, 5, 16, 17, 18, 19, 20, 21, 32, 33, 37, 48, 49, 53, 64, 65, 69, 80, 81, 82, 83, 84, 85, 85}}
-__constant__ int c_m2l_offs[4][28] = MMS_M2L_OFFSETS;  // 32-bit entries: wave-uniform scalar loads
-const int h_m2l_offs[4][28] = MMS_M2L_OFFSETS;          // the same table for the host's operator layout
+// Interaction list of child parity p = px + 2 py: the 6 x 6 block
+// [-2-px, 3-px] x [-2-py, 3-py] of source boxes minus the 3 x 3 neighbourhood
+// (children of the parent's neighbours minus own neighbours, Box.cu:121-145).
+// Walked from the side nearer the box, ox = sx (i - 2), oy = sy (j - 2) with sx =
+// 1 - 2 px, sy = 1 - 2 py and i, j = 0 .. 5, the neighbourhood is i, j = 1 .. 3
+// for every parity: the 27 (i, j) are constants, and a wave's LDS and
+// operator offsets two multiples of wave-uniform steps (no table load, no
+// 64-bit address products in the product loop).  Entry 27 repeats 26: the second offset of the
+// last pair in the 16-slot form, whose operator block is zero.
+struct M2LOffset { int i, j; };  // minus 2
+__host__ __device__ constexpr M2LOffset m2l_offset(int u) {
+    if (u > 26) u = 26;
+    // rows j = 0, 4, 5 hold six offsets, rows 1 .. 3 three (i = 0, 4, 5)
+    if (u < 6) return {u - 2, -2};
+    if (u < 15) return {(u - 6) % 3 == 0 ? -2 : (u - 6) % 3 + 1, (u - 6) / 3 - 1};
+    return {(u - 15) % 6 - 2, (u - 15) / 6 + 2};
+}
+// (ox + 3) | (oy + 3) << 4 for the host's operator layout
+inline int m2l_code(int parity, int u) {
+    const M2LOffset o = m2l_offset(u);
+    const int ox = (parity & 1) ? -o.i : o.i, oy = (parity & 2) ? -o.j : o.j;
+    return (ox + 3) | (oy + 3) << 4;
+}
 
 template <int KP, int MODE, int NC> struct M2LCfg {
     static constexpr int G = KP / 4;    // slots per lane group (lanes 16g..16g+15)
@@ -670,7 +680,7 @@ __global__ __launch_bounds__(256 * ZP) void m2l_mfma_kernel(const float *__restr
     const char *Tfrag = Tall + lv.toff[li];
     constexpr int G = C::G, RT = C::RT, SB = C::SB, SX = C::SX, WX = C::WX, WY = C::WY;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((threadIdx.x >> 6) & 3);
     const int px = wave & 1, py = wave >> 1;
     const int x0 = (tl % lv.ntx[li]) * C::TX, y0 = (tl / lv.ntx[li]) * 16;
     const int j16 = lane & 15, g = lane >> 4;
@@ -692,7 +702,7 @@ __global__ __launch_bounds__(256 * ZP) void m2l_mfma_kernel(const float *__restr
     // in dz: the blocks of +dz and -dz are equal, so only the dz >= 0 half is
     // read (half the operator data through L2)
     const int dzi = (ztc > zs ? ztc - zs : zs - ztc) + zd - 1;
-    const int *offs = c_m2l_offs[__builtin_amdgcn_readfirstlane(wave)];
+    const int sx = px ? -1 : 1, sy = py ? -1 : 1;
     // operator fragments of the first three offsets, in flight while the window is staged
     constexpr bool F16M = (MODE == MMS_M2L_FP16 || MODE == MMS_M2L_FP16X2);  // scaled FP16 source window
     constexpr int NP = (MODE == MMS_M2L_BF16X3 || MODE == MMS_M2L_FP16X2) ? 2 : 1;  // operator planes (hi, lo)
@@ -717,8 +727,8 @@ __global__ __launch_bounds__(256 * ZP) void m2l_mfma_kernel(const float *__restr
                                                             fb + lane * 8);
             return;
         }
-        const int code = offs[u];
-        const long fbase = ((long)dzi * 49 + (code >> 4) * 7 + (code & 15)) * RT;
+        const M2LOffset o = m2l_offset(u);
+        const long fbase = ((long)dzi * 49 + 24 + sy * 7 * o.j + sx * o.i) * RT;
 #pragma unroll
         for (int q = 0; q < NP; q++)
 #pragma unroll
@@ -859,79 +869,77 @@ __global__ __launch_bounds__(256 * ZP) void m2l_mfma_kernel(const float *__restr
     __syncthreads();
     if (zt >= zd) return;  // padding waves of the last layer group (after the only barrier)
 
-    // 27 offsets (14 offset pairs), RG operator blocks in flight (ring of registers)
-#pragma unroll 1
-    for (int ob = 0; ob < NU; ob += RG) {
+    // 27 offsets (14 offset pairs), RG operator blocks in flight (ring of registers).
+    // B operands: this lane's byte address of the target's own box in each
+    // column tile, plus a wave-uniform offset per source box.  The units are
+    // unrolled, their offsets constants: a loop that looked each up in a table
+    // waited for the table, then for the fragments, in every unit (FP32, 250 x
+    // 190 x 4, P 6: 54.4 -> 48.5 us; FP16 hi/lo, 1024 x 1024 x 4: 44.6 -> 42.4;
+    // 16-bit forms are then bound by the operators' way through the vector L1,
+    // 1 KB a fragment in 16 cycles, about as long as its four products).  B
+    // fragments one unit ahead in registers measured no better, eight column
+    // tiles a wave worse (60.9 us at 1024 x 1024 x 4).
+    constexpr int EB = MODE == MMS_M2L_FP32 ? 4 : 2;  // bytes of a window element
+    const char *bp[NC];
 #pragma unroll
-        for (int k = 0; k < RG; k++) {
-            // window offset of the source box; the pair form: lane groups 0-1
-            // read the first offset's box, 2-3 the second's, at slots 8 (g % 2)
-            int woff, slot;
-            if constexpr (PAIR) {
-                const int ca = offs[2 * (ob + k)], cb = offs[2 * (ob + k) + 1], code = (g < 2) ? ca : cb;
-                woff = ((code >> 4) - 3) * WX + ((code & 15) - 3);
-                slot = 8 * (g & 1);
-            } else {
-                const int code = offs[ob + k];
-                woff = ((code >> 4) - 3) * WX + ((code & 15) - 3);
-                slot = g * G;
-            }
-            if constexpr (MODE == MMS_M2L_FP32) {
-                const float *lds = reinterpret_cast<const float *>(smem);
+    for (int c = 0; c < NC; c++) bp[c] = smem + (tbox[c] * SB + (PAIR ? 8 * (g & 1) : g * G)) * EB;
+    const int bx1 = sx * SB * EB, by1 = sy * WX * SB * EB;  // one box in x, in y
+    auto woff = [&](int u) { const M2LOffset o = m2l_offset(u); return o.j * by1 + o.i * bx1; };
+    // the pair form: lane groups 0-1 read the first offset's box, 2-3 the second's
+    auto boff = [&](int u) {
+        if constexpr (PAIR) return g < 2 ? woff(2 * u) : woff(2 * u + 1);
+        else return woff(u);
+    };
 #pragma unroll
-                for (int u4 = 0; u4 < NK; u4++) {
-                    f32x4 b[NC];
+    for (int u = 0; u < NU; u++) {
+        AV(&a)[NP][RT][NK] = abuf[u % RG];
+        const int off = boff(u);
+        if constexpr (MODE == MMS_M2L_FP32) {
 #pragma unroll
-                    for (int c = 0; c < NC; c++)
-                        b[c] = *reinterpret_cast<const f32x4 *>(lds + (tbox[c] + woff) * SB + slot + 4 * u4);
+            for (int u4 = 0; u4 < NK; u4++) {
+                f32x4 b[NC];
 #pragma unroll
-                    for (int u = 0; u < 4; u++)
+                for (int c = 0; c < NC; c++) b[c] = *reinterpret_cast<const f32x4 *>(bp[c] + off + 16 * u4);
 #pragma unroll
-                        for (int r = 0; r < RT; r++)
-#pragma unroll
-                            for (int c = 0; c < NC; c++)
-                                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(abuf[k][0][r][u4][u], b[c][u], acc[r][c], 0, 0, 0);
-                }
-            } else {
-                const unsigned short *hi = reinterpret_cast<const unsigned short *>(smem);
-#pragma unroll
-                for (int sk = 0; sk < NK; sk++) {
-                    BV bh[NC];
-#pragma unroll
-                    for (int c = 0; c < NC; c++)
-                        bh[c] = *reinterpret_cast<const BV *>(hi + (tbox[c] + woff) * SB + slot + 8 * sk);
+                for (int q = 0; q < 4; q++)
 #pragma unroll
                     for (int r = 0; r < RT; r++)
 #pragma unroll
                         for (int c = 0; c < NC; c++)
-                            acc[r][c] = mfma32(abuf[k][0][r][sk], bh[c], acc[r][c]);
-                    if constexpr (MODE == MMS_M2L_FP16X2) {
+                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0][r][u4][q], b[c][q], acc[r][c], 0, 0, 0);
+            }
+        } else {
 #pragma unroll
-                        for (int r = 0; r < RT; r++)
+            for (int sk = 0; sk < NK; sk++) {
+                BV bh[NC], bl[NC];
 #pragma unroll
-                            for (int c = 0; c < NC; c++)
-                                acc[r][c] = mfma32(abuf[k][1][r][sk], bh[c], acc[r][c]);
-                    }
-                    if constexpr (MODE == MMS_M2L_BF16X3) {
-                        bf16x8 bl[NC];
+                for (int c = 0; c < NC; c++) {
+                    bh[c] = *reinterpret_cast<const BV *>(bp[c] + off + 16 * sk);
+                    if constexpr (MODE == MMS_M2L_BF16X3)
+                        bl[c] = *reinterpret_cast<const BV *>(bp[c] + off + 16 * sk + WX * WY * SB * EB);
+                }
 #pragma unroll
-                        for (int c = 0; c < NC; c++)
-                            bl[c] = *reinterpret_cast<const bf16x8 *>(hi + WX * WY * SB + (tbox[c] + woff) * SB + slot + 8 * sk);
+                for (int r = 0; r < RT; r++)
 #pragma unroll
-                        for (int r = 0; r < RT; r++)
+                    for (int c = 0; c < NC; c++) acc[r][c] = mfma32(a[0][r][sk], bh[c], acc[r][c]);
+                if constexpr (MODE == MMS_M2L_BF16X3) {
 #pragma unroll
-                            for (int c = 0; c < NC; c++)
-                                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(abuf[k][0][r][sk], bl[c], acc[r][c], 0, 0, 0);
+                    for (int r = 0; r < RT; r++)
 #pragma unroll
-                        for (int r = 0; r < RT; r++)
+                        for (int c = 0; c < NC; c++) acc[r][c] = mfma32(a[0][r][sk], bl[c], acc[r][c]);
+                }
+                if constexpr (NP == 2) {
 #pragma unroll
-                            for (int c = 0; c < NC; c++)
-                                acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(abuf[k][NP - 1][r][sk], bh[c], acc[r][c], 0, 0, 0);
-                    }
+                    for (int r = 0; r < RT; r++)
+#pragma unroll
+                        for (int c = 0; c < NC; c++) acc[r][c] = mfma32(a[NP - 1][r][sk], bh[c], acc[r][c]);
                 }
             }
-            if (ob + RG < NU) loadA(abuf[k], ob + RG + k);
         }
+        if (u + RG < NU) loadA(a, u + RG);
+        // keep the ring: the operators of unit u + RG are requested here, not
+        // where the compiler's scheduler would sink them, before their use
+        __builtin_amdgcn_sched_barrier(0);
     }
     // D tile row 4g + q (q = 0..3), column j16: slots 16r + 4g .. +3 of target j16
     if constexpr (F16M) {
@@ -1989,7 +1997,7 @@ int FmmPlan::init(const Grid &g, int P_, int w_, int precision_, int cols_, int 
                                 const int m = lane % 16, gg = lane / 16, kk = 8 * (gg & 1) + t, idx = 2 * u + (gg >> 1);
                                 double v = 0.0;
                                 if (idx < 27 && m < K && kk < K) {
-                                    const int code = h_m2l_offs[p][idx], oi = (code >> 4) * 7 + (code & 15);
+                                    const int code = m2l_code(p, idx), oi = (code >> 4) * 7 + (code & 15);
                                     v = T[(((size_t)dzi * 49 + oi) * K + m) * K + kk];
                                     if (f16_ops) v *= fp16_a[m] * fp16_b[kk];
                                 }
