@@ -135,6 +135,7 @@ int mms_ctx::potential(const float *rho_d, float *phi_d) {
 
 int mms_ctx::charge_potential(const float *m) {
     if (p.solver == MMS_SOLVER_DIRECT) return direct_potential_of(g, direct, m, rho, phi, stream, &prof);
+    if (p.solver == MMS_SOLVER_FMM) return fmm_potential_of(g, fmm, m, rho, phi, stream, &prof);
     return launch_div(g, m, rho, stream, &prof) || potential(rho, phi);
 }
 

@@ -131,6 +131,9 @@ __global__ __launch_bounds__(256) void m2m_mfma_kernel(const float *__restrict__
 // ------------------------------------------------ upward / downward subtrees --
 // Float offsets of every level in mult / loc / part (per film).
 struct LevelOffsets { long off[16]; };
+// Upward pass of a state: M (three planes of cells) and where its charges go;
+// m null: the charges are given.
+struct Charges { const float *m; float *rho; float dx, dy, dz; };
 
 // Upward pass of one subtree: the workgroup owns one box of level R of one
 // layer and the S x S leaves under it (S = 2^D, D = Lleaf - R <= 4).  P2M of
@@ -142,7 +145,7 @@ __global__ __launch_bounds__(256) void up_subtree_kernel(const float *__restrict
                                                          const float *__restrict__ p2mf,
                                                          const float *__restrict__ m2mfrag, LevelOffsets lo, int R,
                                                          int D, int nsx, int xd, int yd, long bufA_floats,
-                                                         FilmSet fs) {
+                                                         FilmSet fs, Charges cm) {
     constexpr int G = KP / 4, RT = KP / 16, GP = W * W / 4, SB = KP + 4;
     extern __shared__ __attribute__((aligned(16))) float lds[];
     // S, CS and sp below are powers of two: index splits are shifts and masks
@@ -160,8 +163,41 @@ __global__ __launch_bounds__(256) void up_subtree_kernel(const float *__restrict
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j16 = lane & 15, g = lane >> 4;
     const int cx0 = rbx * CS, cy0 = rby * CS;
     float *q = lds;  // CS x CS charges, later the leaf multipoles [leaf][SB]
+    if (cm.m) {
+        // charges formed here from the state (one film), by the stencil's
+        // expression, and stored for the near field
+        const float *mx = cm.m, *my = mx + plane * fs.zd, *mz = my + plane * fs.zd;
 #pragma unroll 1
-    for (int e0 = 0; e0 < CS * CS; e0 += 256 * 8) {  // 8 loads per thread in flight
+        for (int e0 = 0; e0 < CS * CS; e0 += 256 * 4) {  // 24 loads per thread in flight
+            float x2[4], x0[4], y2[4], y0[4], z2[4], z0[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int e = e0 + threadIdx.x + 256 * k;
+                const int x = cx0 + (e & (CS - 1)), y = cy0 + (e >> LCS);
+                const bool ok = e < CS * CS && x < xd && y < yd;
+                const long c = (long)z * plane + (long)y * xd + x;
+                x2[k] = ok && x != xd - 1 ? mx[c + 1] : 0.0f;
+                x0[k] = ok && x != 0 ? mx[c - 1] : 0.0f;
+                y2[k] = ok && y != yd - 1 ? my[c + xd] : 0.0f;
+                y0[k] = ok && y != 0 ? my[c - xd] : 0.0f;
+                z2[k] = ok && z != fs.zd - 1 ? mz[c + plane] : 0.0f;
+                z0[k] = ok && z != 0 ? mz[c - plane] : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int e = e0 + threadIdx.x + 256 * k;
+                const int x = cx0 + (e & (CS - 1)), y = cy0 + (e >> LCS);
+                const float v = ((x2[k] - x0[k]) / cm.dx + (y2[k] - y0[k]) / cm.dy + (z2[k] - z0[k]) / cm.dz) * 0.5f;
+                if (e < CS * CS) {
+                    const bool ok = x < xd && y < yd;
+                    if (ok) cm.rho[(long)z * plane + (long)y * xd + x] = v;
+                    q[e] = ok ? v : 0.0f;
+                }
+            }
+        }
+    }
+#pragma unroll 1
+    for (int e0 = cm.m ? CS * CS : 0; e0 < CS * CS; e0 += 256 * 8) {  // 8 loads per thread in flight
         float vb[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -1627,8 +1663,27 @@ int launch_near(const Grid &g, const FmmPlan &pl, const float *rho, float *phi, 
     return 0;
 }
 
+// Small films at leaf width 4 stay on one stream: their near field is over in
+// 5 to 7 us, which a second queue costs them (two events and a wait a solve,
+// a branch in a captured graph), and their upward pass forms the charges
+// itself (a launch less; the near field then follows it).  A step, two queues
+// and a charge launch / one queue, us: captured 32 x 32 x 3 123 / 106, 64 x 64
+// x 3 138 / 118, 128 x 128 x 4 (P 6) 195 / 193.5, 256 x 256 x 3 181.6 / 180.9,
+// 400 x 200 x 3 238 / 241; issued eagerly 162 / 120 at 64 x 64 x 3, 218 / 178 at 256 x
+// 256 x 3, 352 / 336 at 250 x 190 x 4 (P 6), 271 / 246 at 512 x 256 x 3.
+constexpr long kOneQueueCapture = 1L << 17, kOneQueueEager = 1L << 19;  // cells
+int one_queue(const Grid &g, const FmmPlan &pl, hipStream_t s, bool *yes) {
+    *yes = false;
+    if (pl.w != 4 || pl.d_films || g.n() > kOneQueueEager) return 0;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    MMS_HIP(hipStreamIsCapturing(s, &cs));
+    *yes = g.n() <= (cs == hipStreamCaptureStatusNone ? kOneQueueEager : kOneQueueCapture);
+    return 0;
+}
+
 template <int K, int W>
-int run_fmm(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_t s, Profiler *prof) {
+int run_fmm(const Grid &g, FmmPlan &pl, const Charges &cm, const float *rho, float *phi, hipStream_t s,
+            Profiler *prof) {
     constexpr int KP = KPad<K>::KP, SB = KP + 4;
     const int zd = g.zd;
     LevelOffsets lo{};
@@ -1650,9 +1705,12 @@ int run_fmm(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_
     // profiling window wants one kernel at a time; L2P adds the far field
     // after the join.  Leaf width 2 keeps the fused near field + L2P at the end.
     constexpr bool split = (W == 4 || W == 8);
-    const bool conc = split && pl.s_near && !(prof && prof->on);
+    bool serial = false;
+    if (one_queue(g, pl, s, &serial)) return 1;
+    const bool conc = split && pl.s_near && !(prof && prof->on) && !serial;
     if constexpr (split) {
-        if (conc) {
+        if (cm.m) {  // the upward pass forms the charges: after it
+        } else if (conc) {
             MMS_HIP(hipEventRecord(pl.ev_fork, s));
         } else {
             KTimer kt(prof, K_P2P_L2P);
@@ -1673,7 +1731,7 @@ int run_fmm(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_
             attr = 1;
         }
         hipLaunchKernelGGL((up_subtree_kernel<K, KP, W>), dim3(nsub, zd * pl.nfilm), dim3(256), lds, s, rho,
-                           pl.mult, pl.d_p2mf, pl.d_m2m, lo, R, D, nsx, g.xd, g.yd, bufA, pl.films());
+                           pl.mult, pl.d_p2mf, pl.d_m2m, lo, R, D, nsx, g.xd, g.yd, bufA, pl.films(), cm);
         MMS_HIP(hipGetLastError());
     }
     if constexpr (split) {
@@ -1681,7 +1739,10 @@ int run_fmm(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_
         // upward pass); it is issued after the upward pass so that a captured
         // step graph keeps the multipole chain, the critical path, on the
         // caller's queue and puts the near field on the second one
-        if (conc) {
+        if (cm.m) {
+            KTimer kt(prof, K_P2P_L2P);
+            if (launch_near<K, KP, W>(g, pl, rho, phi, scale, false, s)) return 1;
+        } else if (conc) {
             MMS_HIP(hipStreamWaitEvent(pl.s_near, pl.ev_fork, 0));
             if (launch_near<K, KP, W>(g, pl, rho, phi, scale, true, pl.s_near)) return 1;
             MMS_HIP(hipEventRecord(pl.ev_join, pl.s_near));
@@ -1763,17 +1824,18 @@ int run_fmm(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_
 }
 
 template <int W>
-int run_fmm_w(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_t s, Profiler *prof) {
+int run_fmm_w(const Grid &g, FmmPlan &pl, const Charges &cm, const float *rho, float *phi, hipStream_t s,
+              Profiler *prof) {
     switch (pl.P) {
-    case 1: return run_fmm<NC<1>::K, W>(g, pl, rho, phi, s, prof);
-    case 2: return run_fmm<NC<2>::K, W>(g, pl, rho, phi, s, prof);
-    case 3: return run_fmm<NC<3>::K, W>(g, pl, rho, phi, s, prof);
-    case 4: return run_fmm<NC<4>::K, W>(g, pl, rho, phi, s, prof);
-    case 5: return run_fmm<NC<5>::K, W>(g, pl, rho, phi, s, prof);
-    case 6: return run_fmm<NC<6>::K, W>(g, pl, rho, phi, s, prof);
-    case 7: return run_fmm<NC<7>::K, W>(g, pl, rho, phi, s, prof);
-    case 8: return run_fmm<NC<8>::K, W>(g, pl, rho, phi, s, prof);
-    case 9: return run_fmm<NC<9>::K, W>(g, pl, rho, phi, s, prof);
+    case 1: return run_fmm<NC<1>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 2: return run_fmm<NC<2>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 3: return run_fmm<NC<3>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 4: return run_fmm<NC<4>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 5: return run_fmm<NC<5>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 6: return run_fmm<NC<6>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 7: return run_fmm<NC<7>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 8: return run_fmm<NC<8>::K, W>(g, pl, cm, rho, phi, s, prof);
+    case 9: return run_fmm<NC<9>::K, W>(g, pl, cm, rho, phi, s, prof);
     default: set_error("FMM expansion order must be 1..9"); return 1;
     }
 }
@@ -1793,14 +1855,27 @@ float host_bf2f(unsigned short h) {
 
 }  // namespace
 
-int fmm_potential(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_t s, Profiler *prof) {
+static int fmm_run(const Grid &g, FmmPlan &pl, const Charges &cm, const float *rho, float *phi, hipStream_t s,
+                   Profiler *prof) {
     MMS_CHECK(pl.mult != nullptr, "FMM plan not initialised");
     switch (pl.w) {
-    case 2: return run_fmm_w<2>(g, pl, rho, phi, s, prof);
-    case 4: return run_fmm_w<4>(g, pl, rho, phi, s, prof);
-    case 8: return run_fmm_w<8>(g, pl, rho, phi, s, prof);
+    case 2: return run_fmm_w<2>(g, pl, cm, rho, phi, s, prof);
+    case 4: return run_fmm_w<4>(g, pl, cm, rho, phi, s, prof);
+    case 8: return run_fmm_w<8>(g, pl, cm, rho, phi, s, prof);
     default: set_error("FMM leaf width must be 2, 4 or 8"); return 1;
     }
+}
+
+int fmm_potential(const Grid &g, FmmPlan &pl, const float *rho, float *phi, hipStream_t s, Profiler *prof) {
+    return fmm_run(g, pl, Charges{}, rho, phi, s, prof);
+}
+
+int fmm_potential_of(const Grid &g, FmmPlan &pl, const float *m, float *rho, float *phi, hipStream_t s, Profiler *prof) {
+    bool fused = false;
+    // a profiling window times the charges by themselves
+    if (!(prof && prof->on) && one_queue(g, pl, s, &fused)) return 1;
+    if (!fused) return launch_div(g, m, rho, s, prof) || fmm_potential(g, pl, rho, phi, s, prof);
+    return fmm_run(g, pl, Charges{m, rho, g.dx, g.dy, g.dz}, rho, phi, s, prof);
 }
 
 int FmmPlan::init_batch(const Grid &g, int P_, int w_, int precision_, int cols_, const std::vector<FilmDesc> &fl) {

@@ -162,6 +162,9 @@ struct FmmPlan {
 };
 int fmm_potential(const Grid &g, FmmPlan &plan, const float *rho, float *phi,
                   hipStream_t s, Profiler *prof);
+// charges of the state m (3 planes of n cells) into rho and their potential
+int fmm_potential_of(const Grid &g, FmmPlan &plan, const float *m, float *rho, float *phi, hipStream_t s,
+                     Profiler *prof);
 
 // Host-side operator construction (FP64), real bases as described above.
 struct FmmHostOps {
