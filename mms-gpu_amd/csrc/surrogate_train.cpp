@@ -110,7 +110,6 @@ struct mms_sur_trainer {
     std::vector<float> inv_norm;
     // batch
     float *d_brho = nullptr, *d_bphi = nullptr, *d_bphs = nullptr, *d_binv = nullptr;
-    std::vector<float> h_binv;
     mms_ctx *solver = nullptr;
     int solver_P = -1;
     ~mms_sur_trainer() {
@@ -156,16 +155,11 @@ int append_norm(mms_sur_trainer *t, long i) {
 // gather the batch idx[0..batch) and run the forward pass
 int forward_batch(mms_sur_trainer *t, const long *idx) {
     MMS_CHECK(idx, "null batch index");
-    const long n = t->npf;
-    for (int b = 0; b < t->batch; b++) {
+    for (int b = 0; b < t->batch; b++)
         MMS_CHECK(idx[b] >= 0 && idx[b] < t->npairs, "batch index outside the training set");
-        MMS_HIP(hipMemcpyAsync(t->d_brho + b * n, t->d_rho + idx[b] * n, sizeof(float) * n, hipMemcpyDeviceToDevice,
-                               t->stream));
-        MMS_HIP(hipMemcpyAsync(t->d_bphi + b * n, t->d_phi + idx[b] * n, sizeof(float) * n, hipMemcpyDeviceToDevice,
-                               t->stream));
-        t->h_binv[b] = t->inv_norm[idx[b]];
-    }
-    MMS_HIP(hipMemcpyAsync(t->d_binv, t->h_binv.data(), sizeof(float) * t->batch, hipMemcpyHostToDevice, t->stream));
+    if (surrogate_gather(t->d_rho, t->d_phi, t->npf, idx, t->inv_norm.data(), t->batch, t->d_brho, t->d_bphi, t->d_binv,
+                         t->stream))
+        return 1;
     return surrogate_potential(t->sp, t->d_brho, t->d_bphs, t->rscale, t->oscale, t->stream, nullptr);
 }
 
@@ -219,7 +213,6 @@ extern "C" int mms_surrogate_trainer_create(mms_sur_trainer **out, int xdim, int
     MMS_HIP(hipMalloc(&t->d_bphi, sizeof(float) * nb));
     MMS_HIP(hipMalloc(&t->d_bphs, sizeof(float) * nb));
     MMS_HIP(hipMalloc(&t->d_binv, sizeof(float) * batch));
-    t->h_binv.assign(batch, 0.0f);
     MMS_HIP(hipStreamSynchronize(t->stream));
     *out = t.release();
     return 0;
