@@ -497,7 +497,18 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
 // The gradient tile dz (16 x 16 pixels x 64 channels, NHWC) transposed into
 // LDS as dzT[co][pixel] (row stride DZS): thread (row, half, channel block)
 // loads 8 pixels x 8 channels and stores 8 channel rows of 8 pixels.
-constexpr int DZS = 256 + 8;
+constexpr int DZS = 256 + 48;
+// Where the 16-byte unit u of channel c's row lies in its row (304 elements:
+// 38 units).  Eight lanes store one unit of eight channel rows (8 cb + k, cb
+// = 0 .. 7) in one LDS cycle, sixteen read one of rows j and j' (lane
+// groups g, g + 1) in one: with units in order the rows' starts fall on two
+// bank groups and a store takes 64 cycles instead of 8 (a third of the kernels'
+// time was such conflicts).  Unit bits 0 .. 2 exchanged by channel bits 5, 2 ^ 3 and 4
+// free both of conflicts.
+__device__ __forceinline__ int row_unit(int c, int u) {
+    const int x = ((c >> 5) & 1) | ((((c >> 2) ^ (c >> 3)) & 1) << 1) | (((c >> 4) & 1) << 2);
+    return 8 * (u < 32 ? u ^ x : u);
+}
 // element k of 8 packed BF16 values
 __device__ __forceinline__ unsigned bf_elem(const uint4 &v, int k) {
     const unsigned w = (k >> 1) == 0 ? v.x : (k >> 1) == 1 ? v.y : (k >> 1) == 2 ? v.z : v.w;
@@ -512,18 +523,24 @@ __device__ __forceinline__ uint4 column8(const uint4 (&v)[8], int k) {
     o.w = bf_elem(v[6], k) | bf_elem(v[7], k) << 16;
     return o;
 }
-__device__ __forceinline__ void stage_dzT(const unsigned short *__restrict__ dz, unsigned short *dzT, int z, int x0,
-                                          int y0, int xd, int yd) {
+// buffer resource over an activation tensor: loads past its end return zeros
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t act_rsrc(const unsigned short *p, int nbytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short *>(p), (short)0, nbytes, 0x00020000);
+}
+__device__ __forceinline__ uint4 act_load(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+}
+__device__ __forceinline__ void load_dzT(__amdgpu_buffer_rsrc_t r, int nbytes, uint4 (&v)[8], int z, int x0, int y0,
+                                         int xd, int yd) {
+    const int py = threadIdx.x >> 4, q = (threadIdx.x >> 3) & 1, cb = threadIdx.x & 7, gy = y0 + py;
+    const int row = ((z * yd + gy) * xd + x0 + 8 * q) * C * 2 + 16 * cb;
+#pragma unroll
+    for (int i = 0; i < 8; i++) v[i] = act_load(r, x0 + 8 * q + i < xd && gy < yd ? row + i * C * 2 : nbytes);
+}
+__device__ __forceinline__ void store_dzT(const uint4 (&v)[8], unsigned short *dzT) {
     const int py = threadIdx.x >> 4, q = (threadIdx.x >> 3) & 1, cb = threadIdx.x & 7;
-    uint4 v[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int gx = x0 + 8 * q + i, gy = y0 + py;
-        v[i] = make_uint4(0u, 0u, 0u, 0u);
-        if (gx < xd && gy < yd) v[i] = *reinterpret_cast<const uint4 *>(dz + (((long)z * yd + gy) * xd + gx) * C + 8 * cb);
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) *reinterpret_cast<uint4 *>(dzT + (8 * cb + k) * DZS + py * 16 + 8 * q) = column8(v, k);
+    for (int k = 0; k < 8; k++) *reinterpret_cast<uint4 *>(dzT + (8 * cb + k) * DZS + row_unit(8 * cb + k, 2 * py + q)) = column8(v, k);
 }
 
 // bias gradient partial of thread t: channel t / 4, pixels 64 (t % 4) .. + 63 of dzT
@@ -532,7 +549,7 @@ __device__ __forceinline__ float dzT_rowsum(const unsigned short *dzT) {
     float s = 0.0f;
 #pragma unroll
     for (int u = 0; u < 8; u++) {
-        const uint4 v = *reinterpret_cast<const uint4 *>(dzT + co * DZS + 64 * qq + 8 * u);
+        const uint4 v = *reinterpret_cast<const uint4 *>(dzT + co * DZS + row_unit(co, 8 * qq + u));
         const unsigned w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
         for (int i = 0; i < 4; i++) s += bf2f((unsigned short)(w[i] & 0xFFFF)) + bf2f((unsigned short)(w[i] >> 16));
@@ -550,7 +567,13 @@ __device__ __forceinline__ float dzT_rowsum(const unsigned short *dzT) {
 // channels (36 accumulator tiles).  Persistent: the workgroup walks tiles
 // blockIdx.x, + gridDim.x, ... over all layers and writes its partial sums
 // to part[blockIdx.x][9 * 64 * 64 + 64].
-constexpr int XS = HS * 16 + 8;   // xc row stride per channel (296)
+// With one workgroup a CU (156 KB of LDS) nothing else covers its waits: the
+// next tile is loaded during the products (by buffer loads, whose zeros
+// outside the film need no select that would wait for them), each k step's
+// fragments during those of the step before, and the stores are free of bank
+// conflicts.  24 layers of 128 x 128: 69.5 -> 62.4 us without conflicts and
+// with the fragments ahead, 49.3 with the tile ahead (products alone 12 us).
+constexpr int XS = DZS;   // xc row stride per channel (36 units used)
 constexpr size_t WGRAD_LDS = sizeof(unsigned short) * ((size_t)C * DZS + 3 * C * XS);
 constexpr long WGRAD_PART = CONVN + C;
 
@@ -568,41 +591,75 @@ __global__ __launch_bounds__(256) void sur_wgrad_kernel(const unsigned short *__
 #pragma unroll
         for (int ct = 0; ct < 4; ct++) acc[tap][ct] = f32x4{0.f, 0.f, 0.f, 0.f};
     float dbs = 0.0f;
-    for (int t = blockIdx.x; t < ntile; t += gridDim.x) {
+    // The next tile's cells, loaded during this one's products: of dz 8 pixels x 8
+    // channels a thread, of the window ten pixels (the three shifts of 8) x 8
+    // channels of row item / 16, half (item / 8) % 2, channel block item % 8,
+    // items threadIdx.x and threadIdx.x + 256.
+    constexpr int WP = (HS * 16 + 255) / 256;
+    uint4 dv[8], wv[WP][10];
+    const int nbytes = nz * yd * xd * C * 2;
+    const __amdgpu_buffer_rsrc_t rz = act_rsrc(dz, nbytes), ra = act_rsrc(a, nbytes);
+    auto load = [&](int t) {
         const int z = t / npl, tl = t % npl, x0 = (tl % ntx) * TS, y0 = (tl / ntx) * TS;
-        __syncthreads();  // the previous tile's products are done with the LDS
-        stage_dzT(dz, dzT, z, x0, y0, xd, yd);
-        for (int item = threadIdx.x; item < 3 * HS * 16; item += 256) {
-            const int cb = item & 7, q = (item >> 3) & 1, wy = (item >> 4) % HS, dx = (item >> 4) / HS;
-            const int gy = y0 - 1 + wy;
-            uint4 v[8];
+        load_dzT(rz, nbytes, dv, z, x0, y0, xd, yd);
 #pragma unroll
-            for (int i = 0; i < 8; i++) {
-                const int gx = x0 - 1 + 8 * q + i + dx;
-                v[i] = make_uint4(0u, 0u, 0u, 0u);
-                if (gx >= 0 && gx < xd && gy >= 0 && gy < yd)
-                    v[i] = *reinterpret_cast<const uint4 *>(a + (((long)z * yd + gy) * xd + gx) * C + 8 * cb);
+        for (int p = 0; p < WP; p++) {
+            const int item = threadIdx.x + 256 * p, cb = item & 7, q = (item >> 3) & 1, wy = item >> 4, gy = y0 - 1 + wy;
+            if (item >= HS * 16) continue;
+            const int row = ((z * yd + gy) * xd + x0 - 1 + 8 * q) * C * 2 + 16 * cb;
+#pragma unroll
+            for (int i = 0; i < 10; i++) {
+                const int gx = x0 - 1 + 8 * q + i;
+                wv[p][i] = act_load(ra, gx >= 0 && gx < xd && gy >= 0 && gy < yd ? row + i * C * 2 : nbytes);
             }
+        }
+    };
+    if ((int)blockIdx.x < ntile) load(blockIdx.x);
+    for (int t = blockIdx.x; t < ntile; t += gridDim.x) {
+        __syncthreads();  // the previous tile's products are done with the LDS
+        store_dzT(dv, dzT);
 #pragma unroll
-            for (int k = 0; k < 8; k++)
-                *reinterpret_cast<uint4 *>(xc + (dx * C + 8 * cb + k) * XS + wy * 16 + 8 * q) = column8(v, k);
+        for (int p = 0; p < WP; p++) {
+            const int item = threadIdx.x + 256 * p, cb = item & 7, q = (item >> 3) & 1, wy = item >> 4;
+            if (item < HS * 16) {
+#pragma unroll
+                for (int dx = 0; dx < 3; dx++) {
+                    uint4 v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; i++) v[i] = wv[p][i + dx];
+#pragma unroll
+                    for (int k = 0; k < 8; k++)
+                        *reinterpret_cast<uint4 *>(xc + (dx * C + 8 * cb + k) * XS + row_unit(8 * cb + k, 2 * wy + q)) =
+                    column8(v, k);
+                }
+            }
         }
         __syncthreads();
+        if (t + (int)gridDim.x < ntile) load(t + gridDim.x);
         dbs += dzT_rowsum(dzT);
-#pragma unroll 1
-        for (int kk = 0; kk < 8; kk++) {
-            const int row = 2 * kk + (g >> 1), px0 = 8 * (g & 1);
-            bf16x8 A[4];
+        // the fragments of k step kk + 1 are read before the products of kk
+        const int px0 = 8 * (g & 1);
+        bf16x8 A[2][4], B[2][9];
+        auto frags = [&](int kk) {
+            const int row = 2 * kk + (g >> 1);
 #pragma unroll
             for (int ct = 0; ct < 4; ct++)
-                A[ct] = *reinterpret_cast<const bf16x8 *>(dzT + (16 * ct + j) * DZS + row * 16 + px0);
+                A[kk & 1][ct] = *reinterpret_cast<const bf16x8 *>(dzT + (16 * ct + j) * DZS + row_unit(16 * ct + j, 2 * row + (g & 1)));
 #pragma unroll
-            for (int tap = 0; tap < 9; tap++) {
-                const int dy = tap / 3, dx = tap % 3;
-                const bf16x8 B = *reinterpret_cast<const bf16x8 *>(xc + (dx * C + 16 * wave + j) * XS + (row + dy) * 16 + px0);
+            for (int tap = 0; tap < 9; tap++)
+                B[kk & 1][tap] = *reinterpret_cast<const bf16x8 *>(xc + ((tap % 3) * C + 16 * wave + j) * XS +
+                                                                    row_unit(16 * wave + j, 2 * (row + tap / 3) + (g & 1)));
+        };
+        frags(0);
 #pragma unroll
-                for (int ct = 0; ct < 4; ct++) acc[tap][ct] = mfma_bf16(A[ct], B, acc[tap][ct]);
-            }
+        for (int kk = 0; kk < 8; kk++) {
+            if (kk + 1 < 8) frags(kk + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int tap = 0; tap < 9; tap++)
+#pragma unroll
+                for (int ct = 0; ct < 4; ct++) acc[tap][ct] = mfma_bf16(A[kk & 1][ct], B[kk & 1][tap], acc[tap][ct]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     // D row 4 g + i of tile (tap, ct) = co 16 ct + 4 g + i; column j = ci 16 wave + j
@@ -631,19 +688,23 @@ __global__ __launch_bounds__(256) void sur_lift_wgrad_kernel(const float *__rest
     __shared__ float in[3][HS][HS];
     const int ntx = (xd + TS - 1) / TS, nty = (yd + TS - 1) / TS, npl = ntx * nty, ntile = npl * nz;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+    const int nbytes = nz * yd * xd * C * 2;
+    const __amdgpu_buffer_rsrc_t rz = act_rsrc(dz, nbytes);
     f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
     float dbs = 0.0f;
     for (int t = blockIdx.x; t < ntile; t += gridDim.x) {
         const int z = t / npl, tl = t % npl, x0 = (tl % ntx) * TS, y0 = (tl / ntx) * TS;
         __syncthreads();
-        stage_dzT(dz, dzT, z, x0, y0, xd, yd);
+        uint4 dv[8];
+        load_dzT(rz, nbytes, dv, z, x0, y0, xd, yd);
+        store_dzT(dv, dzT);
         stage_planes(rho, in, z, zf, x0, y0, xd, yd, rscale);
         __syncthreads();
         dbs += dzT_rowsum(dzT);
 #pragma unroll 1
         for (int kk = 0; kk < 8; kk++) {
             const int row = 2 * kk + (g >> 1), px0 = 8 * (g & 1);
-            const bf16x8 A = *reinterpret_cast<const bf16x8 *>(dzT + (16 * wave + j) * DZS + row * 16 + px0);
+            const bf16x8 A = *reinterpret_cast<const bf16x8 *>(dzT + (16 * wave + j) * DZS + row_unit(16 * wave + j, 2 * row + (g & 1)));
 #pragma unroll
             for (int nt = 0; nt < 2; nt++) {
                 const int k = 16 * nt + j, kc = k < 27 ? k : 0, tap = kc / 3, pl = kc % 3, dy = tap / 3, dx = tap % 3;
@@ -1457,7 +1518,11 @@ int surrogate_backward(SurrogatePlan &sp, const float *rho, const float *phi_s, 
     if (launch_conv(2, sp, a, s)) return 1;
     // lift
     const int ntile = ((g.xd + TS - 1) / TS) * ((g.yd + TS - 1) / TS) * g.zd;
-    const int nb = ntile < SurrogatePlan::kPartBlocks ? ntile : SurrogatePlan::kPartBlocks;
+    // three workgroups a CU fit (38 KB of LDS): 40.1 -> 22.2 us with 768 in
+    // place of 256 on 24 layers of 128 x 128, the sum of the partials 7.4 -> 10
+    constexpr int kLiftBlocks = 768;
+    static_assert(kLiftBlocks * LGRAD_PART <= SurrogatePlan::kPartBlocks * WGRAD_PART, "lift partials fit the buffer");
+    const int nb = ntile < kLiftBlocks ? ntile : kLiftBlocks;
     hipLaunchKernelGGL(sur_lift_wgrad_kernel, dim3(nb), dim3(256), 0, s, rho, sp.d_dzb, sp.d_wpart, g.xd, g.yd, g.zd,
                        sp.zf, rscale);
     MMS_HIP(hipGetLastError());
