@@ -23,6 +23,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "div_by.hpp"
 #include "mms_internal.hpp"
 
 namespace mms {
@@ -102,14 +103,17 @@ __global__ __launch_bounds__(256) void direct_reduce_kernel(const double *__rest
 // along the row, so four LDS words and one 16-byte charge read serve 16
 // products (the batch's table kernel reads a word per product).  A workgroup
 // takes kSmallGroups such groups and splits the source rows (in pieces of
-// kSmallRun) over 32 slices, so that a 32 x 32 x 3 film has 48 workgroups of
+// kSmallRun) over 64 slices, so that a 32 x 32 x 3 film has 96 workgroups of
 // eight waves; FP32 over a piece, FP64 across pieces and slices.  With FROM_M
 // every workgroup forms all charges itself (div M, vector_functions.cpp:8-28)
-// and a separate charge launch falls away; what bounds the kernel is the
-// latency of those loads, so a thread has kSmallBatch cells' loads in flight.
-// A step of the 32 x 32 x 3 film: 128 us with charge, pair loop and reduction
-// as three launches an evaluation, 93 us so; error against 64 bits 6e-7 -> 2.8e-7.
-constexpr int kSmallGroups = 16, kSmallSlices = 32, kSmallRun = 128, kSmallBatch = 8;
+// and a separate charge launch falls away.  A third of the kernel's 10 us is a
+// launch and its first loads, the rest instructions: buffer loads whose range
+// check stands for the stencil's edge branches and divisions by known
+// divisors took 6 of 58.5 us off a step of the 32 x 32 x 3 film, half the groups a workgroup 4
+// (40 x 36 x 4: 84 -> 72 -> 62 us; 4 groups a workgroup 76, 4-cell batches
+// against 8 62 against 64).  Charge, pair loop and reduction as three launches
+// an evaluation took 128 us; error against 64 bits 6e-7 -> 2.8e-7.
+constexpr int kSmallGroups = 8, kSmallSlices = 64, kSmallRun = 128, kSmallBatch = 4;
 constexpr int kSmallThreads = kSmallGroups * kSmallSlices;
 // e / d for 0 <= e < 2^21 with inv = 1 / d: (e + 1/2) / d is at least 1 / 2d
 // away from an integer, the rounding at most e 2^-22 / d
@@ -157,6 +161,9 @@ __global__ __launch_bounds__(kSmallThreads) void direct_small_kernel(const float
     const int tf = small_table_floats(h), n = xd * h.rows, nq = h.rows * h.xq, plane = xd * yd;
     float *tab = slds, *q = slds + tf;
     const float ixq = 1.0f / (float)h.xq, iyd = 1.0f / (float)yd;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(src), (short)0, (FROM_M ? 12 : 4) * n, 0x00020000);
+    const float rdx = 1.0f / dx, rdy = 1.0f / dy, rdz = 1.0f / dz;
+    auto ld = [&](int off) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, off, 0, 0)); };
     for (int e0 = threadIdx.x, k0 = 0; e0 < nq; e0 += kSmallThreads * kSmallBatch, k0 += kSmallBatch) {
         constexpr int NV = FROM_M ? 6 : 1;
         float v[kSmallBatch][NV];
@@ -166,15 +173,15 @@ __global__ __launch_bounds__(kSmallThreads) void direct_small_kernel(const float
             const bool ok = e < nq && x < xd;
             if constexpr (FROM_M) {
                 const int z = small_div(r, iyd), y = r - z * yd;
-                const float *mx = src, *my = src + n, *mz = src + 2 * n;
-                v[k][0] = (ok && x != xd - 1) ? mx[c + 1] : 0.0f;
-                v[k][1] = (ok && x != 0) ? mx[c - 1] : 0.0f;
-                v[k][2] = (ok && y != yd - 1) ? my[c + xd] : 0.0f;
-                v[k][3] = (ok && y != 0) ? my[c - xd] : 0.0f;
-                v[k][4] = (ok && z != zd - 1) ? mz[c + plane] : 0.0f;
-                v[k][5] = (ok && z != 0) ? mz[c - plane] : 0.0f;
+                // buffer loads: zeros past the planes' end, no branches
+                v[k][0] = ld(ok && x != xd - 1 ? 4 * (c + 1) : 12 * n);
+                v[k][1] = ld(ok && x != 0 ? 4 * (c - 1) : 12 * n);
+                v[k][2] = ld(ok && y != yd - 1 ? 4 * (n + c + xd) : 12 * n);
+                v[k][3] = ld(ok && y != 0 ? 4 * (n + c - xd) : 12 * n);
+                v[k][4] = ld(ok && z != zd - 1 ? 4 * (2 * n + c + plane) : 12 * n);
+                v[k][5] = ld(ok && z != 0 ? 4 * (2 * n + c - plane) : 12 * n);
             } else {
-                v[k][0] = ok ? src[c] : 0.0f;
+                v[k][0] = ld(ok ? 4 * c : 4 * n);
             }
         }
         if (k0 == 0)  // the table, while the first charges' loads are in flight
@@ -184,7 +191,7 @@ __global__ __launch_bounds__(kSmallThreads) void direct_small_kernel(const float
         for (int k = 0; k < kSmallBatch; k++) {
             const int e = e0 + k * kSmallThreads;
             float c = v[k][0];
-            if constexpr (FROM_M) c = ((v[k][0] - v[k][1]) / dx + (v[k][2] - v[k][3]) / dy + (v[k][4] - v[k][5]) / dz) * 0.5f;
+            if constexpr (FROM_M) c = (div_by(v[k][0] - v[k][1], dx, rdx) + div_by(v[k][2] - v[k][3], dy, rdy) + div_by(v[k][4] - v[k][5], dz, rdz)) * 0.5f;
             if (e < nq) {
                 q[e] = c;
                 if constexpr (FROM_M) {  // one workgroup writes each charge
@@ -229,13 +236,15 @@ __global__ __launch_bounds__(kSmallThreads) void direct_small_kernel(const float
 #pragma unroll
     for (int i = 0; i < 4; i++) red[sl * 4 * kSmallGroups + 4 * gi + i] = acc[i];
     __syncthreads();
-    // 8 threads per target, four slices each
-    const int o = threadIdx.x >> 3, p = threadIdx.x & 7;
+    // four slices a thread, kRed threads a target
+    constexpr int kRed = kSmallSlices / 4;
+    static_assert(kRed * 4 * kSmallGroups == kSmallThreads, "one thread per four slices of a target");
+    const int o = threadIdx.x / kRed, p = threadIdx.x % kRed;
     double v = 0.0;
 #pragma unroll
     for (int k = 0; k < 4; k++) v += red[(4 * p + k) * 4 * kSmallGroups + o];
 #pragma unroll
-    for (int m = 1; m < 8; m <<= 1) v += __shfl_xor(v, m);
+    for (int m = 1; m < kRed; m <<= 1) v += __shfl_xor(v, m);
     const int go = blockIdx.x * kSmallGroups + (o >> 2);
     if (p == 0 && go < ngroup) {
         const int r = small_div(go, ingx), x = 4 * (go - r * ngx) + (o & 3);
@@ -732,16 +741,19 @@ static void direct_chunks(long n, int split, long *chunk, int *nchunk) {
 }
 
 // Which form serves a grid.  One RK4 step of a film (four evaluations and
-// stage kernels, step graph), table / transforms: 32x32x3 93 / 115 us, 40x40x3
-// 103 / 110, 48x48x3 114 / 111, 55x55x3 126 / 105, 100x30x3 138 / 117 us, so the
-// line lies at 6,000 cells.  The pair loop (37 ms a step on 161x117x3, where
-// the transforms take 1.3) keeps the grids that fit neither.
+// stage kernels, step graph), table / transforms: 50x40x3 64 / 89 us, 48x48x3
+// 67 / 87, 64x64x2 72 / 88, 55x50x3 100 / 93, 64x64x3 157 / 86.  The table is
+// the faster one while its workgroups fit the chip at once (256 of 8 groups);
+// above 6,000 cells the transforms' FP64 sums are kept.  Narrow films fill
+// their groups of four poorly: 5x1100x1 157 / 106.  The pair loop (37 ms a step
+// on 161x117x3, where the transforms take 1.3) keeps the grids that fit neither.
 constexpr long kTableCells = 6000;
 constexpr size_t kSmallLds = 80 * 1024;
 DirectForm direct_form(const Grid &g) {
     const long n = g.n();
     const bool table = n <= 16384 && small_lds(g) <= kSmallLds, fft = direct_fft_fits(g);
-    if (table && (n <= kTableCells || !fft)) return kDirectTable;
+    const long groups = (long)((g.xd + 3) / 4) * g.yd * g.zd;
+    if (table && ((n <= kTableCells && groups <= 256 * kSmallGroups) || !fft)) return kDirectTable;
     return fft ? kDirectFft : kDirectChunks;
 }
 
@@ -839,9 +851,11 @@ int direct_potential(const Grid &g, DirectPlan &plan, const float *rho, float *p
 int direct_potential_of(const Grid &g, DirectPlan &plan, const float *m, float *rho, float *phi, hipStream_t s,
                         Profiler *prof) {
     MMS_CHECK(plan.table != nullptr || plan.work != nullptr, "direct solver plan not initialised");
-    if (plan.form == kDirectChunks) {
+    // the table kernel's charges divide by div_by
+    const bool apart = plan.form == kDirectTable && !(div_by_ok(g.dx) && div_by_ok(g.dy) && div_by_ok(g.dz));
+    if (plan.form == kDirectChunks || apart) {
         if (launch_div(g, m, rho, s, prof)) return 1;
-        return direct_launch(g, plan.chunk, plan.nchunk, static_cast<double *>(plan.work), rho, phi, s, prof);
+        return direct_potential(g, plan, rho, phi, s, prof);
     }
     KTimer kt(prof, K_DIRECT);
     if (plan.form == kDirectTable)
