@@ -19,11 +19,15 @@
 //   fft_back     inverse x transforms, two real rows each, FP32 potential.
 // Measured against the pair loop (FP32 rsqrt pairs, 3.8e12 a second): the
 // 256 x 256 x 3 potential on host arrays 9.46 -> 0.11 ms, an RK4 step of a
-// 161 x 117 x 3 film 3.67 -> 0.13 ms (fft_rows 9.2 us with div M, fft_columns
-// 7.4 us, fft_back 5.8 us an evaluation: launch and load latency at this size);
+// 161 x 117 x 3 film 3.67 -> 0.086 ms (fft_rows 6.8 us with div M, fft_columns
+// 6.4 us, fft_back 4.6 us an evaluation: launch and load latency at this
+// size, so all that a thread loads, twiddles and kernel spectrum too, is
+// requested before the first barrier and none behind a branch; one after the
+// other where needed they took 8.9, 7.0 and 5.4 us, a step 106);
 // relative error against 64 bits 5.8e-7 -> 2.5e-8.
 // A charge that is not finite would spread through the transforms; fft_rows
 // notes it and fft_back then sums that call pair by pair.
+#include "div_by.hpp"
 #include "mms_internal.hpp"
 
 namespace mms {
@@ -72,9 +76,10 @@ __device__ __forceinline__ void dft(cd (&v)[R]) {
 }
 
 // One Stockham pass of radix R after sub-transforms of length NS; thread t of
-// the transform's N / 8.
+// the transform's N / 8, w its twiddle (radix 8; the passes before have none).
 template <int N, int R, int NS>
-__device__ __forceinline__ void fft_pass(cd *buf, int t, const cd *__restrict__ tw) {
+__device__ __forceinline__ void fft_pass(cd *buf, int t, cd w) {
+    static_assert(NS == 1 || R == 8, "one twiddle a thread");
     constexpr int Q = 8 / R;
     cd v[Q][R];
 #pragma unroll
@@ -82,7 +87,7 @@ __device__ __forceinline__ void fft_pass(cd *buf, int t, const cd *__restrict__ 
 #pragma unroll
         for (int k = 0; k < R; k++) v[b][k] = buf[slot(t + b * (N / 8) + k * (N / R))];
         if constexpr (NS > 1) {
-            const cd w1 = tw[((t + b * (N / 8)) & (NS - 1)) * (kTw / (NS * R))];
+            const cd w1 = w;
             v[b][1] = cmul(v[b][1], w1);
             if constexpr (R > 2) {
                 const cd w2 = cmul(w1, w1), w3 = cmul(w2, w1);
@@ -109,11 +114,25 @@ __device__ __forceinline__ void fft_pass(cd *buf, int t, const cd *__restrict__ 
     __syncthreads();
 }
 
-template <int N, int NS>
-__device__ __forceinline__ void fft_rest(cd *buf, int t, const cd *__restrict__ tw) {
+// First radix of a transform (its other passes are radix 8) and its twiddles, loaded
+// with the kernels' other first loads: in the passes each would be waited
+// for between two barriers.
+template <int N>
+constexpr int first_radix() { return __builtin_ctz(N) % 3 == 1 ? 2 : (__builtin_ctz(N) % 3 == 2 ? 4 : 8); }
+struct Twiddles { cd w[4]; };
+template <int N>
+__device__ __forceinline__ Twiddles fft_twiddles(int t, const cd *__restrict__ tw) {
+    Twiddles r;
+#pragma unroll
+    for (int p = 0, ns = first_radix<N>(); p < 4; p++, ns *= 8)
+        r.w[p] = ns < N ? tw[(t & (ns - 1)) * (kTw / (ns * 8))] : make_double2(0.0, 0.0);
+    return r;
+}
+template <int N, int NS, int P>
+__device__ __forceinline__ void fft_rest(cd *buf, int t, const Twiddles &tw) {
     if constexpr (NS < N) {
-        fft_pass<N, 8, NS>(buf, t, tw);
-        fft_rest<N, NS * 8>(buf, t, tw);
+        fft_pass<N, 8, NS>(buf, t, tw.w[P]);
+        fft_rest<N, NS * 8, P + 1>(buf, t, tw);
     }
 }
 
@@ -121,17 +140,10 @@ __device__ __forceinline__ void fft_rest(cd *buf, int t, const cd *__restrict__ 
 // by every thread of the workgroup (the inverse: re and im swapped before
 // and after).
 template <int N>
-__device__ __forceinline__ void fft(cd *buf, int t, const cd *__restrict__ tw) {
-    constexpr int L = __builtin_ctz(N);
-    if constexpr (L % 3 == 1) {
-        fft_pass<N, 2, 1>(buf, t, tw);
-        fft_rest<N, 2>(buf, t, tw);
-    } else if constexpr (L % 3 == 2) {
-        fft_pass<N, 4, 1>(buf, t, tw);
-        fft_rest<N, 4>(buf, t, tw);
-    } else {
-        fft_rest<N, 1>(buf, t, tw);
-    }
+__device__ __forceinline__ void fft(cd *buf, int t, const Twiddles &tw) {
+    constexpr int R = first_radix<N>();
+    fft_pass<N, R, 1>(buf, t, make_double2(1.0, 0.0));
+    fft_rest<N, R, 0>(buf, t, tw);
 }
 
 // transforms per workgroup of the row kernels: at least a wave of threads
@@ -162,31 +174,55 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
     const int z = blockIdx.y, y0 = blockIdx.x * 2 * B, ya = y0 + 2 * f;
     const long plane = (long)A.xd * A.yd, n = plane * A.zd;
     const long row = (long)z * plane + (long)ya * A.xd;
+    const Twiddles tw = fft_twiddles<N>(t, A.tw);
     bool bad = false;
+    // the rows' upper half is padding (xd <= N / 2).  Every load of a thread is
+    // issued before one is used: none sits behind a branch
     float q[8][2];
+    if constexpr (FROM_M) {
+        // div M by the charge kernel's expression (vector_functions.cpp:8-28);
+        // buffer loads return 0 past the three planes
+        const int end = 12 * (int)n;
+        const __amdgpu_buffer_rsrc_t rm = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(A.m), (short)0, end, 0x00020000);
+        auto ld = [&](bool ok, int i) { return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rm, ok ? 4 * i : end, 0, 0)); };
+        const float rdx = 1.0f / A.dx, rdy = 1.0f / A.dy, rdz = 1.0f / A.dz;
+        float v[4][2][6];
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const int x = t + k * T;
+        for (int k = 0; k < 4; k++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            float v = 0.0f;
-            const int y = ya + h;
-            if (x < A.xd && y < A.yd) {
-                const long c = row + (long)h * A.xd + x;
-                if constexpr (FROM_M) {
-                    // div M by the charge kernel's expression (vector_functions.cpp:8-28)
-                    const float *mx = A.m, *my = A.m + n, *mz = A.m + 2 * n;
-                    const float x2 = (x != A.xd - 1) ? mx[c + 1] : 0.0f, x0 = (x != 0) ? mx[c - 1] : 0.0f;
-                    const float y2 = (y != A.yd - 1) ? my[c + A.xd] : 0.0f, yb = (y != 0) ? my[c - A.xd] : 0.0f;
-                    const float z2 = (z != A.zd - 1) ? mz[c + plane] : 0.0f, z0 = (z != 0) ? mz[c - plane] : 0.0f;
-                    v = ((x2 - x0) / A.dx + (y2 - yb) / A.dy + (z2 - z0) / A.dz) * 0.5f;
-                } else {
-                    v = A.rho[c];
-                }
+            for (int h = 0; h < 2; h++) {
+                const int x = t + k * T, y = ya + h, c = (int)row + h * A.xd + x;
+                const bool ok = x < A.xd && y < A.yd;
+                v[k][h][0] = ld(ok && x != A.xd - 1, c + 1);
+                v[k][h][1] = ld(ok && x != 0, c - 1);
+                v[k][h][2] = ld(ok && y != A.yd - 1, (int)n + c + A.xd);
+                v[k][h][3] = ld(ok && y != 0, (int)n + c - A.xd);
+                v[k][h][4] = ld(ok && z != A.zd - 1, 2 * (int)n + c + (int)plane);
+                v[k][h][5] = ld(ok && z != 0, 2 * (int)n + c - (int)plane);
             }
-            q[k][h] = v;
-        }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const float(&u)[6] = v[k][h];
+                q[k][h] = (div_by(u[0] - u[1], A.dx, rdx) + div_by(u[2] - u[3], A.dy, rdy) + div_by(u[4] - u[5], A.dz, rdz)) * 0.5f;
+            }
+    } else {
+        float v[4][2];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {  // past the film: its last cell, then 0
+                const long c = row + (long)h * A.xd + t + k * T;
+                v[k][h] = A.rho[c < n ? c : n - 1];
+            }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int h = 0; h < 2; h++) q[k][h] = (t + k * T < A.xd && ya + h < A.yd) ? v[k][h] : 0.0f;
     }
+#pragma unroll
+    for (int k = 4; k < 8; k++) q[k][0] = q[k][1] = 0.0f;
     cd *buf = lds + f * slots(N);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
@@ -200,7 +236,7 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
     }
     const int any = __syncthreads_or(bad ? 1 : 0);
     if (threadIdx.x == 0) A.flags[blockIdx.y * gridDim.x + blockIdx.x] = any;
-    fft<N>(buf, t, A.tw);
+    fft<N>(buf, t, tw);
     // spectra of the two real rows of each transform: with Z = FFT(a + i b),
     // A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = (Z[k] - conj Z[N-k]) / 2i
     for (int i = threadIdx.x; i < 2 * B * (N / 2 + 1); i += B * T) {
@@ -217,39 +253,39 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
 // the layers' product at one (kx, ky): out[z] = sum_z' ghat[|z - z'|] in[z'];
 // re and im are stored swapped (the inverse transform follows)
 template <int ZD, int N>
-__device__ __forceinline__ void layer_product(cd *lds, const double *__restrict__ gh, long gstride, int zd_rt) {
-    constexpr int ZM = ZD ? ZD : 16;
-    const int zd = ZD ? ZD : zd_rt;
+__device__ __forceinline__ void layer_product(cd *lds, const double (&g)[ZD]) {
+    cd in[ZD];
+#pragma unroll
+    for (int z = 0; z < ZD; z++) in[z] = lds[z * slots(N)];
+#pragma unroll
+    for (int z = 0; z < ZD; z++) {
+        double re = 0.0, im = 0.0;
+#pragma unroll
+        for (int s = 0; s < ZD; s++) {
+            re = fma(g[z > s ? z - s : s - z], in[s].x, re);
+            im = fma(g[z > s ? z - s : s - z], in[s].y, im);
+        }
+        lds[z * slots(N)] = make_double2(im, re);
+    }
+}
+// ... of any number of layers up to 16, its spectrum read from memory
+template <int N>
+__device__ __forceinline__ void layers_product(cd *lds, const double *__restrict__ gh, long gstride, int zd) {
+    constexpr int ZM = 16;
     cd in[ZM];
 #pragma unroll
     for (int z = 0; z < ZM; z++)
         if (z < zd) in[z] = lds[z * slots(N)];
-    if constexpr (ZD != 0) {
-        double g[ZM];
+    for (int z = 0; z < zd; z++) {
+        double re = 0.0, im = 0.0;
 #pragma unroll
-        for (int z = 0; z < ZM; z++) g[z] = gh[z * gstride];
-#pragma unroll
-        for (int z = 0; z < ZM; z++) {
-            double re = 0.0, im = 0.0;
-#pragma unroll
-            for (int s = 0; s < ZM; s++) {
-                re = fma(g[z > s ? z - s : s - z], in[s].x, re);
-                im = fma(g[z > s ? z - s : s - z], in[s].y, im);
+        for (int s = 0; s < ZM; s++)
+            if (s < zd) {
+                const double gv = gh[(z > s ? z - s : s - z) * gstride];
+                re = fma(gv, in[s].x, re);
+                im = fma(gv, in[s].y, im);
             }
-            lds[z * slots(N)] = make_double2(im, re);
-        }
-    } else {
-        for (int z = 0; z < zd; z++) {
-            double re = 0.0, im = 0.0;
-#pragma unroll
-            for (int s = 0; s < ZM; s++)
-                if (s < zd) {
-                    const double gv = gh[(z > s ? z - s : s - z) * gstride];
-                    re = fma(gv, in[s].x, re);
-                    im = fma(gv, in[s].y, im);
-                }
-            lds[z * slots(N)] = make_double2(im, re);
-        }
+        lds[z * slots(N)] = make_double2(im, re);
     }
 }
 
@@ -261,10 +297,28 @@ __global__ __launch_bounds__(ZD ? ZD * N / 8 : 1024) void fft_columns(FftArgs A)
     const int z = threadIdx.x / T, t = threadIdx.x % T, kx = blockIdx.x;
     cd *col = A.w + ((long)z * A.nxh + kx) * A.yd;
     cd *buf = lds + z * slots(N);
+    const Twiddles tw = fft_twiddles<N>(t, A.tw);
+    // the column's upper half is padding (yd <= N / 2); past yd its last entry, then 0
+    cd v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) v[k] = col[min(t + k * T, A.yd - 1)];
+    const long gs = (long)A.nxh * (N / 2 + 1);
+    // this thread's kernel spectrum, in flight during the first transform
+    constexpr int NI = ZD ? (8 + ZD - 1) / ZD : 1;
+    double g[NI][ZD ? ZD : 1];
+    auto spectrum = [&](int ky) { return A.ghat + (long)kx * (N / 2 + 1) + (ky <= N / 2 ? ky : N - ky); };
+    if constexpr (ZD != 0) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const double *gh = spectrum(min((int)threadIdx.x + i * ZD * T, N - 1));
+#pragma unroll
+            for (int s = 0; s < ZD; s++) g[i][s] = gh[s * gs];
+        }
+    }
 #pragma unroll
     for (int k = 0; k < 8; k++) {
         const int y = t + k * T;
-        buf[slot(y)] = y < A.yd ? col[y] : make_double2(0.0, 0.0);
+        buf[slot(y)] = k < 4 && y < A.yd ? v[k & 3] : make_double2(0.0, 0.0);
     }
     if (kx == 0) {  // one flag for fft_back
         int any = 0;
@@ -273,16 +327,20 @@ __global__ __launch_bounds__(ZD ? ZD * N / 8 : 1024) void fft_columns(FftArgs A)
         if (threadIdx.x == 0) A.flags[A.nflags] = any;
     }
     __syncthreads();
-    fft<N>(buf, t, A.tw);
-    const long gs = (long)A.nxh * (N / 2 + 1);
-    for (int ky = threadIdx.x; ky < N; ky += blockDim.x) {
-        const double *gh = A.ghat + (long)kx * (N / 2 + 1) + (ky <= N / 2 ? ky : N - ky);
-        layer_product<ZD, N>(lds + slot(ky), gh, gs, A.zd);
+    fft<N>(buf, t, tw);
+    if constexpr (ZD != 0) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            const int ky = threadIdx.x + i * ZD * T;
+            if (ky < N) layer_product<ZD, N>(lds + slot(ky), g[i]);
+        }
+    } else {
+        for (int ky = threadIdx.x; ky < N; ky += blockDim.x) layers_product<N>(lds + slot(ky), spectrum(ky), gs, A.zd);
     }
     __syncthreads();
-    fft<N>(buf, t, A.tw);
+    fft<N>(buf, t, tw);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < 4; k++) {
         const int y = t + k * T;
         if (y < A.yd) {
             const cd v = buf[slot(y)];
@@ -318,26 +376,44 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_back(FftArgs A) {
     const int f = threadIdx.x / T, t = threadIdx.x % T;
     const int z = blockIdx.y, y0 = blockIdx.x * 2 * B, ya = y0 + 2 * f;
     const long row = ((long)z * A.yd + ya) * A.xd;
+    const Twiddles tw = fft_twiddles<N>(t, A.tw);
+    // the rows' spectra, four k a thread and k = N / 2 by the first ones; past yd the last row's, then 0
+    auto load = [&](int i, cd &u, cd &v) {
+        const int y = y0 + 2 * (i % B);
+        const cd *p = A.w + ((long)z * A.nxh + i / B) * A.yd;
+        u = p[min(y, A.yd - 1)];
+        v = p[min(y + 1, A.yd - 1)];
+    };
+    cd u[4], v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) load(threadIdx.x + q * B * T, u[q], v[q]);
     if (A.flags[A.nflags]) {
         for (int h = 0; h < 2; h++)
             for (int x = t; x < A.xd; x += T)
                 if (ya + h < A.yd) A.phi[row + (long)h * A.xd + x] = (float)pair_sum(A, x, ya + h, z);
         return;
     }
-    for (int i = threadIdx.x; i < B * (N / 2 + 1); i += B * T) {
+    auto put = [&](int i, cd u, cd v) {
         const int r = i % B, k = i / B, y = y0 + 2 * r;
-        const cd *p = A.w + ((long)z * A.nxh + k) * A.yd + y;
-        const cd u = y < A.yd ? p[0] : make_double2(0.0, 0.0), v = y + 1 < A.yd ? p[1] : make_double2(0.0, 0.0);
+        if (y >= A.yd) u = make_double2(0.0, 0.0);
+        if (y + 1 >= A.yd) v = make_double2(0.0, 0.0);
         cd *zb = lds + r * slots(N);
         // Z[k] = U + i V, Z[N-k] = conj(U) + i conj(V), re and im swapped
         zb[slot(k)] = make_double2(u.y + v.x, u.x - v.y);
         if (k > 0 && k < N / 2) zb[slot(N - k)] = make_double2(v.x - u.y, u.x + v.y);
+    };
+#pragma unroll
+    for (int q = 0; q < 4; q++) put(threadIdx.x + q * B * T, u[q], v[q]);
+    if (threadIdx.x < B) {
+        cd ul, vl;
+        load(threadIdx.x + 4 * B * T, ul, vl);
+        put(threadIdx.x + 4 * B * T, ul, vl);
     }
     __syncthreads();
     cd *buf = lds + f * slots(N);
-    fft<N>(buf, t, A.tw);
+    fft<N>(buf, t, tw);
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
+    for (int k = 0; k < 4; k++) {
         const int x = t + k * T;
         if (x < A.xd) {
             const cd v = buf[slot(x)];
@@ -370,7 +446,7 @@ __global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_rows(doubl
         buf[slot(x)] = make_double2(r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0, 0.0);
     }
     __syncthreads();
-    fft<N>(buf, t, tw);
+    fft<N>(buf, t, fft_twiddles<N>(t, tw));
     for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) a[((long)z * (N / 2 + 1) + k) * nyh + y] = buf[slot(k)].x;
 }
 
@@ -383,7 +459,7 @@ __global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_columns(co
     const long o = ((long)blockIdx.y * nxh + blockIdx.x) * (N / 2 + 1);
     for (int y = threadIdx.x; y < N; y += blockDim.x) buf[slot(y)] = make_double2(a[o + (y <= N / 2 ? y : N - y)], 0.0);
     __syncthreads();
-    fft<N>(buf, t, tw);
+    fft<N>(buf, t, fft_twiddles<N>(t, tw));
     for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) ghat[o + k] = buf[slot(k)].x * scale;
 }
 

@@ -741,12 +741,12 @@ static void direct_chunks(long n, int split, long *chunk, int *nchunk) {
 }
 
 // Which form serves a grid.  One RK4 step of a film (four evaluations and
-// stage kernels, step graph), table / transforms: 50x40x3 64 / 89 us, 48x48x3
-// 67 / 87, 64x64x2 72 / 88, 55x50x3 100 / 93, 64x64x3 157 / 86.  The table is
-// the faster one while its workgroups fit the chip at once (256 of 8 groups);
-// above 6,000 cells the transforms' FP64 sums are kept.  Narrow films fill
-// their groups of four poorly: 5x1100x1 157 / 106.  The pair loop (37 ms a step
-// on 161x117x3, where the transforms take 1.3) keeps the grids that fit neither.
+// stage kernels, step graph), table / transforms: 48x48x3 67 / 69 us, 55x55x2
+// 68 / 74, 64x64x2 72 / 72, 55x50x3 100 / 73, 64x64x3 157 / 71; 40x36x4 takes the
+// table 62.  Up to 6,000 cells the table, and only while its workgroups fit the
+// chip at once (256 of 8 groups): narrow films fill their groups of four
+// poorly (5x1100x1 157 / 106).  The pair loop (37 ms a step on 161x117x3, where
+// the transforms take 0.09) keeps the grids that fit neither.
 constexpr long kTableCells = 6000;
 constexpr size_t kSmallLds = 80 * 1024;
 DirectForm direct_form(const Grid &g) {
@@ -851,9 +851,9 @@ int direct_potential(const Grid &g, DirectPlan &plan, const float *rho, float *p
 int direct_potential_of(const Grid &g, DirectPlan &plan, const float *m, float *rho, float *phi, hipStream_t s,
                         Profiler *prof) {
     MMS_CHECK(plan.table != nullptr || plan.work != nullptr, "direct solver plan not initialised");
-    // the table kernel's charges divide by div_by
-    const bool apart = plan.form == kDirectTable && !(div_by_ok(g.dx) && div_by_ok(g.dy) && div_by_ok(g.dz));
-    if (plan.form == kDirectChunks || apart) {
+    // the other forms' charges are read with 32-bit byte offsets and divide by div_by
+    const bool own = 12 * g.n() < (1L << 31) && div_by_ok(g.dx) && div_by_ok(g.dy) && div_by_ok(g.dz);
+    if (plan.form == kDirectChunks || !own) {
         if (launch_div(g, m, rho, s, prof)) return 1;
         return direct_potential(g, plan, rho, phi, s, prof);
     }
