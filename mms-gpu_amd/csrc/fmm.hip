@@ -1550,17 +1550,23 @@ long m2l_groups(const FmmPlan &pl, int ZP) {
 
 // Shape of the M2L workgroups.  A workgroup's products last as long however
 // few of them there are (FP32: 11 us for 16-slot, 46 us for 32-slot blocks with
-// two layers and four column tiles, two waves on a SIMD), so launches that
-// leave CUs idle take half the columns (NC = 2), and FP32, whose products take
-// all of its time, one target layer (ZP = 1) as well.  RK4 steps in us with
-// four columns and two layers / this rule: FP32 leaf 4, 64x64x3 P 3 173 / 142,
-// 256x256x3 P 4 213 / 187, 200x200x2 P 6 390 / 231, 250x190x4 P 6 412 / 363,
-// 400x300x3 P 6 558 / 446; BF16 split leaf 8, 700x700x2 372 / 301, 512x512x2
-// 267 / 247.  kM2lFill = 600 workgroups of the narrow shape: with more, four columns are
-// as good or better (FP32 1024x1024x4 leaf 8 1856 against 1917, BF16 split
-// 1024x1024x2 441 against 472).  The scaled FP16 forms gain nothing from
+// two layers and four column tiles, two waves on a SIMD).  FP32, whose
+// products take all of its time, works on one target layer (ZP = 1) with as
+// many column tiles (NC) as cost least: a CU's share of the workgroups times
+// NC and half a tile for the window.  Four need more than one such round (with one
+// the window's latency shows).  Beside the FP32 near field of leaf width 8,
+// one tile.  RK4 steps in us with 1 / 2 / 4 tiles: leaf 4, 64x64x3 P 3 109 / 119 /
+// 139, 128x128x4 P 6 203 / 195 / 247, 256x256x3 P 4 181 / 182 / 193, 300x280x3
+// P 6 378 / 374 / 417, 400x300x3 P 5 452 / 439 / 430, 512x512x3 P 4 369 / 362
+// / 365; leaf 8, 300x300x2 P 5 261 / 284 / 335, 1000x600x3 P 6 913 / 912 / 933,
+// 1024x1024x4 P 6 1748 / 1881 / 1843.
+// The BF16 split takes two column tiles in place of four while these are no
+// more than kM2lFill workgroups: leaf 8, 700x700x2 372 -> 301, 512x512x2 267 ->
+// 247, but 1024x1024x2 441 -> 472.  The scaled FP16 forms gain nothing from
 // narrower windows beyond 128 x 128 cells and keep the wide shape.
 constexpr long kM2lFill = 600;
+template <int NC>
+long m2l_rounds(const FmmPlan &pl) { return (m2l_groups<NC>(pl, 1) + 255) / 256; }
 
 template <int KP, int MODE>
 int launch_m2l_nc(const FmmPlan &pl, hipStream_t s) {
@@ -1573,7 +1579,9 @@ int launch_m2l_nc(const FmmPlan &pl, hipStream_t s) {
     }
     static_assert(M2LCfg<KP, MODE, 4>::lds_bytes <= 160 * 1024, "M2L source window exceeds LDS");
     if constexpr (KP <= 32 && MODE == MMS_M2L_FP32) {
-        if (m2l_groups<2>(pl, 1) <= kM2lFill) return launch_m2l<KP, MODE, 2, 1>(pl, s);
+        const long r4 = m2l_rounds<4>(pl), c1 = 3 * m2l_rounds<1>(pl), c2 = 5 * m2l_rounds<2>(pl), c4 = 9 * r4;
+        if (pl.w == 8 || (c1 < c2 && (c1 < c4 || r4 == 1))) return launch_m2l<KP, MODE, 1, 1>(pl, s);
+        if (c2 < c4 || r4 == 1) return launch_m2l<KP, MODE, 2, 1>(pl, s);
         return launch_m2l<KP, MODE, 4, 1>(pl, s);
     }
     if constexpr (KP <= 32 && MODE == MMS_M2L_BF16X3) {
