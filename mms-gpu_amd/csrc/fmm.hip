@@ -1560,10 +1560,14 @@ long m2l_groups(const FmmPlan &pl, int ZP) {
 // P 6 378 / 374 / 417, 400x300x3 P 5 452 / 439 / 430, 512x512x3 P 4 369 / 362
 // / 365; leaf 8, 300x300x2 P 5 261 / 284 / 335, 1000x600x3 P 6 913 / 912 / 933,
 // 1024x1024x4 P 6 1748 / 1881 / 1843.
-// The BF16 split takes two column tiles in place of four while these are no
-// more than kM2lFill workgroups: leaf 8, 700x700x2 372 -> 301, 512x512x2 267 ->
-// 247, but 1024x1024x2 441 -> 472.  The scaled FP16 forms gain nothing from
-// narrower windows beyond 128 x 128 cells and keep the wide shape.
+// The 16-bit forms take one tile and one layer while that is one round (64 x
+// 64 x 3, P 6: BF16 split 142 -> 127, FP16 hi/lo 154 -> 132; leaf 8, 200 x 200
+// x 3 212 -> 196), the scaled FP16 and plain BF16 forms then two tiles and two
+// layers while that is one (128 x 128 x 4 184 -> 167, leaf 8, 400 x 300 x 3
+// 254 -> 243; above, 250 x 190 x 4 227 against 240).  The BF16 split takes two
+// tiles, at leaf width 4 up to two rounds of one layer (128 x 128 x 4 165 -> 157, 256 x
+// 256 x 3 162 -> 157) and up to kM2lFill workgroups of two (leaf 8, 700x700x2 372
+// -> 301, 512x512x2 267 -> 247, but 1024x1024x2 441 -> 472).
 constexpr long kM2lFill = 600;
 template <int NC>
 long m2l_rounds(const FmmPlan &pl) { return (m2l_groups<NC>(pl, 1) + 255) / 256; }
@@ -1584,7 +1588,14 @@ int launch_m2l_nc(const FmmPlan &pl, hipStream_t s) {
         if (c2 < c4 || r4 == 1) return launch_m2l<KP, MODE, 2, 1>(pl, s);
         return launch_m2l<KP, MODE, 4, 1>(pl, s);
     }
+    if constexpr (KP <= 32 && MODE != MMS_M2L_FP32) {
+        if (m2l_rounds<1>(pl) == 1) return launch_m2l<KP, MODE, 1, 1>(pl, s);
+        if constexpr (MODE != MMS_M2L_BF16X3) {
+            if (m2l_groups<2>(pl, 2) <= 256) return launch_m2l<KP, MODE, 2, 2>(pl, s);
+        }
+    }
     if constexpr (KP <= 32 && MODE == MMS_M2L_BF16X3) {
+        if (pl.w == 4 && m2l_rounds<2>(pl) <= 2) return launch_m2l<KP, MODE, 2, 1>(pl, s);
         if (m2l_groups<2>(pl, 1) <= kM2lFill) return launch_m2l<KP, MODE, 2, 2>(pl, s);
     }
     return launch_m2l<KP, MODE, 4, ZP>(pl, s);
