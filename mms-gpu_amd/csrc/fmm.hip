@@ -1582,11 +1582,15 @@ int launch_m2l_nc(const FmmPlan &pl, hipStream_t s) {
         if (pl.m2l_cols == 8) return launch_m2l<KP, MODE, 8, ZP>(pl, s);
     }
     static_assert(M2LCfg<KP, MODE, 4>::lds_bytes <= 160 * 1024, "M2L source window exceeds LDS");
+    // one target layer a workgroup while films x layers^2 fit the grid's z
+    const bool fits = (long)pl.nfilm * pl.zd * pl.zd <= 65535;
     if constexpr (KP <= 32 && MODE == MMS_M2L_FP32) {
         const long r4 = m2l_rounds<4>(pl), c1 = 3 * m2l_rounds<1>(pl), c2 = 5 * m2l_rounds<2>(pl), c4 = 9 * r4;
-        if (pl.w == 8 || (c1 < c2 && (c1 < c4 || r4 == 1))) return launch_m2l<KP, MODE, 1, 1>(pl, s);
-        if (c2 < c4 || r4 == 1) return launch_m2l<KP, MODE, 2, 1>(pl, s);
-        return launch_m2l<KP, MODE, 4, 1>(pl, s);
+        if (fits) {
+            if (pl.w == 8 || (c1 < c2 && (c1 < c4 || r4 == 1))) return launch_m2l<KP, MODE, 1, 1>(pl, s);
+            if (c2 < c4 || r4 == 1) return launch_m2l<KP, MODE, 2, 1>(pl, s);
+            return launch_m2l<KP, MODE, 4, 1>(pl, s);
+        }
     }
     if constexpr (KP <= 32 && MODE != MMS_M2L_FP32) {
         if (m2l_rounds<1>(pl) == 1) return launch_m2l<KP, MODE, 1, 1>(pl, s);

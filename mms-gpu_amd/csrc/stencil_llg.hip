@@ -793,7 +793,7 @@ unsigned xcd_grid(const Grid &g) {
 // 62.9 / 46.9, 705x498x4 (1.4 M cells) 92.9 / 92.3; above, the walk's fewer
 // loads count.
 constexpr long kSplitCells = 1L << 20;
-bool split_layers(const Grid &g) { return g.n() < kSplitCells; }
+bool split_layers(const Grid &g) { return g.n() < kSplitCells && g.zd <= 65535; }  // layers in the grid's y
 
 }  // namespace
 
