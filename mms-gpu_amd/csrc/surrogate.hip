@@ -129,42 +129,45 @@ __device__ __forceinline__ void input_planes(const float *__restrict__ rho, int 
 }
 
 // the 18 x 18 window of the three input planes around the tile (x0, y0) of
-// layer z; films of up to 8 layers issue every charge load of a thread's
+// layer z, rounded to BF16 (once here, not in the 27 products that read each);
+// films of up to ZM layers issue every charge load of a thread's
 // pixels before combining them (the same sums in the same order)
-__device__ __forceinline__ void stage_planes(const float *__restrict__ rho, float (*in)[HS][HS], int z, int zf,
-                                             int x0, int y0, int xd, int yd, float rscale) {
+template <int ZM>
+__device__ __forceinline__ void stage_planes_of(const float *__restrict__ rho, unsigned short (*in)[HS][HS], int z,
+                                                int zf, int x0, int y0, int xd, int yd, float rscale) {
     const long plane = (long)xd * yd;
-    constexpr int ZM = 8, NP = (HS * HS + 255) / 256;
-    if (zf <= ZM) {
-        const int f0 = (z / zf) * zf, zl = z - f0;
-        float r[NP][ZM];
+    constexpr int NP = (HS * HS + 255) / 256;
+    const int f0 = (z / zf) * zf, zl = z - f0;
+    float r[NP][ZM];
 #pragma unroll
-        for (int q = 0; q < NP; q++) {
-            const int e = threadIdx.x + 256 * q, sy = e / HS, sx = e % HS, gx = x0 - 1 + sx, gy = y0 - 1 + sy;
-            const bool ok = e < HS * HS && gx >= 0 && gx < xd && gy >= 0 && gy < yd;
-            const long c2 = (long)gy * xd + gx;
+    for (int q = 0; q < NP; q++) {
+        const int e = threadIdx.x + 256 * q, sy = e / HS, sx = e % HS, gx = x0 - 1 + sx, gy = y0 - 1 + sy;
+        const bool ok = e < HS * HS && gx >= 0 && gx < xd && gy >= 0 && gy < yd;
+        const long c2 = (long)gy * xd + gx;
 #pragma unroll
-            for (int k = 0; k < ZM; k++) r[q][k] = (ok && k < zf) ? rho[(long)(f0 + k) * plane + c2] : 0.0f;
-        }
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            const int e = threadIdx.x + 256 * q;
-            if (e >= HS * HS) break;
-            float v[3];
-            combine_planes<ZM>(r[q], zl, zf, rscale, v);
-            in[0][e / HS][e % HS] = v[0];
-            in[1][e / HS][e % HS] = v[1];
-            in[2][e / HS][e % HS] = v[2];
-        }
-        return;
+        for (int k = 0; k < ZM; k++) r[q][k] = (ok && k < zf) ? rho[(long)(f0 + k) * plane + c2] : 0.0f;
     }
+#pragma unroll
+    for (int q = 0; q < NP; q++) {
+        const int e = threadIdx.x + 256 * q;
+        if (e >= HS * HS) break;
+        float v[3];
+        combine_planes<ZM>(r[q], zl, zf, rscale, v);
+#pragma unroll
+        for (int k = 0; k < 3; k++) in[k][e / HS][e % HS] = f2bf(v[k]);
+    }
+}
+__device__ __forceinline__ void stage_planes(const float *__restrict__ rho, unsigned short (*in)[HS][HS], int z, int zf,
+                                             int x0, int y0, int xd, int yd, float rscale) {
+    if (zf <= 4) return stage_planes_of<4>(rho, in, z, zf, x0, y0, xd, yd, rscale);
+    if (zf <= 8) return stage_planes_of<8>(rho, in, z, zf, x0, y0, xd, yd, rscale);
+    const long plane = (long)xd * yd;
     for (int e = threadIdx.x; e < HS * HS; e += 256) {
         const int sy = e / HS, sx = e % HS, gx = x0 - 1 + sx, gy = y0 - 1 + sy;
         float v[3] = {0.0f, 0.0f, 0.0f};
         if (gx >= 0 && gx < xd && gy >= 0 && gy < yd) input_planes(rho, z, zf, plane, (long)gy * xd + gx, rscale, v);
-        in[0][sy][sx] = v[0];
-        in[1][sy][sx] = v[1];
-        in[2][sy][sx] = v[2];
+#pragma unroll
+        for (int k = 0; k < 3; k++) in[k][sy][sx] = f2bf(v[k]);
     }
 }
 
@@ -178,14 +181,18 @@ __global__ __launch_bounds__(256) void sur_lift_kernel(const float *__restrict__
                                                        const float *__restrict__ bias, unsigned short *__restrict__ out,
                                                        unsigned short *__restrict__ zsave, int xd, int yd, int zf,
                                                        float rscale) {
-    __shared__ float in[3][HS][HS];
+    __shared__ unsigned short in[3][HS][HS];
     const int z = blockIdx.z, x0 = blockIdx.x * TS, y0 = blockIdx.y * TS;
     stage_planes(rho, in, z, zf, x0, y0, xd, yd, rscale);
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
+    // output channel of row 4 gq + i of row tile r: a lane's rows of two tiles
+    // are eight consecutive channels and its 16-byte stores make 64-byte runs
+    // (8-byte stores in 32-byte runs: 187 us on 1024 x 1024 x 4, so 160)
+    auto channel = [](int r, int gq, int i) { return 32 * (r >> 1) + 8 * gq + 4 * (r & 1) + i; };
     bf16x8 a[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) a[r] = *reinterpret_cast<const bf16x8 *>(wl + (16 * r + j) * 32 + 8 * g);
+    for (int r = 0; r < 4; r++) a[r] = *reinterpret_cast<const bf16x8 *>(wl + channel(r, j >> 2, j & 3) * 32 + 8 * g);
 #pragma unroll
     for (int ct = 0; ct < 4; ct++) {
         const int py = 4 * wave + ct, px = j;  // pixel of this lane's column
@@ -193,25 +200,32 @@ __global__ __launch_bounds__(256) void sur_lift_kernel(const float *__restrict__
 #pragma unroll
         for (int t = 0; t < 8; t++) {
             const int k = 8 * g + t, kc = k < 27 ? k : 0, tap = kc / 3, pl = kc % 3;  // kc: reads stay in the window
-            bv[t] = (k < 27) ? f2bf(in[pl][py + tap / 3][px + tap % 3]) : (unsigned short)0;
+            bv[t] = (k < 27) ? in[pl][py + tap / 3][px + tap % 3] : (unsigned short)0;
         }
         const bf16x8 b = __builtin_bit_cast(bf16x8, bv);
         const int gx = x0 + px, gy = y0 + py;
         const bool ok = gx < xd && gy < yd;
         const long o = (((long)z * yd + gy) * xd + gx) * C;
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const f32x4 acc = mfma_bf16(a[r], b, f32x4{0.f, 0.f, 0.f, 0.f});
-            // D row 4 g + i of row tile r = output channel 16 r + 4 g + i of pixel j
-            float zv[4], v[4];
+        for (int q = 0; q < 2; q++) {
+            uint2 vp[2], zp[2];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                zv[i] = acc[i] + bias[16 * r + 4 * g + i];
-                v[i] = gelu(zv[i]);
+            for (int h = 0; h < 2; h++) {
+                const int r = 2 * q + h;
+                const f32x4 acc = mfma_bf16(a[r], b, f32x4{0.f, 0.f, 0.f, 0.f});
+                float zv[4], v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    zv[i] = acc[i] + bias[channel(r, g, i)];
+                    v[i] = gelu(zv[i]);
+                }
+                vp[h] = pack4(v);
+                zp[h] = pack4(zv);
             }
             if (ok) {
-                *reinterpret_cast<uint2 *>(out + o + 16 * r + 4 * g) = pack4(v);
-                if (zsave) *reinterpret_cast<uint2 *>(zsave + o + 16 * r + 4 * g) = pack4(zv);
+                const long oc = o + 32 * q + 8 * g;
+                *reinterpret_cast<uint4 *>(out + oc) = make_uint4(vp[0].x, vp[0].y, vp[1].x, vp[1].y);
+                if (zsave) *reinterpret_cast<uint4 *>(zsave + oc) = make_uint4(zp[0].x, zp[0].y, zp[1].x, zp[1].y);
             }
         }
     }
@@ -685,7 +699,7 @@ __global__ __launch_bounds__(256) void sur_lift_wgrad_kernel(const float *__rest
                                                              float *__restrict__ part, int xd, int yd, int nz, int zf,
                                                              float rscale) {
     __shared__ __attribute__((aligned(16))) unsigned short dzT[C * DZS];
-    __shared__ float in[3][HS][HS];
+    __shared__ unsigned short in[3][HS][HS];
     const int ntx = (xd + TS - 1) / TS, nty = (yd + TS - 1) / TS, npl = ntx * nty, ntile = npl * nz;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane & 15, g = lane >> 4;
     const int nbytes = nz * yd * xd * C * 2;
@@ -710,7 +724,7 @@ __global__ __launch_bounds__(256) void sur_lift_wgrad_kernel(const float *__rest
                 const int k = 16 * nt + j, kc = k < 27 ? k : 0, tap = kc / 3, pl = kc % 3, dy = tap / 3, dx = tap % 3;
                 u16x8 bv;
 #pragma unroll
-                for (int u = 0; u < 8; u++) bv[u] = (k < 27) ? f2bf(in[pl][row + dy][px0 + u + dx]) : (unsigned short)0;
+                for (int u = 0; u < 8; u++) bv[u] = (k < 27) ? in[pl][row + dy][px0 + u + dx] : (unsigned short)0;
                 acc[nt] = mfma_bf16(A, __builtin_bit_cast(bf16x8, bv), acc[nt]);
             }
         }
