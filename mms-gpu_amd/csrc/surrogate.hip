@@ -51,6 +51,7 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 __device__ __forceinline__ unsigned short f2bf(float x) { return __builtin_bit_cast(unsigned short, (__bf16)x); }
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ unsigned pack2(float a, float b) {
     return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
@@ -273,11 +274,26 @@ constexpr size_t CONV_LDS = sizeof(unsigned short) * ((size_t)HS * HS * CP + 9 *
 // and LDS reads interleave.  With EPI 1 the two channel
 // halves' projections of a pixel meet in LDS (half 0 + half 1) and are stored
 // at the start of the next tile, after its first barrier.
+// Output channel (within a 32-channel half) of row 4 g + i of row tile r, and
+// the LDS row of a weight row (tap, channel).  WIDE: a lane's rows of both tiles
+// are eight consecutive channels of a pixel and its stores 16 bytes (8-byte
+// stores: conv2 with the spectral term 398 -> 382 us on 1024 x 1024 x 4, 24
+// layers of 128 x 128 57.8 -> 51.5; conv1 there 44.5 -> 39.1).  The fused
+// projection keeps the plain order of its sums, the spectral backward pass is
+// short of registers for the held half.
+template <bool WIDE>
+__device__ __forceinline__ int conv_channel(int r, int g, int i) { return WIDE ? 8 * g + 4 * r + i : 16 * r + 4 * g + i; }
+template <bool WIDE>
+__device__ __forceinline__ int conv_row(int row) {
+    const int c = row & 31;
+    return WIDE ? (row & ~31) + 16 * ((c >> 2) & 1) + 4 * (c >> 3) + (c & 3) : row;
+}
 constexpr int NT8 = 512, WPT8 = (WCH + NT8 - 1) / NT8;
 constexpr size_t CONV8_LDS = CONV_LDS + sizeof(float) * 2 * 2 * 4 * 4 * 16;
 template <int EPI, bool SPEC>
 __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
     extern __shared__ __attribute__((aligned(16))) unsigned short lds[];
+    constexpr bool WIDE = EPI == 0 || (EPI == 2 && !SPEC);
     unsigned short *win = lds;                 // [HS * HS][CP]
     unsigned short *wt = lds + HS * HS * CP;   // [9 * 64][CP]
     float *pproj = reinterpret_cast<float *>(lds + HS * HS * CP + 9 * C * CP);  // [slot][half][pg][c][j]
@@ -327,7 +343,7 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
 #pragma unroll
         for (int q = 0; q < NW; q++) {
             const int e = tid + NT8 * q, row = e >> 3, ch = e & 7;
-            *reinterpret_cast<uint4 *>(wt + row * CP + 8 * ch) = v[q];
+            *reinterpret_cast<uint4 *>(wt + conv_row<WIDE>(row) * CP + 8 * ch) = v[q];
         }
     }
     const int lane = tid & 63, wave = tid >> 6, j = lane & 15, g = lane >> 4;
@@ -338,7 +354,7 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
     for (int r = 0; r < 2; r++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            const int co = 32 * hf + 16 * r + 4 * g + i;
+            const int co = 32 * hf + conv_channel<WIDE>(r, g, i);
             bias_c[r][i] = EPI == 2 ? 0.0f : A.bias[co];
             wp_c[r][i] = EPI == 1 ? A.wp[co] : 0.0f;
         }
@@ -364,12 +380,13 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
     bool have = false;
     float proj = 0.0f;
     int slot = 0;  // EPI 1: projection partials of the epilogue run in this iteration
-    // one 4-channel block (r, c) of the held tile's epilogue
+    // one 4-channel block (r, c) of the held tile's epilogue (WIDE: block (1, c) stores both)
+    uint2 zlo = make_uint2(0u, 0u), vlo = make_uint2(0u, 0u);
     auto epi_block = [&](int r, int c) {
         const int gx = hx0 + j, gy = hy0 + 4 * pg + c;
         const bool ok = have && gx < xd && gy < yd;
         const long pix = ((long)hz0 * yd + gy) * xd + gx;
-        const int bo = ok ? (int)((pix * C + 32 * hf + 16 * r + 4 * g) * 2) : nact;  // out of range if not ok
+        const int bo = ok ? (int)((pix * C + 32 * hf + conv_channel<WIDE>(WIDE ? 0 : r, g, 0)) * 2) : nact;  // out of range if not ok
         float zz[4], v[4];
         if (EPI == 2) {
             unpack4(hz[c][r], zz);
@@ -383,11 +400,15 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
                 if (EPI == 1) proj += bf2f(f2bf(v[i])) * wp_c[r][i];
             }
             const uint2 zp = pack4(zz);
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, zp), r_zs, bo, 0, 0);
+            if (!WIDE) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, zp), r_zs, bo, 0, 0);
+            else if (r == 0) zlo = zp;
+            else __builtin_amdgcn_raw_buffer_store_b128((u32x4{zlo.x, zlo.y, zp.x, zp.y}), r_zs, bo, 0, 0);
         }
         if (EPI != 1) {
             const uint2 vp = pack4(v);
-            __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, vp), r_out, bo, 0, 0);
+            if (!WIDE) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, vp), r_out, bo, 0, 0);
+            else if (r == 0) vlo = vp;
+            else __builtin_amdgcn_raw_buffer_store_b128((u32x4{vlo.x, vlo.y, vp.x, vp.y}), r_out, bo, 0, 0);
         }
         if (EPI == 1 && r == 1) {
             // this half's 32 channels of pixel j: lanes j, j + 16, j + 32, j + 48
@@ -436,9 +457,9 @@ __global__ __launch_bounds__(512) void sur_conv8_kernel(ConvArgs A) {
 #pragma unroll
             for (int r = 0; r < 2; r++) {
                 pzin[c][r] = make_uint2(0u, 0u);
-                if (EPI == 2 && ok) pzin[c][r] = *reinterpret_cast<const uint2 *>(A.zin + pix * C + 32 * hf + 16 * r + 4 * g);
+                if (EPI == 2 && ok) pzin[c][r] = *reinterpret_cast<const uint2 *>(A.zin + pix * C + 32 * hf + conv_channel<WIDE>(r, g, 0));
                 if (spec)
-                    sa[c][r] = *reinterpret_cast<const bf16x8 *>(A.x2t + (srow * C + 32 * hf + 16 * r + j) * 32 + 8 * g);
+                    sa[c][r] = *reinterpret_cast<const bf16x8 *>(A.x2t + (srow * C + 32 * hf + conv_channel<WIDE>(r, j >> 2, j & 3)) * 32 + 8 * g);
             }
         }
         if (spec) sb = *reinterpret_cast<const bf16x8 *>(A.bxt + (long)(x0 + j < xd ? x0 + j : xd - 1) * 32 + 8 * g);
