@@ -296,8 +296,8 @@ int launch_zero_nonmagnetic(float *m, const uint8_t *matl, long n, hipStream_t s
 int launch_fill_f32(float *p, float v, long n, hipStream_t s);
 
 // ------------------------------------------------------------ host copies --
-// The caller's arrays to or from the device through pinned chunks, all of a
-// call back to back, ordered on the stream; a null host array is skipped.  To
+// The caller's arrays to or from the device, large ones through pinned chunks,
+// all of a call back to back, ordered on the stream; a null host array is skipped.  To
 // the device: the host arrays may be read until the stream is waited for (as
 // every entry point does before it returns).  To the host: the arrays are
 // complete.  transfer_user: +1 / -1 per live context, trainer

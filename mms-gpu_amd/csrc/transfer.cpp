@@ -26,7 +26,12 @@ namespace {
 
 constexpr int kSlots = 4;
 constexpr size_t kChunk = 4u << 20;   // largest chunk, and a slot's size
-constexpr size_t kRuntime = 3u << 19;  // below 1.5 MB the runtime's own pageable copy (0.8 MB: 40 us) is as good
+// Below these sizes the runtime's own pageable copy is as good or better.  To
+// the host: 1.5 MB 121 us against 115, 4 MB 291 against 241.  To the device it
+// moves 32 GB/s by itself, a single thread's chunks 30 (set_m of 2 MB 85 us
+// against 108, 4 MB 141 / 170, 8 MB 256 / 270), and only several threads are
+// faster: 16 MB 474 / 465 (new arrays 625 / 569), 24 MB 681 / 625, 48 MB 1662 / 1155.
+constexpr size_t kRuntimeDown = 3u << 19, kRuntimeUp = 16u << 20;
 constexpr size_t kAlone = 12u << 20;   // copies of this size and more use kThreads threads
 constexpr int kThreads = 4;           // divides kSlots
 constexpr size_t kKeep = 4;
@@ -131,7 +136,7 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
     for (int i = 0; i < count; i++)
         if (x[i].host) total += x[i].bytes;
     if (!total) return 0;
-    if (total < kRuntime) {
+    if (total < (to_device ? kRuntimeUp : kRuntimeDown)) {
         for (int i = 0; i < count; i++)
             if (x[i].host)
                 MMS_HIP(hipMemcpyAsync(to_device ? x[i].dev : x[i].host, to_device ? x[i].host : x[i].dev, x[i].bytes,
