@@ -131,29 +131,39 @@ bool run_pieces(Ring *r, const std::vector<Piece> &pieces, bool to_device, int w
     return true;
 }
 
+// the runtime's own copies, to the host complete on return
+int run_runtime(const Xfer *x, int count, bool to_device, hipStream_t s) {
+    for (int i = 0; i < count; i++)
+        if (x[i].host)
+            MMS_HIP(hipMemcpyAsync(to_device ? x[i].dev : x[i].host, to_device ? x[i].host : x[i].dev, x[i].bytes,
+                                   to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s));
+    if (!to_device) MMS_HIP(hipStreamSynchronize(s));
+    return 0;
+}
+
 int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
     size_t total = 0;
     for (int i = 0; i < count; i++)
         if (x[i].host) total += x[i].bytes;
     if (!total) return 0;
-    if (total < (to_device ? kRuntimeUp : kRuntimeDown)) {
-        for (int i = 0; i < count; i++)
-            if (x[i].host)
-                MMS_HIP(hipMemcpyAsync(to_device ? x[i].dev : x[i].host, to_device ? x[i].host : x[i].dev, x[i].bytes,
-                                       to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s));
-        if (!to_device) MMS_HIP(hipStreamSynchronize(s));
-        return 0;
-    }
+    if (total < (to_device ? kRuntimeUp : kRuntimeDown)) return run_runtime(x, count, to_device, s);
     // events and threads on the stream's device, whatever the caller's is
     int caller = 0;
     hipDevice_t device = 0;
     MMS_HIP(hipGetDevice(&caller));
     MMS_HIP(hipStreamGetDevice(s, &device));
+    if (caller != device) MMS_HIP(hipSetDevice(device));
+    Ring *r = ring_take(device);
+    if (caller != device) MMS_HIP(hipSetDevice(caller));
+    if (!r) {  // no pinned memory to be had
+        (void)hipGetLastError();
+        return run_runtime(x, count, to_device, s);
+    }
     const int nt = total >= kAlone ? kThreads : 1;
     // A chunk costs about 14 us of DMA start and event on top of its bytes at
     // 53 GB/s, and the last one's CPU copy is not overlapped: both together are
     // least at a chunk of sqrt(14 us x 50 GB/s x total), in steps of 64 KB
-    // (0.8 MB in one piece, 2.3 MB in two, 17 MB in five).
+    // (2.3 MB in two pieces, 17 MB in five).
     size_t chunk = (size_t)sqrt(7e5 * (double)total);
     chunk = std::min(kChunk, (chunk + 65535) & ~(size_t)65535);
     std::vector<Piece> pieces;
@@ -161,10 +171,6 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
         for (size_t o = 0; x[i].host && o < x[i].bytes; o += chunk)
             pieces.push_back({static_cast<char *>(x[i].host) + o, static_cast<char *>(x[i].dev) + o,
                               std::min(chunk, x[i].bytes - o)});
-    if (caller != device) MMS_HIP(hipSetDevice(device));
-    Ring *r = ring_take(device);
-    if (caller != device) MMS_HIP(hipSetDevice(caller));
-    MMS_CHECK(r, "no pinned memory for a host copy");
     std::atomic<bool> ok(true);
     std::vector<std::thread> th;
     int started = 1;  // this thread takes chunks 0 mod nt

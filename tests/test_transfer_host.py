@@ -25,3 +25,18 @@ with mg.Film(n, 1, 1, F(5e-9), F(5e-9), F(5e-9), demag=0) as g:
     assert len(copies()) > 1 and all(s != M.ctypes.data for _, s, _ in copies())
     assert np.array_equal(g.get_m(), M)
 """)
+
+
+def test_a_call_without_pinned_memory_is_the_runtimes_copy(tmp_path):
+    """Where the chunks' memory cannot be had, both directions still serve
+    every array, and the next call tries the chunks again."""
+    run(tmp_path, FILM.replace("200000", "2000000") + r"""
+stub.stub_fail_pinned(1)
+f.set_m(M)
+out = f.get_m()
+assert np.array_equal(out, M) and len(copies()) == 2, copies()
+stub.stub_fail_pinned(0)
+stub.stub_clear()
+f.set_m(-M)
+assert np.array_equal(f.get_m(), -M) and len(copies()) > 2
+""")
