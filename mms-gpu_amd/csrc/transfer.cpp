@@ -131,22 +131,24 @@ bool run_pieces(Ring *r, const std::vector<Piece> &pieces, bool to_device, int w
     return true;
 }
 
-// the runtime's own copies, to the host complete on return
-int run_runtime(const Xfer *x, int count, bool to_device, hipStream_t s) {
-    for (int i = 0; i < count; i++)
-        if (x[i].host)
-            MMS_HIP(hipMemcpyAsync(to_device ? x[i].dev : x[i].host, to_device ? x[i].host : x[i].dev, x[i].bytes,
-                                   to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s));
-    if (!to_device) MMS_HIP(hipStreamSynchronize(s));
+// the runtime's own copy
+int copy_runtime(const Xfer &x, bool to_device, hipStream_t s) {
+    MMS_HIP(hipMemcpyAsync(to_device ? x.dev : x.host, to_device ? x.host : x.dev, x.bytes,
+                           to_device ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost, s));
     return 0;
 }
 
-int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
-    size_t total = 0;
-    for (int i = 0; i < count; i++)
-        if (x[i].host) total += x[i].bytes;
-    if (!total) return 0;
-    if (total < (to_device ? kRuntimeUp : kRuntimeDown)) return run_runtime(x, count, to_device, s);
+// Memory the runtime knows (pinned, managed or a device's) is copied by DMA
+// without a chunk in between, and may not be the CPU's to read.
+bool pageable(const void *p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();
+    return true;
+}
+
+// the arrays of `mask` through a ring; -1: no pinned memory to be had
+int run_ring(const Xfer *x, int count, unsigned mask, size_t total, bool to_device, hipStream_t s) {
     // events and threads on the stream's device, whatever the caller's is
     int caller = 0;
     hipDevice_t device = 0;
@@ -155,9 +157,9 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
     if (caller != device) MMS_HIP(hipSetDevice(device));
     Ring *r = ring_take(device);
     if (caller != device) MMS_HIP(hipSetDevice(caller));
-    if (!r) {  // no pinned memory to be had
+    if (!r) {
         (void)hipGetLastError();
-        return run_runtime(x, count, to_device, s);
+        return -1;
     }
     const int nt = total >= kAlone ? kThreads : 1;
     // A chunk costs about 14 us of DMA start and event on top of its bytes at
@@ -168,7 +170,7 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
     chunk = std::min(kChunk, (chunk + 65535) & ~(size_t)65535);
     std::vector<Piece> pieces;
     for (int i = 0; i < count; i++)
-        for (size_t o = 0; x[i].host && o < x[i].bytes; o += chunk)
+        for (size_t o = 0; (mask >> i & 1) && o < x[i].bytes; o += chunk)
             pieces.push_back({static_cast<char *>(x[i].host) + o, static_cast<char *>(x[i].dev) + o,
                               std::min(chunk, x[i].bytes - o)});
     std::atomic<bool> ok(true);
@@ -190,6 +192,35 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
     for (std::thread &t : th) t.join();
     ring_give(r);
     MMS_CHECK(ok.load(), to_device ? "copy to the device failed" : "copy to the host failed");
+    return 0;
+}
+
+// a call has at most 32 arrays (rk4_step: six)
+int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
+    const size_t line = to_device ? kRuntimeUp : kRuntimeDown;
+    size_t total = 0;
+    for (int i = 0; i < count; i++)
+        if (x[i].host) total += x[i].bytes;
+    if (!total) return 0;
+    unsigned ring = 0;  // arrays that take the chunks
+    if (total >= line) {
+        total = 0;
+        for (int i = 0; i < count; i++)
+            if (x[i].host && pageable(x[i].host)) {
+                ring |= 1u << i;
+                total += x[i].bytes;
+            }
+        if (total < line) ring = 0;
+    }
+    for (int i = 0; i < count; i++)
+        if (x[i].host && !(ring >> i & 1) && copy_runtime(x[i], to_device, s)) return 1;
+    if (ring) {
+        const int st = run_ring(x, count, ring, total, to_device, s);
+        if (st > 0) return 1;
+        for (int i = 0; st < 0 && i < count; i++)
+            if ((ring >> i & 1) && copy_runtime(x[i], to_device, s)) return 1;
+    }
+    if (!to_device) MMS_HIP(hipStreamSynchronize(s));
     return 0;
 }
 

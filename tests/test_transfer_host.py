@@ -40,3 +40,32 @@ stub.stub_clear()
 f.set_m(-M)
 assert np.array_equal(f.get_m(), -M) and len(copies()) > 2
 """)
+
+
+def test_memory_the_runtime_knows_is_copied_directly(tmp_path):
+    """Pinned and device arrays of the caller, also inside a larger
+    allocation, go to the runtime as they are; a call's pageable arrays beside
+    them take the chunks if they are large enough by themselves."""
+    run(tmp_path, FILM.replace("200000", "2000000") + r"""
+check = lambda rc: (_ for _ in ()).throw(AssertionError(mg.last_error())) if rc else None
+for alloc in (stub.stub_pin, stub.stub_device):
+    p = alloc(M.nbytes + 64) + 64
+    C.memmove(p, M.ctypes.data, M.nbytes)
+    a = np.ctypeslib.as_array((C.c_float * M.size).from_address(p))
+    stub.stub_clear()
+    f.set_m(a)
+    assert [(s, b) for _, s, b in copies()] == [(p, M.nbytes)], copies()
+    a[:] = 0
+    stub.stub_clear()
+    check(lib.mms_get_m(f._ctx, a))
+    assert [(d, b) for d, _, b in copies()] == [(p, M.nbytes)] and np.array_equal(a, M)
+# Hfield's three results, the field pinned: the others (16 MB) by chunks
+n, dims, d = 2000000, (2000, 1000, 1), (F(5e-9),) * 3
+H = np.ctypeslib.as_array((C.c_float * (3 * n)).from_address(stub.stub_pin(12 * n)))
+ch, pot = np.full(n, F(7)), np.full(n, F(7))
+stub.stub_clear()
+assert mg.Hfield(M, H, ch, pot, F(0), *dims, *d, 3, F(1.2566e-6), F(8.6e5), F(1.3e-11), 1, 1, 0, 1) == 0
+to = [t for t, _, b in copies()]
+assert to.count(H.ctypes.data) == 1 and ch.ctypes.data not in to and pot.ctypes.data not in to
+assert not ch.any() and not pot.any()  # the stand-in's device memory
+""")
