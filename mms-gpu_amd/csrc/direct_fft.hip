@@ -496,10 +496,13 @@ int launch_rows(const FftArgs &A, bool from_m, hipStream_t s) {
 template <int N, int ZD>
 int launch_columns_z(const FftArgs &A, hipStream_t s) {
     if constexpr (ZD * N <= 8192) {
-        // set on every call (a host-side table write) rather than remembered per device
+        // The limit is the kernel's, not this call's: callers of other depths
+        // share it.  Set on every call (a host-side table write) rather than
+        // remembered per device.
+        constexpr int layers = ZD ? ZD : (8192 / N < 16 ? 8192 / N : 16);
         const size_t lds = sizeof(cd) * (size_t)A.zd * slots(N);
         MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_columns<N, ZD>),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(cd) * layers * slots(N))));
         hipLaunchKernelGGL((fft_columns<N, ZD>), dim3(A.nxh), dim3(A.zd * (N / 8)), lds, s, A);
         MMS_HIP(hipGetLastError());
         return 0;
