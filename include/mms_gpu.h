@@ -217,9 +217,9 @@ int mms_potential_probes_f64(mms_ctx *ctx, const float *charge, const int64_t *p
 
 /* Autotuner: time the solver's launch shapes on the context's current
  * charge (call after mms_set_m) -- FMM leaf width in {4, 8} x M2L column tiles
- * in {4, 8}; direct sum source-chunk multiplier in {1, 2, 4} -- `reps` solves
- * each, keep the fastest.  Accuracy settings (P, M2L precision) are not
- * changed.  report (may be NULL) receives one line per candidate. */
+ * in {4, 8}; direct sum source-chunk multiplier in {1, 2, 4} where the pair loop
+ * serves the grid (its other forms have one shape) -- `reps` solves each, keep
+ * the fastest.  Accuracy settings (P, M2L precision) are not changed.  report (may be NULL) receives one line per candidate. */
 int mms_autotune(mms_ctx *ctx, int reps, char *report, int report_len);
 /* Current launch shape: leaf width, M2L column tiles, direct split. */
 int mms_get_shape(mms_ctx *ctx, int *leaf_width, int *m2l_cols, int *direct_split);

@@ -480,6 +480,10 @@ extern "C" int mms_autotune(mms_ctx *c, int reps, char *report, int report_len) 
         rep += line;
     } else if (c->p.solver == MMS_SOLVER_DIRECT_REFGPU) {
         rep += "reference-order direct sum: fixed launch shape (the reference's 1024-way split)\n";
+    } else if (c->direct.form != kDirectChunks) {
+        // only the pair loop has source chunks to choose
+        rep += c->direct.form == kDirectTable ? "chosen: direct sum by the 1/r table (one launch shape)\n"
+                                              : "chosen: direct sum by transforms (one launch shape)\n";
     } else {
         int best_s = c->p.direct_split;
         double best = 1e30;
