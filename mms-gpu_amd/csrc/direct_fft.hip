@@ -268,29 +268,33 @@ __device__ __forceinline__ void layer_product(cd *lds, const double (&g)[ZD]) {
         lds[z * slots(N)] = make_double2(im, re);
     }
 }
-// ... of any number of layers up to 16, its spectrum read from memory
-template <int N>
-__device__ __forceinline__ void layers_product(cd *lds, const double *__restrict__ gh, long gstride, int zd) {
-    constexpr int ZM = 16;
+// ... of zd layers, at most ZM, whose spectrum is read from memory, all of it
+// at once: a load a product, each waited for, took most of the kernel (a step of a
+// 20 x 20 x 16 film 145 us, so 74; 128 x 64 x 16 176 / 94; 500 x 64 x 7 161 /
+// 122).  Layers past the last add 0.
+template <int ZM, int N>
+__device__ __forceinline__ void layers_product(cd *lds, const double *gh, long gstride, int zd) {
     cd in[ZM];
+    double g[ZM];
 #pragma unroll
-    for (int z = 0; z < ZM; z++)
-        if (z < zd) in[z] = lds[z * slots(N)];
-    for (int z = 0; z < zd; z++) {
+    for (int z = 0; z < ZM; z++) {
+        g[z] = gh[min(z, zd - 1) * gstride];
+        in[z] = z < zd ? lds[z * slots(N)] : make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int z = 0; z < ZM; z++) {
         double re = 0.0, im = 0.0;
 #pragma unroll
-        for (int s = 0; s < ZM; s++)
-            if (s < zd) {
-                const double gv = gh[(z > s ? z - s : s - z) * gstride];
-                re = fma(gv, in[s].x, re);
-                im = fma(gv, in[s].y, im);
-            }
-        lds[z * slots(N)] = make_double2(im, re);
+        for (int s = 0; s < ZM; s++) {
+            re = fma(g[z > s ? z - s : s - z], in[s].x, re);
+            im = fma(g[z > s ? z - s : s - z], in[s].y, im);
+        }
+        if (z < zd) lds[z * slots(N)] = make_double2(im, re);
     }
 }
 
 template <int N, int ZD>
-__global__ __launch_bounds__(ZD ? ZD * N / 8 : 1024) void fft_columns(FftArgs A) {
+__global__ __launch_bounds__(ZD ? ZD * N / 8 : (16 * N / 8 < 1024 ? 16 * N / 8 : 1024)) void fft_columns(FftArgs A) {
     extern __shared__ __attribute__((aligned(16))) char fft_lds[];
     cd *lds = reinterpret_cast<cd *>(fft_lds);
     constexpr int T = N / 8;
@@ -335,7 +339,10 @@ __global__ __launch_bounds__(ZD ? ZD * N / 8 : 1024) void fft_columns(FftArgs A)
             if (ky < N) layer_product<ZD, N>(lds + slot(ky), g[i]);
         }
     } else {
-        for (int ky = threadIdx.x; ky < N; ky += blockDim.x) layers_product<N>(lds + slot(ky), spectrum(ky), gs, A.zd);
+        for (int ky = threadIdx.x; ky < N; ky += blockDim.x) {
+            if (A.zd <= 8) layers_product<8, N>(lds + slot(ky), spectrum(ky), gs, A.zd);
+            else layers_product<16, N>(lds + slot(ky), spectrum(ky), gs, A.zd);
+        }
     }
     __syncthreads();
     fft<N>(buf, t, tw);
