@@ -17,6 +17,10 @@
 //   fft_columns  one kx per workgroup: y transforms of every layer, product
 //                with the kernel's spectrum, inverse y transforms, in place;
 //   fft_back     inverse x transforms, two real rows each, FP32 potential.
+// A call that keeps no tables forms them in the first two (fft_rows_tables,
+// fft_columns<.., true>): three more launches before them took 12 of 26 us on
+// 33 x 32 x 6 (now 15; the pair loop 23) and 9 of 37 on 1300 x 5 x 1, where
+// the padded length is 40 times the film (now 28; 23).
 // Measured against the pair loop (FP32 rsqrt pairs, 3.8e12 a second): the
 // 256 x 256 x 3 potential on host arrays 9.46 -> 0.11 ms, an RK4 step of a
 // 161 x 117 x 3 film 3.67 -> 0.086 ms (fft_rows 6.8 us with div M, fft_columns
@@ -37,9 +41,16 @@ typedef double2 cd;
 
 constexpr int kTw = 4096;  // entries of the twiddle table, the longest transform
 
-__device__ __forceinline__ cd cmul(cd a, cd b) { return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); }
+// Several kernels run the same transform, and their results must not depend on
+// which one: no multiply-adds but the written ones.
+#pragma clang fp contract(off)
+
+__device__ __forceinline__ cd cmul(cd a, cd b) {
+    return make_double2(fma(-a.y, b.y, a.x * b.x), fma(a.x, b.y, a.y * b.x));
+}
 __device__ __forceinline__ cd cadd(cd a, cd b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ cd csub(cd a, cd b) { return make_double2(a.x - b.x, a.y - b.y); }
+__device__ __forceinline__ cd cfma(double h, cd a, cd b) { return make_double2(fma(h, a.x, b.x), fma(h, a.y, b.y)); }
 __device__ __forceinline__ cd mul_mi(cd a) { return make_double2(a.y, -a.x); }  // -i a
 
 // LDS slot of element i: one free slot in nine keeps the strided stores of
@@ -64,14 +75,14 @@ __device__ __forceinline__ void dft(cd (&v)[R]) {
         const double h = 0.70710678118654752440;  // sqrt(1/2)
         dft4(v[0], v[2], v[4], v[6]);
         dft4(v[1], v[3], v[5], v[7]);
-        const cd t1 = make_double2(h * (v[3].x + v[3].y), h * (v[3].y - v[3].x));    // w_8 v
-        const cd t2 = mul_mi(v[5]);                                                  // w_8^2 v
-        const cd t3 = make_double2(h * (v[7].y - v[7].x), -h * (v[7].x + v[7].y));  // w_8^3 v
+        // w_8 v = h t1, w_8^2 v = t2, w_8^3 v = h t3
+        const cd t1 = make_double2(v[3].x + v[3].y, v[3].y - v[3].x), t2 = mul_mi(v[5]);
+        const cd t3 = make_double2(v[7].y - v[7].x, -(v[7].x + v[7].y));
         const cd e0 = v[0], e1 = v[2], e2 = v[4], e3 = v[6], o0 = v[1];
         v[0] = cadd(e0, o0); v[4] = csub(e0, o0);
-        v[1] = cadd(e1, t1); v[5] = csub(e1, t1);
+        v[1] = cfma(h, t1, e1); v[5] = cfma(-h, t1, e1);
         v[2] = cadd(e2, t2); v[6] = csub(e2, t2);
-        v[3] = cadd(e3, t3); v[7] = csub(e3, t3);
+        v[3] = cfma(h, t3, e3); v[7] = cfma(-h, t3, e3);
     }
 }
 
@@ -119,13 +130,21 @@ __device__ __forceinline__ void fft_pass(cd *buf, int t, cd w) {
 // for between two barriers.
 template <int N>
 constexpr int first_radix() { return __builtin_ctz(N) % 3 == 1 ? 2 : (__builtin_ctz(N) % 3 == 2 ? 4 : 8); }
+// FORM: formed instead, by the expression that fills the table.
 struct Twiddles { cd w[4]; };
-template <int N>
+__device__ __forceinline__ cd twiddle(int i) {
+    double s, c;
+    sincospi(-2.0 * (double)i / (double)kTw, &s, &c);
+    return make_double2(c, s);
+}
+template <int N, bool FORM = false>
 __device__ __forceinline__ Twiddles fft_twiddles(int t, const cd *__restrict__ tw) {
     Twiddles r;
 #pragma unroll
-    for (int p = 0, ns = first_radix<N>(); p < 4; p++, ns *= 8)
-        r.w[p] = ns < N ? tw[(t & (ns - 1)) * (kTw / (ns * 8))] : make_double2(0.0, 0.0);
+    for (int p = 0, ns = first_radix<N>(); p < 4; p++, ns *= 8) {
+        const int i = (t & (ns - 1)) * (kTw / (ns * 8));
+        r.w[p] = ns < N ? (FORM ? twiddle(i) : tw[i]) : make_double2(0.0, 0.0);
+    }
     return r;
 }
 template <int N, int NS, int P>
@@ -157,24 +176,29 @@ struct FftArgs {
     const float *m;    // FP32 SoA magnetisation
     float *phi;
     cd *w;             // [zd][nxh][yd]
-    const double *ghat;  // [zd][nxh][ny / 2 + 1]
+    double *ghat;      // [zd][nxh][ny / 2 + 1]; before its y transforms [zd][nxh][|dy|]
     const cd *tw;
     int *flags;        // [workgroups of fft_rows], then the combined flag
     int nflags;
     int xd, yd, zd, nxh, ny;
     float dx, dy, dz, ay, az;
     double scale;
+    double ayd, azd, gscale;  // of the kernel's spectrum
 };
 
-template <int N, bool FROM_M>
-__global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
+// workgroups of a layer's rows of charges
+template <int N>
+__device__ __forceinline__ int row_groups(int yd) { return (yd + 2 * row_batch<N>() - 1) / (2 * row_batch<N>()); }
+
+// rows 2 B bx .. of layer z
+template <int N, bool FROM_M, bool FORM>
+__device__ __forceinline__ void rows_of(const FftArgs A, cd *lds, int bx, int z) {
     constexpr int B = row_batch<N>(), T = N / 8;
-    __shared__ cd lds[B * slots(N)];
     const int f = threadIdx.x / T, t = threadIdx.x % T;
-    const int z = blockIdx.y, y0 = blockIdx.x * 2 * B, ya = y0 + 2 * f;
+    const int y0 = bx * 2 * B, ya = y0 + 2 * f;
     const long plane = (long)A.xd * A.yd, n = plane * A.zd;
     const long row = (long)z * plane + (long)ya * A.xd;
-    const Twiddles tw = fft_twiddles<N>(t, A.tw);
+    const Twiddles tw = fft_twiddles<N, FORM>(t, A.tw);
     bool bad = false;
     // the rows' upper half is padding (xd <= N / 2).  Every load of a thread is
     // issued before one is used: none sits behind a branch
@@ -235,7 +259,7 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
         buf[slot(x)] = make_double2((double)q[k][0], (double)q[k][1]);
     }
     const int any = __syncthreads_or(bad ? 1 : 0);
-    if (threadIdx.x == 0) A.flags[blockIdx.y * gridDim.x + blockIdx.x] = any;
+    if (threadIdx.x == 0) A.flags[z * row_groups<N>(A.yd) + bx] = any;
     fft<N>(buf, t, tw);
     // spectra of the two real rows of each transform: with Z = FFT(a + i b),
     // A[k] = (Z[k] + conj Z[N-k]) / 2, B[k] = (Z[k] - conj Z[N-k]) / 2i
@@ -248,6 +272,65 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
                              : make_double2(0.5 * (u.x + v.x), 0.5 * (u.y - v.y));
         A.w[((long)z * A.nxh + k) * A.yd + y] = s;
     }
+}
+
+template <int N, bool FROM_M>
+__global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows(FftArgs A) {
+    __shared__ cd lds[row_batch<N>() * slots(N)];
+    rows_of<N, FROM_M, false>(A, lds, blockIdx.x, blockIdx.y);
+}
+
+// The tables' first launch: x transforms of the rows |dy| = 0 .. ny/2 of 1/r
+// (real and even in both axes) into ghat[dz][kx][|dy|] and the twiddles, by
+// workgroups nbx .. of each layer; the first nbx transform the charges' rows, where a
+// call forms its tables anew (nbx 0: a plan's tables).
+template <int N>
+__global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_rows_tables(FftArgs A, cd *tw, int nbx) {
+    constexpr int B = row_batch<N>(), T = N / 8;
+    __shared__ cd lds[B * slots(N)];
+    if ((int)blockIdx.x < nbx) {
+        rows_of<N, false, true>(A, lds, blockIdx.x, blockIdx.y);
+        return;
+    }
+    const int f = threadIdx.x / T, t = threadIdx.x % T, z = blockIdx.y, bk = blockIdx.x - nbx, nyh = A.ny / 2 + 1;
+    const int y = bk * B + f;
+    cd *buf = lds + f * slots(N);
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int x = t + k * T;
+        const double rx = (double)(x <= N / 2 ? x : N - x), ry = y * A.ayd, rz = z * A.azd;
+        const double r2 = rx * rx + ry * ry + rz * rz;
+        buf[slot(x)] = make_double2(r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0, 0.0);
+    }
+    const int nk = gridDim.x - nbx;
+    for (int i = ((int)blockIdx.y * nk + bk) * B * T + threadIdx.x; i < kTw; i += nk * gridDim.y * B * T) tw[i] = twiddle(i);
+    __syncthreads();
+    fft<N>(buf, t, fft_twiddles<N, true>(t, nullptr));
+    for (int i = threadIdx.x; i < B * (N / 2 + 1); i += B * T) {
+        const int r = i % B, k = i / B;
+        if (bk * B + r < nyh) A.ghat[((long)z * A.nxh + k) * nyh + bk * B + r] = lds[r * slots(N) + slot(k)].x;
+    }
+}
+
+// The tables' second launch: y transforms of the mirrored columns of
+// ghat, in place and scaled; one column of N elements by its N / 8 threads.
+template <int N>
+__device__ __forceinline__ void kernel_column(double *col, cd *buf, int t, const Twiddles &tw, double scale) {
+    constexpr int T = N / 8;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const int y = t + k * T;
+        buf[slot(y)] = make_double2(col[y <= N / 2 ? y : N - y], 0.0);
+    }
+    __syncthreads();
+    fft<N>(buf, t, tw);
+    for (int k = t; k <= N / 2; k += T) col[k] = buf[slot(k)].x * scale;
+}
+template <int N>
+__global__ __launch_bounds__(N / 8) void fft_kernel_columns(FftArgs A) {
+    __shared__ cd buf[slots(N)];
+    kernel_column<N>(A.ghat + ((long)blockIdx.y * A.nxh + blockIdx.x) * (N / 2 + 1), buf, threadIdx.x,
+                     fft_twiddles<N>(threadIdx.x, A.tw), A.gscale);
 }
 
 // the layers' product at one (kx, ky): out[z] = sum_z' ghat[|z - z'|] in[z'];
@@ -293,7 +376,8 @@ __device__ __forceinline__ void layers_product(cd *lds, const double *gh, long g
     }
 }
 
-template <int N, int ZD>
+// TAB: ghat holds the kernel's rows; their columns are transformed here first
+template <int N, int ZD, bool TAB>
 __global__ __launch_bounds__(ZD ? ZD * N / 8 : (16 * N / 8 < 1024 ? 16 * N / 8 : 1024)) void fft_columns(FftArgs A) {
     extern __shared__ __attribute__((aligned(16))) char fft_lds[];
     cd *lds = reinterpret_cast<cd *>(fft_lds);
@@ -302,6 +386,10 @@ __global__ __launch_bounds__(ZD ? ZD * N / 8 : (16 * N / 8 < 1024 ? 16 * N / 8 :
     cd *col = A.w + ((long)z * A.nxh + kx) * A.yd;
     cd *buf = lds + z * slots(N);
     const Twiddles tw = fft_twiddles<N>(t, A.tw);
+    if constexpr (TAB) {
+        kernel_column<N>(A.ghat + ((long)z * A.nxh + kx) * (N / 2 + 1), buf, t, tw, A.gscale);
+        __syncthreads();  // the layers' spectra are read below, buf is written again
+    }
     // the column's upper half is padding (yd <= N / 2); past yd its last entry, then 0
     cd v[4];
 #pragma unroll
@@ -310,7 +398,7 @@ __global__ __launch_bounds__(ZD ? ZD * N / 8 : (16 * N / 8 < 1024 ? 16 * N / 8 :
     // this thread's kernel spectrum, in flight during the first transform
     constexpr int NI = ZD ? (8 + ZD - 1) / ZD : 1;
     double g[NI][ZD ? ZD : 1];
-    auto spectrum = [&](int ky) { return A.ghat + (long)kx * (N / 2 + 1) + (ky <= N / 2 ? ky : N - ky); };
+    auto spectrum = [&](int ky) -> const double * { return A.ghat + (long)kx * (N / 2 + 1) + (ky <= N / 2 ? ky : N - ky); };
     if constexpr (ZD != 0) {
 #pragma unroll
         for (int i = 0; i < NI; i++) {
@@ -430,46 +518,6 @@ __global__ __launch_bounds__(row_batch<N>() * N / 8) void fft_back(FftArgs A) {
     }
 }
 
-__global__ __launch_bounds__(256) void fft_twiddle_kernel(cd *tw) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= kTw) return;
-    double s, c;
-    sincospi(-2.0 * (double)i / (double)kTw, &s, &c);
-    tw[i] = make_double2(c, s);
-}
-
-// Spectrum of 1/r (real and even in both axes): x transforms of the rows
-// |dy| = 0 .. ny/2 into a[dz][kx][y], then y transforms of the mirrored
-// columns, scaled.
-template <int N>
-__global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_rows(double *a, const cd *tw, int nyh, double ay,
-                                                                           double az) {
-    constexpr int T = N / 8;
-    __shared__ cd buf[slots(N)];
-    const int y = blockIdx.x, z = blockIdx.y, t = threadIdx.x % T;
-    for (int x = threadIdx.x; x < N; x += blockDim.x) {
-        const double rx = (double)(x <= N / 2 ? x : N - x), ry = y * ay, rz = z * az;
-        const double r2 = rx * rx + ry * ry + rz * rz;
-        buf[slot(x)] = make_double2(r2 > 0.0 ? 1.0 / sqrt(r2) : 0.0, 0.0);
-    }
-    __syncthreads();
-    fft<N>(buf, t, fft_twiddles<N>(t, tw));
-    for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) a[((long)z * (N / 2 + 1) + k) * nyh + y] = buf[slot(k)].x;
-}
-
-template <int N>
-__global__ __launch_bounds__(N / 8 < 64 ? 64 : N / 8) void fft_kernel_columns(const double *a, double *ghat, const cd *tw,
-                                                                              int nxh, double scale) {
-    constexpr int T = N / 8;
-    __shared__ cd buf[slots(N)];
-    const int t = threadIdx.x % T;
-    const long o = ((long)blockIdx.y * nxh + blockIdx.x) * (N / 2 + 1);
-    for (int y = threadIdx.x; y < N; y += blockDim.x) buf[slot(y)] = make_double2(a[o + (y <= N / 2 ? y : N - y)], 0.0);
-    __syncthreads();
-    fft<N>(buf, t, fft_twiddles<N>(t, tw));
-    for (int k = threadIdx.x; k <= N / 2; k += blockDim.x) ghat[o + k] = buf[slot(k)].x * scale;
-}
-
 int fft_len(int d) {
     int n = 64;
     while (n < 2 * d - 1) n <<= 1;
@@ -500,7 +548,17 @@ int launch_rows(const FftArgs &A, bool from_m, hipStream_t s) {
     return 0;
 }
 
-template <int N, int ZD>
+// the tables, with the charges' rows if the call has any
+template <int N>
+int launch_rows_tables(const FftArgs &A, cd *tw, bool charges, hipStream_t s) {
+    constexpr int B = row_batch<N>();
+    const int nbx = charges ? (A.yd + 2 * B - 1) / (2 * B) : 0;
+    hipLaunchKernelGGL((fft_rows_tables<N>), dim3(nbx + (A.ny / 2 + B) / B, A.zd), dim3(B * N / 8), 0, s, A, tw, nbx);
+    MMS_HIP(hipGetLastError());
+    return 0;
+}
+
+template <int N, int ZD, bool TAB>
 int launch_columns_z(const FftArgs &A, hipStream_t s) {
     if constexpr (ZD * N <= 8192) {
         // The limit is the kernel's, not this call's: callers of other depths
@@ -508,9 +566,9 @@ int launch_columns_z(const FftArgs &A, hipStream_t s) {
         // remembered per device.
         constexpr int layers = ZD ? ZD : (8192 / N < 16 ? 8192 / N : 16);
         const size_t lds = sizeof(cd) * (size_t)A.zd * slots(N);
-        MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_columns<N, ZD>),
+        MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&fft_columns<N, ZD, TAB>),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(cd) * layers * slots(N))));
-        hipLaunchKernelGGL((fft_columns<N, ZD>), dim3(A.nxh), dim3(A.zd * (N / 8)), lds, s, A);
+        hipLaunchKernelGGL((fft_columns<N, ZD, TAB>), dim3(A.nxh), dim3(A.zd * (N / 8)), lds, s, A);
         MMS_HIP(hipGetLastError());
         return 0;
     } else {
@@ -519,14 +577,14 @@ int launch_columns_z(const FftArgs &A, hipStream_t s) {
     }
 }
 
-template <int N>
+template <int N, bool TAB>
 int launch_columns(const FftArgs &A, hipStream_t s) {
     switch (A.zd) {
-    case 1: return launch_columns_z<N, 1>(A, s);
-    case 2: return launch_columns_z<N, 2>(A, s);
-    case 3: return launch_columns_z<N, 3>(A, s);
-    case 4: return launch_columns_z<N, 4>(A, s);
-    default: return launch_columns_z<N, 0>(A, s);
+    case 1: return launch_columns_z<N, 1, TAB>(A, s);
+    case 2: return launch_columns_z<N, 2, TAB>(A, s);
+    case 3: return launch_columns_z<N, 3, TAB>(A, s);
+    case 4: return launch_columns_z<N, 4, TAB>(A, s);
+    default: return launch_columns_z<N, 0, TAB>(A, s);
     }
 }
 
@@ -558,60 +616,77 @@ size_t direct_fft_table_bytes(const Grid &g) {
     return (sizeof(cd) * kTw + sizeof(double) * g.zd * nxh * nyh + 255) & ~(size_t)255;
 }
 size_t direct_fft_work_bytes(const Grid &g) {
-    const size_t nxh = fft_len(g.xd) / 2 + 1, nyh = fft_len(g.yd) / 2 + 1;
-    const size_t w = sizeof(cd) * g.zd * nxh * g.yd, a = sizeof(double) * g.zd * nxh * nyh;
-    return ((w > a ? w : a) + sizeof(int) * (row_blocks(fft_len(g.xd), g) + 1) + 511) & ~(size_t)255;
+    const int nx = fft_len(g.xd);
+    return (sizeof(cd) * g.zd * (nx / 2 + 1) * g.yd + sizeof(int) * (row_blocks(nx, g) + 1) + 255) & ~(size_t)255;
 }
 
-int direct_fft_tables(const Grid &g, void *table, void *work, hipStream_t s) {
-    const int nx = fft_len(g.xd), ny = fft_len(g.yd), nxh = nx / 2 + 1, nyh = ny / 2 + 1;
+static FftArgs fft_args(const Grid &g, void *table, void *work) {
+    const int nx = fft_len(g.xd), ny = fft_len(g.yd);
+    FftArgs A{};
+    A.tw = static_cast<const cd *>(table);
+    A.ghat = reinterpret_cast<double *>(static_cast<cd *>(table) + kTw);
+    A.w = static_cast<cd *>(work);
+    A.xd = g.xd; A.yd = g.yd; A.zd = g.zd; A.nxh = nx / 2 + 1; A.ny = ny;
+    A.flags = reinterpret_cast<int *>(A.w + (size_t)g.zd * A.nxh * g.yd);
+    A.nflags = row_blocks(nx, g);
+    A.dx = g.dx; A.dy = g.dy; A.dz = g.dz; A.ay = g.ay; A.az = g.az;
+    A.scale = (double)g.dy * (double)g.dz;
+    A.ayd = (double)g.dy / (double)g.dx;
+    A.azd = (double)g.dz / (double)g.dx;
+    A.gscale = A.scale / ((double)nx * (double)ny);
+    return A;
+}
+
+int direct_fft_tables(const Grid &g, void *table, hipStream_t s) {
+    const FftArgs A = fft_args(g, table, nullptr);
     cd *tw = static_cast<cd *>(table);
-    double *ghat = reinterpret_cast<double *>(tw + kTw), *a = static_cast<double *>(work);
-    const double ay = (double)g.dy / (double)g.dx, az = (double)g.dz / (double)g.dx;
-    const double scale = (double)g.dy * (double)g.dz / ((double)nx * (double)ny);
-    hipLaunchKernelGGL(fft_twiddle_kernel, dim3(kTw / 256), dim3(256), 0, s, tw);
-    MMS_HIP(hipGetLastError());
-#define X(N, ...)                                                                                                      \
-    hipLaunchKernelGGL((fft_kernel_rows<N>), dim3(nyh, g.zd), dim3(N / 8 < 64 ? 64 : N / 8), 0, s, a, tw, nyh, ay, az)
-    MMS_FFT_SIZES(X, nx, 0)
+#define X(N, ...) \
+    if (launch_rows_tables<N>(A, tw, false, s)) return 1
+    MMS_FFT_SIZES(X, 2 * (A.nxh - 1), 0)
+#undef X
+#define X(N, ...) hipLaunchKernelGGL((fft_kernel_columns<N>), dim3(A.nxh, A.zd), dim3(N / 8), 0, s, A)
+    MMS_FFT_SIZES(X, A.ny, 0)
 #undef X
     MMS_HIP(hipGetLastError());
-#define X(N, ...)                                                                                                 \
-    hipLaunchKernelGGL((fft_kernel_columns<N>), dim3(nxh, g.zd), dim3(N / 8 < 64 ? 64 : N / 8), 0, s, a, ghat, tw, \
-                       nxh, scale)
-    MMS_FFT_SIZES(X, ny, 0)
+    return 0;
+}
+
+static int fft_back_of(const FftArgs &A, hipStream_t s) {
+#define X(N, ...) \
+    if (launch_back<N>(A, s)) return 1
+    MMS_FFT_SIZES(X, 2 * (A.nxh - 1), 0)
 #undef X
-    MMS_HIP(hipGetLastError());
     return 0;
 }
 
 int direct_fft_potential(const Grid &g, const void *table, void *work, const float *m, float *rho, float *phi,
                          hipStream_t s) {
-    const int nx = fft_len(g.xd), ny = fft_len(g.yd), nxh = nx / 2 + 1, nyh = ny / 2 + 1;
-    FftArgs A{};
+    FftArgs A = fft_args(g, const_cast<void *>(table), work);
     A.rho = rho; A.rho_out = rho; A.m = m; A.phi = phi;
-    A.tw = static_cast<const cd *>(table);
-    A.ghat = reinterpret_cast<const double *>(A.tw + kTw);
-    A.w = static_cast<cd *>(work);
-    const size_t w = sizeof(cd) * (size_t)g.zd * nxh * g.yd, a = sizeof(double) * (size_t)g.zd * nxh * nyh;
-    A.flags = reinterpret_cast<int *>(static_cast<char *>(work) + (((w > a ? w : a) + 15) & ~(size_t)15));
-    A.nflags = row_blocks(nx, g);
-    A.xd = g.xd; A.yd = g.yd; A.zd = g.zd; A.nxh = nxh; A.ny = ny;
-    A.dx = g.dx; A.dy = g.dy; A.dz = g.dz; A.ay = g.ay; A.az = g.az;
-    A.scale = (double)g.dy * (double)g.dz;
 #define X(N, ...) \
     if (launch_rows<N>(A, m != nullptr, s)) return 1
-    MMS_FFT_SIZES(X, nx, 0)
+    MMS_FFT_SIZES(X, 2 * (A.nxh - 1), 0)
 #undef X
 #define X(N, ...) \
-    if (launch_columns<N>(A, s)) return 1
-    MMS_FFT_SIZES(X, ny, 0)
+    if (launch_columns<N, false>(A, s)) return 1
+    MMS_FFT_SIZES(X, A.ny, 0)
+#undef X
+    return fft_back_of(A, s);
+}
+
+int direct_fft_potential_once(const Grid &g, void *table, void *work, const float *rho, float *phi, hipStream_t s) {
+    FftArgs A = fft_args(g, table, work);
+    A.rho = rho; A.phi = phi;
+    cd *tw = static_cast<cd *>(table);
+#define X(N, ...) \
+    if (launch_rows_tables<N>(A, tw, true, s)) return 1
+    MMS_FFT_SIZES(X, 2 * (A.nxh - 1), 0)
 #undef X
 #define X(N, ...) \
-    if (launch_back<N>(A, s)) return 1
-    MMS_FFT_SIZES(X, nx, 0)
+    if (launch_columns<N, true>(A, s)) return 1
+    MMS_FFT_SIZES(X, A.ny, 0)
 #undef X
-    return 0;
+    return fft_back_of(A, s);
 }
 
 }  // namespace mms

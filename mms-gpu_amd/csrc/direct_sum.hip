@@ -40,7 +40,8 @@ constexpr long kRefPad = 8, kRefTableMin = 4096, kRefTableMax = 1L << 24;
 // (mms_potential_exact_noalloc), per GPU, held until the process ends: chunk
 // partial sums (16 MiB for its largest grids) or the transforms' tables and
 // work arrays (at most 32 bytes a cell each while no side is padded more
-// than four times; 121 MiB is the most any grid of 2,097,152 cells takes).
+// than four times; 124.2 MiB, on 1025 x 136 x 15, is the most that any grid
+// of 2,097,152 cells takes).
 constexpr long kScratchCells = 2L * 1024 * 1024;
 constexpr size_t kScratchBytes = 128u << 20;
 static __device__ __align__(256) double scratch[kScratchBytes / sizeof(double)];
@@ -800,7 +801,7 @@ int DirectPlan::init(const Grid &g, int split_) {
     } else if (form == kDirectFft) {
         MMS_HIP(hipMalloc(&table, direct_fft_table_bytes(g)));
         MMS_HIP(hipMalloc(&work, direct_fft_work_bytes(g)));
-        if (direct_fft_tables(g, table, work, nullptr)) return 1;
+        if (direct_fft_tables(g, table, nullptr)) return 1;
         MMS_HIP(hipStreamSynchronize(nullptr));
     } else {
         direct_chunks(n, split, &chunk, &nchunk);
@@ -951,8 +952,7 @@ extern "C" int mms_potential_exact_noalloc(const float *charge_dev, float *poten
         const size_t tb = direct_fft_table_bytes(g);
         MMS_CHECK(tb + direct_fft_work_bytes(g) <= kScratchBytes, "mms_potential_exact_noalloc: scratch too small");
         void *work = reinterpret_cast<char *>(mem) + tb;
-        if (direct_fft_tables(g, mem, work, s)) return 1;
-        return direct_fft_potential(g, mem, work, nullptr, const_cast<float *>(charge_dev), potential_dev, s);
+        return direct_fft_potential_once(g, mem, work, charge_dev, potential_dev, s);
     }
     long chunk = 0;
     int nchunk = 0;

@@ -97,9 +97,11 @@ int direct_potential_of(const Grid &g, DirectPlan &plan, const float *m, float *
 bool direct_fft_fits(const Grid &g);
 size_t direct_fft_table_bytes(const Grid &g);
 size_t direct_fft_work_bytes(const Grid &g);
-int direct_fft_tables(const Grid &g, void *table, void *work, hipStream_t s);
+int direct_fft_tables(const Grid &g, void *table, hipStream_t s);
 int direct_fft_potential(const Grid &g, const void *table, void *work, const float *m, float *rho, float *phi,
                          hipStream_t s);
+// the potential and the tables that it needs in the same three launches
+int direct_fft_potential_once(const Grid &g, void *table, void *work, const float *rho, float *phi, hipStream_t s);
 // the float arithmetic and summation order of the reference's CUDA direct-sum kernel
 struct RefgpuPlan {
     double *tab = nullptr;  // 1 / r of the absolute offsets (null: the dividing kernel alone)
