@@ -56,9 +56,8 @@ __device__ __forceinline__ void batch_column(const int4 &t, const BatchFilm &f, 
 
 // The z walk of a thread: its whole column, or with SPLIT the one layer
 // blockIdx.y, whose z neighbours are then loaded like the others (the same
-// expressions on the same values; the compiler may fuse a multiply-add
-// differently, which after hundreds of steps shows in the last bit of a cell
-// or two in a million).
+// expressions on the same values: over 400 steps of films of 1 to 5 layers the
+// states are the same bit for bit).
 struct Layers { int first, end; };
 template <bool SPLIT>
 __device__ __forceinline__ Layers layers(int zd) {
@@ -793,7 +792,17 @@ unsigned xcd_grid(const Grid &g) {
 // 62.9 / 46.9, 705x498x4 (1.4 M cells) 92.9 / 92.3; above, the walk's fewer
 // loads count.
 constexpr long kSplitCells = 1L << 20;
-bool split_layers(const Grid &g) { return g.n() < kSplitCells && g.zd <= 65535; }  // layers in the grid's y
+// MMS_GPU_STAGE_ONE_CELL=1 keeps the one-cell column walk in the stage,
+// charge and field kernels, so that tests can hold the other forms against it.
+// The per-layer form and the four-cell charges are bitwise the same; in the
+// four-cell stage form the compiler fuses other multiply-adds: without the demag
+// field 13 of 3.1 million values differ in their last bit after 80 steps and
+// 1525 after 200.
+bool column_walk() {
+    const char *one = std::getenv("MMS_GPU_STAGE_ONE_CELL");
+    return one && one[0] == '1';
+}
+bool split_layers(const Grid &g) { return g.n() < kSplitCells && g.zd <= 65535 && !column_walk(); }  // layers in the grid's y
 
 }  // namespace
 
@@ -806,7 +815,7 @@ int launch_div(const Grid &g, const float *m, float *rho, hipStream_t s, Profile
         MMS_HIP(hipGetLastError());
         return 0;
     }
-    if (g.xd % 4 == 0 && ((reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(rho)) & 15) == 0) {
+    if (g.xd % 4 == 0 && ((reinterpret_cast<uintptr_t>(m) | reinterpret_cast<uintptr_t>(rho)) & 15) == 0 && !column_walk()) {
         const long ntiles = (long)((g.xd + 4 * BX - 1) / (4 * BX)) * ((g.yd + BY - 1) / BY);
         dim3 grid((unsigned)(8 * ((ntiles + 7) / 8)));
         switch (g.zd) {
@@ -843,16 +852,12 @@ int launch_stage_ex(const Grid &g, const Material &mat, int stage, double dt, co
     const uintptr_t al = reinterpret_cast<uintptr_t>(m_in) | reinterpret_cast<uintptr_t>(m_out) |
                          reinterpret_cast<uintptr_t>(mn) | reinterpret_cast<uintptr_t>(acc) |
                          reinterpret_cast<uintptr_t>(phi) | reinterpret_cast<uintptr_t>(ex.m_base);
-    // MMS_GPU_STAGE_ONE_CELL=1 keeps the one-cell column walk (the four-cell
-    // and per-layer forms' results are bitwise the same; the switch lets tests show it)
-    const char *one = std::getenv("MMS_GPU_STAGE_ONE_CELL");
-    const bool walk = one && one[0] == '1';
-    if (split_layers(g) && !walk) {
+    if (split_layers(g)) {
         launch_stage_zd<0, true>(dim3(xcd_grid(g), g.zd), block, s, A, plain);
         MMS_HIP(hipGetLastError());
         return 0;
     }
-    if (plain && !walk && g.xd % 4 == 0 && (al & 15) == 0 &&
+    if (plain && !column_walk() && g.xd % 4 == 0 && (al & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(matl) & 3) == 0) {
         const long ntiles = (long)((g.xd + 4 * BX - 1) / (4 * BX)) * ((g.yd + BY4 - 1) / BY4);
         dim3 grid4((unsigned)(8 * ((ntiles + 7) / 8))), block4(BX, BY4);
