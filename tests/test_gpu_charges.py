@@ -29,3 +29,18 @@ def test_quotients_beyond_the_float_range(mg, orc, dims, use_fmm):
         want = orc.divergence_3d(M, dims, D)
     assert np.isinf(want).sum() >= 20
     assert np.array_equal(ch, want, equal_nan=True)
+
+
+# the charge kernel's forms, reached by the FMM above 524,288 cells: four cells a thread at 2, 3 and 4 layers, the column
+# walk at a width that is no multiple of four (3, 4 and other layers), one cell per thread and layer below 1,048,576 cells
+@pytest.mark.parametrize("dims", [(1024, 512, 2), (1000, 350, 3), (640, 410, 4), (701, 500, 3), (701, 380, 4),
+                                  (1049, 1000, 1), (900, 600, 1), (449, 400, 3)])
+def test_charge_kernels(mg, orc, dims, monkeypatch):
+    n = int(np.prod(dims))
+    M = (np.random.default_rng(n).standard_normal(3 * n) * 5e5).astype(F)
+    M[np.random.default_rng(1).random(3 * n) < 0.2] = 0.0
+    want = orc.divergence_3d(M, dims, D)
+    for walk in ("0", "1"):
+        monkeypatch.setenv("MMS_GPU_STAGE_ONE_CELL", walk)
+        ch, _ = _hfield(mg, M, dims, 1)
+        assert np.array_equal(ch, want), walk
