@@ -770,20 +770,20 @@ extern "C" int rk4_step(float t, float dt, float *t2, const unsigned char *mater
 namespace {
 struct LoopState {
     double *red = nullptr;  // device [2 + 5][red_blocks]
-    double *pin = nullptr;  // the same on the host
+    HostBuffer host;        // the same on the host
     hipEvent_t ready = nullptr;
     TextDump text;
     bool ramp = false;
     int init(mms_ctx *c) {
         MMS_HIP(hipMalloc(&red, sizeof(double) * 7 * c->red_blocks));
-        MMS_HIP(hipHostMalloc(&pin, sizeof(double) * 7 * c->red_blocks, hipHostMallocDefault));
+        if (host.alloc(sizeof(double) * 7 * c->red_blocks)) return 1;
         MMS_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
         ramp = c->p.external == MMS_EXT_RAMP;
         return text.init(c->g);
     }
     ~LoopState() {
         if (red) (void)hipFree(red);
-        if (pin) (void)hipHostFree(pin);
+        host.release();
         if (ready) (void)hipEventDestroy(ready);
         text.release();
     }
@@ -796,7 +796,7 @@ struct LoopState {
     int reduce(mms_ctx *c, const float *m, const float *h) {
         if (launch_energy_h(m, h, c->matl, c->g.n(), red, c->red_blocks, c->stream, &c->prof)) return 1;
         if (launch_mavg(m, c->matl, c->g.n(), red + 2 * c->red_blocks, c->red_blocks, c->stream)) return 1;
-        MMS_HIP(hipMemcpyAsync(pin, red, sizeof(double) * 7 * c->red_blocks, hipMemcpyDeviceToHost, c->stream));
+        MMS_HIP(hipMemcpyAsync(host.p, red, sizeof(double) * 7 * c->red_blocks, hipMemcpyDeviceToHost, c->stream));
         MMS_HIP(hipEventRecord(ready, c->stream));
         return 0;
     }
@@ -804,10 +804,11 @@ struct LoopState {
         MMS_HIP(hipEventSynchronize(ready));
         return 0;
     }
+    const double *part() const { return reinterpret_cast<const double *>(host.p); }
     void averages(const mms_ctx *c, double out[5]) const {
         for (int q = 0; q < 5; q++) out[q] = 0;
         for (int i = 0; i < c->red_blocks; i++)
-            for (int q = 0; q < 5; q++) out[q] += pin[2 * c->red_blocks + 5 * i + q];
+            for (int q = 0; q < 5; q++) out[q] += part()[2 * c->red_blocks + 5 * i + q];
     }
     // the dump's pieces from `first` on, one after the other
     int dump_rest(mms_ctx *c, const float *m, FILE *fh, long first) {
@@ -908,7 +909,7 @@ extern "C" int time_marching(unsigned char *material, float *M, float finaltime,
         pending = false;
         if (defer && loop.text.enqueue(c->m32[d], 0, s)) { status = 1; break; }
         if (loop.wait()) { status = 1; break; }
-        energy_torque_sum(c, loop.pin, &E2d, &torqued);
+        energy_torque_sum(c, loop.part(), &E2d, &torqued);
         const float E2 = (float)E2d, torque = (float)torqued;
         if (E2 - E > .1) {
             // rejected: M and H stay as they were

@@ -308,6 +308,14 @@ struct Xfer { void *host; void *dev; size_t bytes; };
 int copy_to_device(const Xfer *x, int count, hipStream_t s);
 int copy_to_host(const Xfer *x, int count, hipStream_t s);
 void transfer_user(int delta);
+// Host memory that enqueued copies fill: pinned, or plain where none can be
+// had (its copies then hold up the caller).
+struct HostBuffer {
+    char *p = nullptr;
+    bool pinned = false;
+    int alloc(size_t bytes);
+    void release();
+};
 inline Xfer up(const void *host, void *dev, size_t bytes) { return Xfer{const_cast<void *>(host), dev, bytes}; }
 inline int copy_to_device(const void *host, void *dev, size_t bytes, hipStream_t s) {
     const Xfer x = up(host, dev, bytes);
@@ -324,7 +332,8 @@ inline int copy_to_host(void *host, const void *dev, size_t bytes, hipStream_t s
 struct TextDump {
     Grid g{};
     long blocks = 0, cap = 0;
-    char *dev = nullptr, *pin = nullptr;
+    char *dev = nullptr;
+    HostBuffer host;
     hipEvent_t copied = nullptr;
     int init(const Grid &g);
     void release();

@@ -79,16 +79,16 @@ int TextDump::init(const Grid &g_) {
     cap = blocks < 256 ? blocks : 256;
     const size_t bytes = (size_t)cap * kBlockBytes + sizeof(int) * cap;
     MMS_HIP(hipMalloc(&dev, bytes));
-    MMS_HIP(hipHostMalloc(&pin, bytes, hipHostMallocDefault));
+    if (host.alloc(bytes)) return 1;
     MMS_HIP(hipEventCreateWithFlags(&copied, hipEventDisableTiming));
     return 0;
 }
 
 void TextDump::release() {
     if (dev) (void)hipFree(dev);
-    if (pin) (void)hipHostFree(pin);
+    host.release();
     if (copied) (void)hipEventDestroy(copied);
-    dev = pin = nullptr;
+    dev = nullptr;
     copied = nullptr;
     blocks = cap = 0;
 }
@@ -100,7 +100,7 @@ int TextDump::enqueue(const float *m, long first, hipStream_t s) {
     hipLaunchKernelGGL(text_kernel, dim3((unsigned)nb), dim3(kBlockLines), 0, s, m, first * kBlockLines, g.n(), g.xd, g.yd,
                        dev, len);
     MMS_HIP(hipGetLastError());
-    MMS_HIP(hipMemcpyAsync(pin, dev, (size_t)cap * kBlockBytes + sizeof(int) * nb, hipMemcpyDeviceToHost, s));
+    MMS_HIP(hipMemcpyAsync(host.p, dev, (size_t)cap * kBlockBytes + sizeof(int) * nb, hipMemcpyDeviceToHost, s));
     MMS_HIP(hipEventRecord(copied, s));
     return 0;
 }
@@ -109,8 +109,8 @@ int TextDump::enqueue(const float *m, long first, hipStream_t s) {
 int TextDump::write(FILE *fh, long first) const {
     MMS_HIP(hipEventSynchronize(copied));
     const long nb = blocks - first < cap ? blocks - first : cap;
-    const int *len = reinterpret_cast<const int *>(pin + (size_t)cap * kBlockBytes);
-    for (long b = 0; b < nb; b++) fwrite(pin + b * kBlockBytes, 1, len[b], fh);
+    const int *len = reinterpret_cast<const int *>(host.p + (size_t)cap * kBlockBytes);
+    for (long b = 0; b < nb; b++) fwrite(host.p + b * kBlockBytes, 1, len[b], fh);
     return 0;
 }
 

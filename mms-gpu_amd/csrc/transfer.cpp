@@ -12,6 +12,7 @@
 // most kKeep are kept, and they are freed with the last context.
 #include <hip/hip_runtime.h>
 #include <math.h>
+#include <stdlib.h>
 #include <string.h>
 #include <algorithm>
 #include <atomic>
@@ -225,6 +226,25 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
 }
 
 }  // namespace
+
+int HostBuffer::alloc(size_t bytes) {
+    void *m = nullptr;
+    pinned = hipHostMalloc(&m, bytes, hipHostMallocDefault) == hipSuccess;
+    if (!pinned) {
+        (void)hipGetLastError();
+        m = malloc(bytes);
+    }
+    p = static_cast<char *>(m);
+    MMS_CHECK(p, "no host memory for the time loop");
+    return 0;
+}
+
+void HostBuffer::release() {
+    if (pinned) (void)hipHostFree(p);
+    else free(p);
+    p = nullptr;
+    pinned = false;
+}
 
 int copy_to_device(const Xfer *x, int count, hipStream_t s) { return run(x, count, true, s); }
 int copy_to_host(const Xfer *x, int count, hipStream_t s) { return run(x, count, false, s); }

@@ -24,7 +24,7 @@ struct Limit { const void *f; int value; };
 std::vector<Copy> copies;
 std::vector<Limit> limits;
 std::map<const char *, size_t> pinned, device;
-int fail_pinned, launches;
+int fail_pinned, fail_malloc, mallocs, launches;
 float event_ms;
 dim3 cfg_grid, cfg_block;
 size_t cfg_lds;
@@ -53,6 +53,8 @@ hipError_t copy(void *d, const void *s, size_t n, int kind) {
 }  // namespace
 extern "C" {
 void stub_fail_pinned(int on) { fail_pinned = on; }
+void stub_fail_malloc(int k) { fail_malloc = k; mallocs = 0; }  // the k-th hipMalloc from here fails
+int stub_mallocs() { return mallocs; }
 void stub_clear() { std::lock_guard<std::mutex> lk(mu); copies.clear(); limits.clear(); launches = 0; }
 int stub_copies() { return (int)copies.size(); }
 const void *stub_copy_dst(int i) { return copies[i].dst; }
@@ -66,7 +68,11 @@ long stub_pinned() { return (long)pinned.size(); }
 void *stub_pin(long n) { return take(pinned, n); }
 void *stub_device(long n) { return take(device, n); }
 
-hipError_t hipMalloc(void **p, size_t n) { *p = take(device, n); return hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) {
+    if (++mallocs == fail_malloc) { *p = nullptr; return hipErrorOutOfMemory; }
+    *p = take(device, n);
+    return hipSuccess;
+}
 hipError_t hipFree(void *p) { drop(device, p); return hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
     if (fail_pinned) { *p = nullptr; return hipErrorOutOfMemory; }
