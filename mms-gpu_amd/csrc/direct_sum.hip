@@ -648,9 +648,13 @@ int RefgpuPlan::init(const Grid &g) {
     const float small = fminf(g.dx, fminf(g.dy, g.dz));
     if (n < kRefTableMin || n > kRefTableMax || small < 1e-15f || ext > 1e15) return 0;  // direct_refgpu_kernel alone
     qmin = (float)(ext * 2.3509887e-38);
-    MMS_HIP(hipMalloc(&tab, sizeof(double) * (n + kRefPad)));
     split = refgpu_groups(g) < 1024 ? 16 : 4;  // workgroups a target group: enough to fill the chip
-    MMS_HIP(hipMalloc(&qd, sizeof(double) * n + sizeof(float) * split * n + 256));
+    if (hipMalloc(&tab, sizeof(double) * (n + kRefPad)) != hipSuccess ||
+        hipMalloc(&qd, sizeof(double) * n + sizeof(float) * split * n + 256) != hipSuccess) {
+        (void)hipGetLastError();
+        release();
+        return 0;  // no memory for it: direct_refgpu_kernel alone
+    }
     part = reinterpret_cast<float *>(qd + n);
     need = reinterpret_cast<int *>(part + split * n);
     hipLaunchKernelGGL(refgpu_table_kernel, dim3((unsigned)((n + kRefPad + 255) / 256)), dim3(256), 0, nullptr, tab, g.xd,
@@ -799,11 +803,19 @@ int DirectPlan::init(const Grid &g, int split_) {
         if (small_table(g, static_cast<float *>(table), nullptr)) return 1;
         MMS_HIP(hipStreamSynchronize(nullptr));
     } else if (form == kDirectFft) {
-        MMS_HIP(hipMalloc(&table, direct_fft_table_bytes(g)));
-        MMS_HIP(hipMalloc(&work, direct_fft_work_bytes(g)));
-        if (direct_fft_tables(g, table, nullptr)) return 1;
-        MMS_HIP(hipStreamSynchronize(nullptr));
-    } else {
+        // tables and work arrays of up to 64 bytes a cell; where they cannot be
+        // had the pair loop serves the grid, with 8 bytes a cell at least
+        if (hipMalloc(&table, direct_fft_table_bytes(g)) != hipSuccess ||
+            hipMalloc(&work, direct_fft_work_bytes(g)) != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            form = kDirectChunks;
+        } else {
+            if (direct_fft_tables(g, table, nullptr)) return 1;
+            MMS_HIP(hipStreamSynchronize(nullptr));
+        }
+    }
+    if (form == kDirectChunks) {
         direct_chunks(n, split, &chunk, &nchunk);
         MMS_HIP(hipMalloc(&work, sizeof(double) * (size_t)n * nchunk));
     }
