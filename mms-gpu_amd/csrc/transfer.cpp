@@ -213,15 +213,22 @@ int run(const Xfer *x, int count, bool to_device, hipStream_t s) {
             }
         if (total < line) ring = 0;
     }
-    for (int i = 0; i < count; i++)
-        if (x[i].host && !(ring >> i & 1) && copy_runtime(x[i], to_device, s)) return 1;
+    bool direct = false;
+    auto runtime = [&](unsigned mask) {
+        for (int i = 0; i < count; i++)
+            if (x[i].host && (mask >> i & 1)) {
+                direct = true;
+                if (copy_runtime(x[i], to_device, s)) return 1;
+            }
+        return 0;
+    };
+    if (runtime(~ring)) return 1;
     if (ring) {
         const int st = run_ring(x, count, ring, total, to_device, s);
-        if (st > 0) return 1;
-        for (int i = 0; st < 0 && i < count; i++)
-            if ((ring >> i & 1) && copy_runtime(x[i], to_device, s)) return 1;
+        if (st > 0 || (st < 0 && runtime(ring))) return 1;
     }
-    if (!to_device) MMS_HIP(hipStreamSynchronize(s));
+    // (the chunks have been waited for one by one; a wait for the stream after them takes 50 us)
+    if (direct && !to_device) MMS_HIP(hipStreamSynchronize(s));
     return 0;
 }
 

@@ -24,7 +24,7 @@ struct Limit { const void *f; int value; };
 std::vector<Copy> copies;
 std::vector<Limit> limits;
 std::map<const char *, size_t> pinned, device;
-int fail_pinned, fail_malloc, mallocs, launches;
+int fail_pinned, fail_malloc, mallocs, launches, syncs;
 float event_ms;
 dim3 cfg_grid, cfg_block;
 size_t cfg_lds;
@@ -55,7 +55,8 @@ extern "C" {
 void stub_fail_pinned(int on) { fail_pinned = on; }
 void stub_fail_malloc(int k) { fail_malloc = k; mallocs = 0; }  // the k-th hipMalloc from here fails
 int stub_mallocs() { return mallocs; }
-void stub_clear() { std::lock_guard<std::mutex> lk(mu); copies.clear(); limits.clear(); launches = 0; }
+void stub_clear() { std::lock_guard<std::mutex> lk(mu); copies.clear(); limits.clear(); launches = syncs = 0; }
+int stub_syncs() { return syncs; }
 int stub_copies() { return (int)copies.size(); }
 const void *stub_copy_dst(int i) { return copies[i].dst; }
 const void *stub_copy_src(int i) { return copies[i].src; }
@@ -121,7 +122,7 @@ hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) { *ms = event_ms += 1.0f; return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { *s = reinterpret_cast<hipStream_t>(malloc(1)); return hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { free(s); return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { syncs++; return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) { *d = 0; return hipSuccess; }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *c) { *c = hipStreamCaptureStatusNone; return hipSuccess; }

@@ -69,3 +69,19 @@ to = [t for t, _, b in copies()]
 assert to.count(H.ctypes.data) == 1 and ch.ctypes.data not in to and pot.ctypes.data not in to
 assert not ch.any() and not pot.any()  # the stand-in's device memory
 """)
+
+
+def test_downloads_wait_once(tmp_path):
+    """Chunks are waited for one by one, and the stream is not waited for
+    again after them; the runtime's copies need that wait."""
+    run(tmp_path, FILM + r"""
+f.set_m(M)
+stub.stub_clear()
+assert np.array_equal(f.get_m(), M)  # 2.4 MB: chunks
+assert len(copies()) > 1 and stub.stub_syncs() == 0
+with mg.Film(1000, 1, 1, F(5e-9), F(5e-9), F(5e-9), demag=0) as g:
+    g.set_m(M[:3000])
+    stub.stub_clear()
+    assert np.array_equal(g.get_m(), M[:3000])
+    assert len(copies()) == 1 and stub.stub_syncs() == 1
+""")
