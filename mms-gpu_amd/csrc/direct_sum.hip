@@ -641,12 +641,15 @@ static int refgpu_groups(const Grid &g) { return (int)(((long)((g.xd + 3) / 4) *
 
 // The table form needs r finite and well inside the float range, and quotients
 // that are normal floats (checked charge by charge against qmin = 2^-125 rmax).
+// Films one cell wide fill a quarter of its groups of four x neighbours and
+// stay with the division (1 x 5000 x 1: 144 us by the table, 96 by the
+// division; 2 x 2100 x 1: 67 and 78).
 int RefgpuPlan::init(const Grid &g) {
     release();
     const long n = g.n();
     const double ext = (double)g.xd * g.dx + (double)g.yd * g.dy + (double)g.zd * g.dz;
     const float small = fminf(g.dx, fminf(g.dy, g.dz));
-    if (n < kRefTableMin || n > kRefTableMax || small < 1e-15f || ext > 1e15) return 0;  // direct_refgpu_kernel alone
+    if (g.xd == 1 || n < kRefTableMin || n > kRefTableMax || small < 1e-15f || ext > 1e15) return 0;  // direct_refgpu_kernel alone
     qmin = (float)(ext * 2.3509887e-38);
     split = refgpu_groups(g) < 1024 ? 16 : 4;  // workgroups a target group: enough to fill the chip
     if (hipMalloc(&tab, sizeof(double) * (n + kRefPad)) != hipSuccess ||

@@ -229,10 +229,10 @@ int surrogate_backward(SurrogatePlan &sp, const float *rho, const float *phi_s, 
                        const float *inv_norm, float gscale, float rscale, float oscale, float *grad, hipStream_t s);
 // Adam step `step` (from 1) at rate lr on sp.d_param with moments m, v; refreshes the BF16 copies
 int surrogate_adam(SurrogatePlan &sp, float *m, float *v, const float *grad, long step, float lr, hipStream_t s);
-// sum of x^2 over n values (synchronous)
 // pairs idx[0 .. batch) of a training set [pair][npf] and their 1 / |phi|^2 (host) into the batch buffers
 int surrogate_gather(const float *rho, const float *phi, long npf, const long *idx, const float *inv_norm, int batch,
                      float *brho, float *bphi, float *binv, hipStream_t s);
+// sum of x^2 over n values (synchronous)
 int surrogate_sqnorm(SurrogatePlan &sp, const float *x, long n, double *out, hipStream_t s);
 // relative L2 residual ||a - b|| / ||b|| (r null: partials only, left on the device)
 int surrogate_residual(SurrogatePlan &sp, const float *a, const float *b, long n, double *r, hipStream_t s);

@@ -40,3 +40,15 @@ for dims in ((1025, 136, 15), (1025, 146, 14), (1025, 292, 7), (2048, 1024, 1), 
     assert lib.mms_potential_exact_noalloc(p, p, *dims, F(5e-9), F(5e-9), F(5e-9), None) == 0, (dims, mg.last_error())
 assert lib.mms_potential_exact_noalloc(p, p, 2097153, 1, 1, F(5e-9), F(5e-9), F(5e-9), None) != 0
 """)
+
+
+def test_reference_order_form_by_width(tmp_path):
+    """One launch (the dividing kernel) for films one cell wide, five (flag,
+    charges, pairs, join and the dividing kernel's check) for wider ones."""
+    run(tmp_path, r"""
+for dims, want in (((1, 5000, 1), 1), ((1, 100, 150), 1), ((2, 2500, 1), 5), ((5000, 1, 1), 5), ((2, 2000, 1), 1)):
+    with mg.Film(*dims, F(5e-9), F(5e-9), F(5e-9), solver=mg.SOLVER_DIRECT_REFGPU) as f:
+        stub.stub_clear()
+        f.potential(np.ones(int(np.prod(dims)), F))
+        assert stub.stub_launches() == want, (dims, stub.stub_launches())
+""")
