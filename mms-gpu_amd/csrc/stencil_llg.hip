@@ -604,6 +604,7 @@ __global__ __launch_bounds__(BX * BY) void stage_batch_kernel(StageArgs A, const
     stage_column<ZD, ST>(A, x, y, f.xd, f.yd, f.zd, f.off, pstride, f.hx, f.hy, f.hz);
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(BX * BY) void hfield_kernel(StageArgs A) {
     const int x = blockIdx.x * BX + threadIdx.x, y = blockIdx.y * BY + threadIdx.y;
     const int xd = A.xd, yd = A.yd, zd = A.zd;
@@ -616,7 +617,7 @@ __global__ __launch_bounds__(BX * BY) void hfield_kernel(StageArgs A) {
     if (A.external == 1) { hex = ramp_hx(t, A.inv_mu0); hey = 0.0f; hez = 0.0f; }
     const float dx2 = A.dx * A.dx, dy2 = A.dy * A.dy, dz2 = A.dz * A.dz;
     // one layer per grid z, or the whole column
-    const int zf = gridDim.z > 1 ? (int)blockIdx.z : 0, ze = gridDim.z > 1 ? zf + 1 : zd;
+    const int zf = SPLIT ? (int)blockIdx.z : 0, ze = SPLIT ? zf + 1 : zd;
     for (int z = zf; z < ze; z++) {
         const long c = (long)z * plane + c0;
         float Hx = 0.0f, Hy = 0.0f, Hz = 0.0f;
@@ -890,8 +891,10 @@ int launch_hfield(const Grid &g, const Material &mat, const float *phi, const fl
     KTimer kt(prof, K_HFIELD);
     StageArgs A = make_args(g, mat);
     A.phi = phi; A.m_in = m; A.t_dev = t_dev; A.h_out = H_aos;
-    dim3 grid((g.xd + BX - 1) / BX, (g.yd + BY - 1) / BY, split_layers(g) ? g.zd : 1), block(BX, BY);
-    hipLaunchKernelGGL(hfield_kernel, grid, block, 0, s, A);
+    const bool split = split_layers(g);
+    dim3 grid((g.xd + BX - 1) / BX, (g.yd + BY - 1) / BY, split ? g.zd : 1), block(BX, BY);
+    if (split) hipLaunchKernelGGL(hfield_kernel<true>, grid, block, 0, s, A);
+    else hipLaunchKernelGGL(hfield_kernel<false>, grid, block, 0, s, A);
     MMS_HIP(hipGetLastError());
     return 0;
 }
