@@ -132,7 +132,9 @@ __global__ __launch_bounds__(256) void m2m_mfma_kernel(const float *__restrict__
 // Float offsets of every level in mult / loc / part (per film).
 struct LevelOffsets { long off[16]; };
 // Upward pass of a state: M (three planes of cells) and where its charges go;
-// m null: the charges are given.
+// m null: the charges are given.  The two are compiled apart: with one kernel
+// the pass on given charges took 17.2 us on 1024 x 1024 x 4 (P 6, leaf width
+// 8), by itself 16.6 (leaf width 4 37.3 and 35.5).
 struct Charges { const float *m; float *rho; float dx, dy, dz; };
 
 // Upward pass of one subtree: the workgroup owns one box of level R of one
@@ -140,7 +142,7 @@ struct Charges { const float *m; float *rho; float dx, dy, dz; };
 // the leaves as FP32 MFMA [KP x W^2] . [W^2 x leaves] with the charges staged
 // in LDS, then D levels of M2M on the LDS copy; every level's multipoles are
 // written to HBM.  Wave w takes MFMA column tiles w, w + 4, ... of 16 boxes.
-template <int K, int KP, int W>
+template <int K, int KP, int W, bool FROM_M>
 __global__ __launch_bounds__(256) void up_subtree_kernel(const float *__restrict__ rho, float *__restrict__ Mall,
                                                          const float *__restrict__ p2mf,
                                                          const float *__restrict__ m2mfrag, LevelOffsets lo, int R,
@@ -163,7 +165,7 @@ __global__ __launch_bounds__(256) void up_subtree_kernel(const float *__restrict
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j16 = lane & 15, g = lane >> 4;
     const int cx0 = rbx * CS, cy0 = rby * CS;
     float *q = lds;  // CS x CS charges, later the leaf multipoles [leaf][SB]
-    if (cm.m) {
+    if constexpr (FROM_M) {
         // charges formed here from the state (one film), by the stencil's
         // expression, and stored for the near field
         const float *mx = cm.m, *my = mx + plane * fs.zd, *mz = my + plane * fs.zd;
@@ -197,7 +199,7 @@ __global__ __launch_bounds__(256) void up_subtree_kernel(const float *__restrict
         }
     }
 #pragma unroll 1
-    for (int e0 = cm.m ? CS * CS : 0; e0 < CS * CS; e0 += 256 * 8) {  // 8 loads per thread in flight
+    for (int e0 = FROM_M ? CS * CS : 0; e0 < CS * CS; e0 += 256 * 8) {  // 8 loads per thread in flight
         float vb[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -1747,14 +1749,24 @@ int run_fmm(const Grid &g, FmmPlan &pl, const Charges &cm, const float *rho, flo
         const long bufB = (long)std::max(1, (S / 2) * (S / 2)) * SB;
         const size_t lds = sizeof(float) * (size_t)(bufA + bufB);
         MMS_CHECK(lds <= 160 * 1024, "FMM upward pass: subtree exceeds LDS");
-        static int attr = 0;
-        if (!attr) {
-            MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&up_subtree_kernel<K, KP, W>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-            attr = 1;
+        auto up = [&](auto from_m) -> int {
+            constexpr bool FROM_M = decltype(from_m)::value;
+            static int attr = 0;
+            if (!attr) {
+                MMS_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&up_subtree_kernel<K, KP, W, FROM_M>),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+                attr = 1;
+            }
+            hipLaunchKernelGGL((up_subtree_kernel<K, KP, W, FROM_M>), dim3(nsub, zd * pl.nfilm), dim3(256), lds, s,
+                               rho, pl.mult, pl.d_p2mf, pl.d_m2m, lo, R, D, nsx, g.xd, g.yd, bufA, pl.films(), cm);
+            return 0;
+        };
+        // (only leaf width 4 forms the charges: one_queue)
+        if constexpr (W == 4) {
+            if (cm.m ? up(std::true_type()) : up(std::false_type())) return 1;
+        } else {
+            if (up(std::false_type())) return 1;
         }
-        hipLaunchKernelGGL((up_subtree_kernel<K, KP, W>), dim3(nsub, zd * pl.nfilm), dim3(256), lds, s, rho,
-                           pl.mult, pl.d_p2mf, pl.d_m2m, lo, R, D, nsx, g.xd, g.yd, bufA, pl.films(), cm);
         MMS_HIP(hipGetLastError());
     }
     if constexpr (split) {
