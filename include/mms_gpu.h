@@ -173,8 +173,8 @@ typedef struct {
     int demag, exchange;        /* 0/1 switches                                */
     int external;               /* enum mms_external                           */
     float hext[3];              /* A/m, for MMS_EXT_CONST                      */
-    int m2l_cols;               /* M2L targets per wavefront in 16-column MFMA tiles (4 or 8; 0 = 4;
-                                   4 becomes 2 where the launch leaves CUs idle) */
+    int m2l_cols;               /* M2L targets per wavefront in 16-column MFMA tiles: 0 or 4 lets the
+                                   library take 1, 2 or 4 by size and form, 8 takes 8 where they fit */
     int direct_split;           /* direct sum: source-chunk multiplier of the pair loop (1, 2 or 4; 0 = 1) */
 } mms_params;
 

@@ -643,7 +643,7 @@ __global__ __launch_bounds__(256) void down_coarse_kernel(const float *__restric
 }
 
 // -------------------------------------------------------- M2L + L2L --
-// A workgroup owns a dense TX x 16 block of target boxes (TX = 8, 16 or 32) of one
+// A workgroup owns a dense TX x 16 block of target boxes (TX = 4, 8, 16 or 32) of one
 // target layer; wave w handles child parity (w & 1, w >> 1): an SX x 8
 // sub-lattice (SX = TX / 2) of targets in NC = SX / 2 MFMA column tiles of 16.
 // The source window holds the tile plus a 3-box halo: (TX + 6) x 22 boxes.
@@ -1557,11 +1557,13 @@ long m2l_groups(const FmmPlan &pl, int ZP) {
 // many column tiles (NC) as cost least: a CU's share of the workgroups times
 // NC and half a tile for the window.  Four need more than one such round (with one
 // the window's latency shows).  Beside the FP32 near field of leaf width 8,
-// one tile.  RK4 steps in us with 1 / 2 / 4 tiles: leaf 4, 64x64x3 P 3 109 / 119 /
+// one tile: M2L alone then takes longer (1024 x 1024 x 4 P 6 197 us against 170
+// with four tiles), the step less.  RK4 steps in us with 1 / 2 / 4 tiles: leaf 4, 64x64x3 P 3 109 / 119 /
 // 139, 128x128x4 P 6 203 / 195 / 247, 256x256x3 P 4 181 / 182 / 193, 300x280x3
 // P 6 378 / 374 / 417, 400x300x3 P 5 452 / 439 / 430, 512x512x3 P 4 369 / 362
-// / 365; leaf 8, 300x300x2 P 5 261 / 284 / 335, 1000x600x3 P 6 913 / 912 / 933,
-// 1024x1024x4 P 6 1748 / 1881 / 1843.
+// / 365; leaf 8, 300x300x2 P 5 261 / 284 / 335, 1000x600x3 P 6 907 / 908 / 935,
+// 1024x1024x4 P 6 1735 / 1881 / 1837 (four tiles and two layers 1861),
+// 2048x1024x4 P 6 3463 / 3641 / 3587, 1024x1024x2 P 4 705 / 697 / 700.
 // The 16-bit forms take one tile and one layer while that is one round (64 x
 // 64 x 3, P 6: BF16 split 142 -> 127, FP16 hi/lo 154 -> 132; leaf 8, 200 x 200
 // x 3 212 -> 196), the scaled FP16 and plain BF16 forms then two tiles and two

@@ -6,8 +6,9 @@
 // it), pinned memory 57 GB/s.  Here the DMA of one chunk runs while the CPU
 // copies another, over all arrays of a call back to back, and large copies use a
 // few threads, since one thread touches fresh pages at 33 GB/s.  Of 48 MB
-// fresh (the state of a 1024 x 1024 x 4 film) 4.7 -> 1.8 ms, one rk4_step of a
-// 250 x 190 x 4 film with all its arrays 1.32 -> 1.11 ms.  The rings belong
+// fresh (the state of a 1024 x 1024 x 4 film) 4.7 -> 1.6 ms to the host, 1.7 ->
+// 1.2 to the device.  Smaller uploads and memory that the runtime knows are left
+// to the runtime.  The rings belong
 // to a pool: a call takes one, so calls of several threads do not meet, at
 // most kKeep are kept, and they are freed with the last context.
 #include <hip/hip_runtime.h>
